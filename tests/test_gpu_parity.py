@@ -429,6 +429,33 @@ def test_int8_rows_holding_infinities_quantize_as_the_oracle():
         p.assert_cache_equal(j)
 
 
+# The multi-row int8 append holds a page's tile in registers and takes most codes from y * (1 / s)
+# instead of y / s: bit for bit the row-by-row result for prompts that start anywhere in a page and
+# end on either side of its edge, one row and single rows after a prompt, rows whose amplitude grows
+# (a scale increase at every row) or falls, and quotients exactly on a half (a row of amplitude 127
+# makes s = 1, so x.5 are ties).
+@pytest.mark.parametrize("act,kvh", [("bf16", 8), ("f32", 2)])
+@pytest.mark.parametrize("grow", [1.0, 1.7, 0.6])
+def test_int8_prompt_rows_quantize_bit_for_bit(act, kvh, grow):
+    p = Pair(cache="i8", act=act, KVH=kvh, streams=6, cap=112, seed=67, L=1, page_seed=3)
+    for i, parts in enumerate([(16,), (1, 15, 17), (7, 9, 33), (31, 2, 1, 1), (5, 40, 3), (48, 1, 40)]):
+        for n in parts:
+            k, v = p.x(n, kvh, 64), p.x(n, kvh, 64)
+            amp = np.float32(grow) ** np.arange(n, dtype=np.float32)[:, None, None] % 1e6
+            k, v = k * amp, v * amp
+            v[n // 2] = np.arange(64) - 31.5  # ties once a row of amplitude 127 sets the scale to 1
+            if grow == 1.0:
+                v[n // 2, :, 0] = 127.0
+            if act == "bf16":
+                k, v = bf16_round(k), bf16_round(v)
+            p.pool.begin([p.ids[i]], t=n)
+            p.pool.append(0, dev(k, act), dev(v, act))
+            p.pool.end()
+            p.orc[i].append(0, k, v)
+            p.orc[i].commit(n)
+        p.assert_cache_equal(i)
+
+
 def test_int8_window_cache_matches_the_ring_it_stands_for():
     # An int8 window has no counterpart in the reference; it is an absolute ring of `context`
     # slots whose every row evicts the oldest, so the oracle's ring driven that way is its bar:
