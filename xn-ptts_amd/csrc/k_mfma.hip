@@ -10,14 +10,16 @@ namespace xnp {
 // prompt prefill on MFMA (bf16 cache and activations), transformer.rs:231-248 batched, with the
 // append of the prompt's K/V rows (complete_kv, transformer.rs:84-91) fused in.
 //
-// One work group of 8 waves per (stream, head).  Query rows are taken in rounds of 256: 16 tiles
-// of 16 rows, wave w owning tiles w and 15 - w of the round, so that every wave sees about the
-// same number of causal keys.  Keys are staged through LDS in chunks of 64 (four pages), K and
+// One work group of 8 waves per (stream, head, round), a round being 256 query rows: 16 tiles of 16
+// rows, wave w owning tiles w and 15 - w of the round, so that every wave sees about the same number
+// of causal keys.  Rounds are groups of their own, since a few long prompts leave the chip short of
+// groups (24 streams x 600 rows after 125: 192 groups of three rounds in turn, 64 us a layer;
+// 576 groups: 43 us).  Keys are staged through LDS in chunks of 64 (four pages), K and
 // V both as [key][dim], double-buffered, with the next chunk's loads in flight while one is
 // attended over.  Keys before the prompt come from the pages; the prompt's own keys come
 // from the k/v inputs, rotated at their position and rounded to bf16, and are written into
-// their pages during the last round, so that each is written exactly once and never read back
-// from HBM.
+// their pages by the last round's group, which sees them all, so that each is written exactly once
+// and never read back from HBM.
 //
 // Both contractions are computed transposed so that P never leaves registers:
 //   S^T = K Q^T   v_mfma_f32_16x16x32_bf16, A = K rows from LDS (lane: key lane%16, 8 dims),
@@ -90,8 +92,11 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
     __shared__ float ssc[2][kPfKeys / kBlock][2]; // int8: each chunk's pages' K and V scales
     const int t = bv.t;
     // plan b is the batch's row b (its out_row): the inputs' and the output's rows are b's, so their
-    // addresses do not wait for the plan
-    const int h = blockIdx.x % pv.H, b = blockIdx.x / pv.H;
+    // addresses do not wait for the plan.  The grid is round-major, the last round (the most keys)
+    // first: the groups of one (stream, head) stay n H apart, on one XCD where 8 divides n H.
+    const int nqt = (t + 15) / 16, per = bv.n * pv.H;
+    const int tq0 = ((int)gridDim.x / per - 1 - (int)blockIdx.x / per) * (kPfRound / 16); // the round's first tile
+    const int h = (int)blockIdx.x % per % pv.H, b = (int)blockIdx.x % per / pv.H;
     const StreamPlan P = bv.plans[b];
     const int32_t *tab = pv.tables + (size_t)P.sid * pv.mbps;
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
@@ -102,78 +107,52 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
     uint16_t *vpages = (uint16_t *)pv.pages + tile_index(pv, layer, 1, 0, kvh) * (kBlock * kHeadDim);
     const int8_t *kpages8 = (const int8_t *)pv.pages + tile_index(pv, layer, 0, 0, kvh) * (kBlock * kHeadDim);
     const int8_t *vpages8 = (const int8_t *)pv.pages + tile_index(pv, layer, 1, 0, kvh) * (kBlock * kHeadDim);
-    // the stream's page ids for every key any round sees, at most one per thread, loaded straight
+    // the stream's page ids for every key the round sees, at most one per thread, loaded straight
     // into LDS (lane l of wave w: id 64 w + l): no register holds them, and nothing waits for them
-    // before the first round's queries and first chunk go out.  Loads complete in the order
+    // before the round's queries and first chunk go out.  Loads complete in the order
     // issued, so the waits for those (every wave's query loads come after these) cover them, and
-    // the first round's barrier follows those waits; no earlier read of spages exists.
-    const int npg = min((c0 + t + kBlock - 1) / kBlock, kPfMaxPages);
+    // the barrier follows those waits; no earlier read of spages exists.
+    const int npg = min((c0 + min(t, 16 * tq0 + kPfRound) + kBlock - 1) / kBlock, kPfMaxPages);
     static_assert(kPfMaxPages <= 64 * kPfWaves, "one page id per thread");
     if (64 * w < npg) dma4_at(tab + min(tid, npg - 1), lds_addr(&spages[0]) + 256 * w);
     // this thread's share of a chunk: 16 bytes (8 dims) of one key's K and V
     const int skey = tid >> 3, spart = tid & 7;
 
-    const int nqt = (t + 15) / 16;
-    for (int tq0 = 0; tq0 < nqt; tq0 += kPfRound / 16) {
-        const int nq = min(kPfRound / 16, nqt - tq0);
-        const bool last = tq0 + nq == nqt;
-        // this wave's tiles: (w, nq-1-w) for w < nq/2; the middle one alone when nq is odd
-        int tile[2] = {-1, -1};
-        if (w < nq / 2) {
-            tile[0] = tq0 + w;
-            tile[1] = tq0 + nq - 1 - w;
-        } else if (w == nq / 2 && (nq & 1)) {
-            tile[0] = tq0 + w;
-        }
-        const int kend = c0 + min(t, 16 * (tq0 + nq)); // the round's rows see keys [0, kend)
-        const int nch = (kend + kPfKeys - 1) / kPfKeys;
+    const int nq = min(kPfRound / 16, nqt - tq0);
+    const bool last = tq0 + nq == nqt;
+    // this wave's tiles: (w, nq-1-w) for w < nq/2; the middle one alone when nq is odd
+    int tile[2] = {-1, -1};
+    if (w < nq / 2) {
+        tile[0] = tq0 + w;
+        tile[1] = tq0 + nq - 1 - w;
+    } else if (w == nq / 2 && (nq & 1)) {
+        tile[0] = tq0 + w;
+    }
+    const int kend = c0 + min(t, 16 * (tq0 + nq)); // the round's rows see keys [0, kend)
+    const int nch = (kend + kPfKeys - 1) / kPfKeys;
 
-        // Loads run one chunk ahead: chunk c's registers are consumed (rotated, stored to LDS
-        // buffer c & 1) at step c, which then issues chunk c + 1's loads into them.
-        struct Stage {
-            uint4 k, v, rope; // the key's K and V pieces (int8: 8 codes each in x, y), 4 (cos, sin) pairs as packed bf16
-            int info;         // bit 0: a prompt key, bit 1: write it to its page
-            float sk, sv;     // int8, the first thread of each page's keys: the page's scales
-        };
-        // LDS: the page ids are in LDS (all but the first round's first chunk, which reads the
-        // table itself); a compile-time choice, so that no pointer is selected between the two
-        auto issue = [&](int c, Stage &st, auto LDS) {
-            const int slot = c * kPfKeys + skey;
-            const bool in = c < nch && slot < kend;
-            const bool fresh = !I8 && fused && slot >= c0; // a prompt key: from the inputs, rotated here
-            const int i = fresh ? min(slot - c0, t - 1) : 0;
-            const size_t arow = (((size_t)b * t + i) * pv.KVH + kvh) * kHeadDim + 8 * spart;
-            st.k = st.v = make_uint4(0, 0, 0, 0);
-            st.sk = st.sv = 0.f;
-            if constexpr (I8) {
-                // int8 pages (the prompt's rows appended before): 8 codes of K and of V; the first
-                // thread of each page's keys also takes its scales (0 for a page outside the pool,
-                // as the bf16 path's zero rows: score 0, no value)
-                if (in) {
-                    const int blk = min(slot >> 4, kPfMaxPages - 1);
-                    int page;
-                    if constexpr (decltype(LDS)::value)
-                        page = spages[blk];
-                    else
-                        page = tab[blk];
-                    if (page >= 0 && page < pv.NB) {
-                        const size_t poff = (size_t)page * page_elems + (slot & 15) * kHeadDim + 8 * spart;
-                        const uint2 kk = *(const uint2 *)(kpages8 + poff), vv = *(const uint2 *)(vpages8 + poff);
-                        st.k = make_uint4(kk.x, kk.y, 0, 0);
-                        st.v = make_uint4(vv.x, vv.y, 0, 0);
-                        if ((skey & 15) == 0 && spart == 0) {
-                            st.sk = pv.scales[tile_index(pv, layer, 0, page, kvh)];
-                            st.sv = pv.scales[tile_index(pv, layer, 1, page, kvh)];
-                        }
-                    }
-                }
-                st.info = 0;
-                return;
-            }
-            if (in && fresh) {
-                st.k = ld_stream((const uint16_t *)knew + arow);
-                st.v = ld_stream((const uint16_t *)vnew + arow);
-            } else if (in) {
+    // Loads run one chunk ahead: chunk c's registers are consumed (rotated, stored to LDS
+    // buffer c & 1) at step c, which then issues chunk c + 1's loads into them.
+    struct Stage {
+        uint4 k, v, rope; // the key's K and V pieces (int8: 8 codes each in x, y), 4 (cos, sin) pairs as packed bf16
+        int info;         // bit 0: a prompt key, bit 1: write it to its page
+        float sk, sv;     // int8, the first thread of each page's keys: the page's scales
+    };
+    // LDS: the page ids are in LDS (all but the first chunk, which reads the table itself); a
+    // compile-time choice, so that no pointer is selected between the two
+    auto issue = [&](int c, Stage &st, auto LDS) {
+        const int slot = c * kPfKeys + skey;
+        const bool in = c < nch && slot < kend;
+        const bool fresh = !I8 && fused && slot >= c0; // a prompt key: from the inputs, rotated here
+        const int i = fresh ? min(slot - c0, t - 1) : 0;
+        const size_t arow = (((size_t)b * t + i) * pv.KVH + kvh) * kHeadDim + 8 * spart;
+        st.k = st.v = make_uint4(0, 0, 0, 0);
+        st.sk = st.sv = 0.f;
+        if constexpr (I8) {
+            // int8 pages (the prompt's rows appended before): 8 codes of K and of V; the first
+            // thread of each page's keys also takes its scales (0 for a page outside the pool,
+            // as the bf16 path's zero rows: score 0, no value)
+            if (in) {
                 const int blk = min(slot >> 4, kPfMaxPages - 1);
                 int page;
                 if constexpr (decltype(LDS)::value)
@@ -182,212 +161,231 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
                     page = tab[blk];
                 if (page >= 0 && page < pv.NB) {
                     const size_t poff = (size_t)page * page_elems + (slot & 15) * kHeadDim + 8 * spart;
-                    st.k = ld_stream(kpages + poff);
-                    st.v = ld_stream(vpages + poff);
+                    const uint2 kk = *(const uint2 *)(kpages8 + poff), vv = *(const uint2 *)(vpages8 + poff);
+                    st.k = make_uint4(kk.x, kk.y, 0, 0);
+                    st.v = make_uint4(vv.x, vv.y, 0, 0);
+                    if ((skey & 15) == 0 && spart == 0) {
+                        st.sk = pv.scales[tile_index(pv, layer, 0, page, kvh)];
+                        st.sv = pv.scales[tile_index(pv, layer, 1, page, kvh)];
+                    }
                 }
             }
-            st.rope = *(const uint4 *)(pv.rope16 + (size_t)(P.key_pos + i) * (kHeadDim / 2) + 4 * spart);
-            st.info = (in && fresh ? 1 : 0) | (in && fresh && last ? 2 : 0);
-        };
-
-        // B operands of S^T: query row 16 tile + l16, dims 32 kc + 8 g .. +7, rotated at its
-        // position and rounded to bf16 as the reference's bf16 q is.  The queries' loads and the
-        // first chunk's go out before any is used (rows past the prompt read row t - 1 and are
-        // zeroed after).
-        bf16x8_t qb[2][2];
-        f16x8_t qh[2][2];                // int8: the queries as f16, scaled by 2^-x per column
-        float qsum[2] = {0.f, 0.f}, qpow[2] = {1.f, 1.f}; // int8: their sums, 2^x
-        float m[2], lsum[2]; // running max (scaled, log2 units) and this lane's share of the sum
-        f32x4_t o[2][4];
-        Stage st;
-        {
-            uint4 qraw[2][2], qcs[2][2]; // q pieces; their 4 (cos, sin) pairs as packed bf16
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int qr = min(16 * max(tile[j], 0) + l16, t - 1);
-                const uint16_t *qp = (const uint16_t *)q + (((size_t)b * t + qr) * pv.H + h) * kHeadDim;
-                const uint32_t *cs = pv.rope16 + (size_t)(P.pos + qr) * (kHeadDim / 2);
-#pragma unroll
-                for (int kc = 0; kc < 2; ++kc) {
-                    qraw[j][kc] = *(const uint4 *)(qp + 32 * kc + 8 * g);
-                    qcs[j][kc] = *(const uint4 *)(cs + 16 * kc + 4 * g);
-                }
-            }
-            if (tq0 > 0)
-                issue(0, st, std::true_type{});
+            st.info = 0;
+            return;
+        }
+        if (in && fresh) {
+            st.k = ld_stream((const uint16_t *)knew + arow);
+            st.v = ld_stream((const uint16_t *)vnew + arow);
+        } else if (in) {
+            const int blk = min(slot >> 4, kPfMaxPages - 1);
+            int page;
+            if constexpr (decltype(LDS)::value)
+                page = spages[blk];
             else
-                issue(0, st, std::false_type{});
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                m[j] = -1e30f;
-                lsum[j] = 0.f;
-#pragma unroll
-                for (int dg = 0; dg < 4; ++dg) o[j][dg] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-                const bool live = tile[j] >= 0 && 16 * tile[j] + l16 < t;
-#pragma unroll
-                for (int kc = 0; kc < 2; ++kc) {
-                    const uint4 r = rotate8(qraw[j][kc], qcs[j][kc]);
-                    qb[j][kc] = as_bf16x8(live ? r : make_uint4(0, 0, 0, 0));
-                }
-                if constexpr (I8) queries_f16(qb[j], qh[j], qsum[j], qpow[j]);
+                page = tab[blk];
+            if (page >= 0 && page < pv.NB) {
+                const size_t poff = (size_t)page * page_elems + (slot & 15) * kHeadDim + 8 * spart;
+                st.k = ld_stream(kpages + poff);
+                st.v = ld_stream(vpages + poff);
             }
         }
-        __syncthreads(); // spages written
+        st.rope = *(const uint4 *)(pv.rope16 + (size_t)(P.key_pos + i) * (kHeadDim / 2) + 4 * spart);
+        st.info = (in && fresh ? 1 : 0) | (in && fresh && last ? 2 : 0);
+    };
 
-        auto step = [&](int c, Stage &st) {
-            const int buf = c & 1, kbase = c * kPfKeys, lb = buf * kPfKeys;
-            if constexpr (I8) {
-                // K codes as f16 1152 + c (one byte permute each: c ^ 0x80 under the f16 exponent of
-                // 1024), V codes as bf16 (exact); the pages' scales beside them
-                uint32_t hk[4], bv2[4];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const uint32_t kx = (i ? st.k.y : st.k.x) ^ 0x80808080u, vx = i ? st.v.y : st.v.x;
-                    hk[2 * i] = __builtin_amdgcn_perm(0x64646464u, kx, 0x04010400u);
-                    hk[2 * i + 1] = __builtin_amdgcn_perm(0x64646464u, kx, 0x04030402u);
-                    bv2[2 * i] = pack_bf16((float)(int8_t)(vx & 0xffu), (float)(int8_t)((vx >> 8) & 0xffu));
-                    bv2[2 * i + 1] = pack_bf16((float)(int8_t)((vx >> 16) & 0xffu), (float)(int8_t)(vx >> 24));
-                }
-                *(uint4 *)&ks[lb + skey][8 * spart] = make_uint4(hk[0], hk[1], hk[2], hk[3]);
-                *(uint4 *)&vs[lb + skey][8 * spart] = make_uint4(bv2[0], bv2[1], bv2[2], bv2[3]);
-                if ((skey & 15) == 0 && spart == 0) {
-                    ssc[buf][skey >> 4][0] = st.sk;
-                    ssc[buf][skey >> 4][1] = st.sv;
-                }
-            } else {
-            // rotate a prompt key at its position; store this thread's piece of the chunk
-            {
-                const uint4 kk = st.info & 1 ? rotate8(st.k, st.rope) : st.k;
-                if (st.info & 2) { // complete_kv: the prompt's rows go into their pages once
-                    const int slot = kbase + skey;
-                    const int page = spages[min(slot >> 4, kPfMaxPages - 1)];
-                    if (page >= 0 && page < pv.NB) {
-                        const size_t poff = (size_t)page * page_elems + (slot & 15) * kHeadDim + 8 * spart;
-                        st_stream(kpages + poff, kk);
-                        st_stream(vpages + poff, st.v);
-                    }
-                }
-                *(uint4 *)&ks[lb + skey][8 * spart] = kk;
-                *(uint4 *)&vs[lb + skey][8 * spart] = st.v;
-            }
-            }
-            issue(c + 1, st, std::true_type{});
-            __syncthreads(); // chunk c is in LDS; every reader of chunk c - 2 (same buffer) is done
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int r0 = c0 + 16 * tile[j]; // slot of the tile's first row
-                // skip a tile when every key of the chunk comes after all of its rows
-                if (tile[j] < 0 || kbase > r0 + 15) continue;
-                f32x4_t s[4];
-#pragma unroll
-                for (int kg = 0; kg < 4; ++kg) {
-                    s[kg] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int kc = 0; kc < 2; ++kc) {
-                        const uint4 a = *(const uint4 *)&ks[lb + 16 * kg + l16][32 * kc + 8 * g];
-                        if constexpr (I8)
-                            s[kg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), qh[j][kc],
-                                                                          s[kg], 0, 0, 0);
-                        else
-                            s[kg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), qb[j][kc], s[kg], 0, 0, 0);
-                    }
-                    if constexpr (I8) { // the 16 keys of group kg are one page: its K scale, the bias out
-                        const float f = ssc[buf][kg][0] * qpow[j];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) s[kg][r] = __builtin_fmaf(-1152.f, qsum[j], s[kg][r]) * f;
-                    }
-                }
-                // lane: query slot r0 + l16 against key slots kbase + 16 kg + 4 g + r
-                if (kbase + kPfKeys - 1 > r0) { // the chunk reaches past the tile's first row: mask
-                    const int qs = r0 + l16;
-#pragma unroll
-                    for (int kg = 0; kg < 4; ++kg)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            if (kbase + 16 * kg + 4 * g + r > qs) s[kg][r] = -INFINITY;
-                }
-                // the row's max: a chain of pairs (v_max3), then over the row's 4 lanes by row swaps
-                float mx = fmax_fin(s[0][0], s[0][1]);
-#pragma unroll
-                for (int e = 2; e < 16; e += 2) mx = fmaxf(fmaxf(mx, s[e >> 2][e & 3]), s[e >> 2][(e & 3) + 1]);
-                mx = swap_max<32>(swap_max<16>(mx));
-                // lazy rescaling, as in decode: the row's sum and accumulators move to a new max only
-                // when some row of the wave saw its max grow by more than 8 (log2 units); until then
-                // exponents are taken against the older max and stay below 2^8
-                const float mn = fmax_fin(m[j], mx * qmul);
-                if (__any(mn > m[j] + 8.f)) {
-                    const float alpha = fast_exp2(m[j] - mn);
-                    lsum[j] *= alpha;
-#pragma unroll
-                    for (int dg = 0; dg < 4; ++dg)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) o[j][dg][r] *= alpha;
-                    m[j] = mn;
-                }
-                const float mref = m[j];
-                float psum = 0.f;
-                uint32_t pk[4][2];
-#pragma unroll
-                for (int kg = 0; kg < 4; ++kg) {
-                    float p[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        p[r] = fast_exp2(__builtin_fmaf(s[kg][r], qmul, -mref));
-                        psum += p[r];
-                    }
-                    if constexpr (I8) { // P^T carries p sv (the page's V scale), so O needs none
-                        const float sv = ssc[buf][kg][1];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) p[r] *= sv;
-                    }
-                    pk[kg][0] = pack_bf16(p[0], p[1]);
-                    pk[kg][1] = pack_bf16(p[2], p[3]);
-                }
-                lsum[j] += psum;
-#pragma unroll
-                for (int kp = 0; kp < 2; ++kp) {
-                    // k slots: keys 32 kp + 4 g .. +3 (elements 0-3) and 32 kp + 16 + 4 g .. +3 (4-7)
-                    const bf16x8_t pb =
-                        as_bf16x8(make_uint4(pk[2 * kp][0], pk[2 * kp][1], pk[2 * kp + 1][0], pk[2 * kp + 1][1]));
-#pragma unroll
-                    for (int dg = 0; dg < 4; ++dg) {
-                        // V^T: lane gets dim 16 dg + l16 of the same eight keys, by two transposed reads
-                        const uint16_t *vp = &vs[lb + 32 * kp + 4 * g + (l16 >> 2)][16 * dg + 4 * (l16 & 3)];
-                        const uint2 lo = lds_read_tr16(vp), hi = lds_read_tr16(vp + 16 * kPfLd);
-                        const bf16x8_t a = as_bf16x8(make_uint4(lo.x, lo.y, hi.x, hi.y));
-                        o[j][dg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, o[j][dg], 0, 0, 0);
-                    }
-                }
-            }
-        };
-        for (int c = 0; c < nch; ++c) step(c, st);
-        __syncthreads(); // the next round's staging overwrites both buffers
-
-        // out[row][h][..] = O / l, the row's sum reduced over its 4 lanes.  The lane holds dims
-        // 16 dg + 4 g .. +3 of row l16; through rows 16 w .. 16 w + 15 of ks (free after the barrier
-        // above), each store instruction writes 8 whole 128-byte rows, so the non-temporal stores go
-        // out as full lines.
+    // B operands of S^T: query row 16 tile + l16, dims 32 kc + 8 g .. +7, rotated at its
+    // position and rounded to bf16 as the reference's bf16 q is.  The queries' loads and the
+    // first chunk's go out before any is used (rows past the prompt read row t - 1 and are
+    // zeroed after).
+    bf16x8_t qb[2][2];
+    f16x8_t qh[2][2];                // int8: the queries as f16, scaled by 2^-x per column
+    float qsum[2] = {0.f, 0.f}, qpow[2] = {1.f, 1.f}; // int8: their sums, 2^x
+    float m[2], lsum[2]; // running max (scaled, log2 units) and this lane's share of the sum
+    f32x4_t o[2][4];
+    Stage st;
+    {
+        uint4 qraw[2][2], qcs[2][2]; // q pieces; their 4 (cos, sin) pairs as packed bf16
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if (tile[j] < 0) continue;
-            const float l = swap_sum<32>(swap_sum<16>(lsum[j]));
-            const float inv = 1.0f / l;
-            uint16_t(*st)[kPfLd] = &ks[16 * w];
+            const int qr = min(16 * max(tile[j], 0) + l16, t - 1);
+            const uint16_t *qp = (const uint16_t *)q + (((size_t)b * t + qr) * pv.H + h) * kHeadDim;
+            const uint32_t *cs = pv.rope16 + (size_t)(P.pos + qr) * (kHeadDim / 2);
 #pragma unroll
-            for (int dg = 0; dg < 4; ++dg)
-                *(uint2 *)&st[l16][16 * dg + 4 * g] = make_uint2(pack_bf16(o[j][dg][0] * inv, o[j][dg][1] * inv),
-                                                                 pack_bf16(o[j][dg][2] * inv, o[j][dg][3] * inv));
-            // the lane index recomputed here (lane_here): hoisted out of the rounds, the output's
-            // address pieces were held across them and spilled
-            const int ln = lane_here(lane);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int r = (ln >> 3) + 8 * i, unit = ln & 7, qrow = 16 * tile[j] + r;
-                const uint4 v = *(const uint4 *)&st[r][8 * unit];
-                if (qrow < t) st_stream((uint16_t *)out + (((size_t)b * t + qrow) * pv.H + h) * kHeadDim + 8 * unit, v);
+            for (int kc = 0; kc < 2; ++kc) {
+                qraw[j][kc] = *(const uint4 *)(qp + 32 * kc + 8 * g);
+                qcs[j][kc] = *(const uint4 *)(cs + 16 * kc + 4 * g);
             }
         }
-        if (!last) __syncthreads(); // the next round's staging overwrites ks
+        issue(0, st, std::false_type{});
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            m[j] = -1e30f;
+            lsum[j] = 0.f;
+#pragma unroll
+            for (int dg = 0; dg < 4; ++dg) o[j][dg] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            const bool live = tile[j] >= 0 && 16 * tile[j] + l16 < t;
+#pragma unroll
+            for (int kc = 0; kc < 2; ++kc) {
+                const uint4 r = rotate8(qraw[j][kc], qcs[j][kc]);
+                qb[j][kc] = as_bf16x8(live ? r : make_uint4(0, 0, 0, 0));
+            }
+            if constexpr (I8) queries_f16(qb[j], qh[j], qsum[j], qpow[j]);
+        }
+    }
+    __syncthreads(); // spages written
+
+    auto step = [&](int c, Stage &st) {
+        const int buf = c & 1, kbase = c * kPfKeys, lb = buf * kPfKeys;
+        if constexpr (I8) {
+            // K codes as f16 1152 + c (one byte permute each: c ^ 0x80 under the f16 exponent of
+            // 1024), V codes as bf16 (exact); the pages' scales beside them
+            uint32_t hk[4], bv2[4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t kx = (i ? st.k.y : st.k.x) ^ 0x80808080u, vx = i ? st.v.y : st.v.x;
+                hk[2 * i] = __builtin_amdgcn_perm(0x64646464u, kx, 0x04010400u);
+                hk[2 * i + 1] = __builtin_amdgcn_perm(0x64646464u, kx, 0x04030402u);
+                bv2[2 * i] = pack_bf16((float)(int8_t)(vx & 0xffu), (float)(int8_t)((vx >> 8) & 0xffu));
+                bv2[2 * i + 1] = pack_bf16((float)(int8_t)((vx >> 16) & 0xffu), (float)(int8_t)(vx >> 24));
+            }
+            *(uint4 *)&ks[lb + skey][8 * spart] = make_uint4(hk[0], hk[1], hk[2], hk[3]);
+            *(uint4 *)&vs[lb + skey][8 * spart] = make_uint4(bv2[0], bv2[1], bv2[2], bv2[3]);
+            if ((skey & 15) == 0 && spart == 0) {
+                ssc[buf][skey >> 4][0] = st.sk;
+                ssc[buf][skey >> 4][1] = st.sv;
+            }
+        } else {
+        // rotate a prompt key at its position; store this thread's piece of the chunk
+        {
+            const uint4 kk = st.info & 1 ? rotate8(st.k, st.rope) : st.k;
+            if (st.info & 2) { // complete_kv: the prompt's rows go into their pages once
+                const int slot = kbase + skey;
+                const int page = spages[min(slot >> 4, kPfMaxPages - 1)];
+                if (page >= 0 && page < pv.NB) {
+                    const size_t poff = (size_t)page * page_elems + (slot & 15) * kHeadDim + 8 * spart;
+                    st_stream(kpages + poff, kk);
+                    st_stream(vpages + poff, st.v);
+                }
+            }
+            *(uint4 *)&ks[lb + skey][8 * spart] = kk;
+            *(uint4 *)&vs[lb + skey][8 * spart] = st.v;
+        }
+        }
+        issue(c + 1, st, std::true_type{});
+        __syncthreads(); // chunk c is in LDS; every reader of chunk c - 2 (same buffer) is done
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int r0 = c0 + 16 * tile[j]; // slot of the tile's first row
+            // skip a tile when every key of the chunk comes after all of its rows
+            if (tile[j] < 0 || kbase > r0 + 15) continue;
+            f32x4_t s[4];
+#pragma unroll
+            for (int kg = 0; kg < 4; ++kg) {
+                s[kg] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int kc = 0; kc < 2; ++kc) {
+                    const uint4 a = *(const uint4 *)&ks[lb + 16 * kg + l16][32 * kc + 8 * g];
+                    if constexpr (I8)
+                        s[kg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), qh[j][kc],
+                                                                      s[kg], 0, 0, 0);
+                    else
+                        s[kg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), qb[j][kc], s[kg], 0, 0, 0);
+                }
+                if constexpr (I8) { // the 16 keys of group kg are one page: its K scale, the bias out
+                    const float f = ssc[buf][kg][0] * qpow[j];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[kg][r] = __builtin_fmaf(-1152.f, qsum[j], s[kg][r]) * f;
+                }
+            }
+            // lane: query slot r0 + l16 against key slots kbase + 16 kg + 4 g + r
+            if (kbase + kPfKeys - 1 > r0) { // the chunk reaches past the tile's first row: mask
+                const int qs = r0 + l16;
+#pragma unroll
+                for (int kg = 0; kg < 4; ++kg)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (kbase + 16 * kg + 4 * g + r > qs) s[kg][r] = -INFINITY;
+            }
+            // the row's max: a chain of pairs (v_max3), then over the row's 4 lanes by row swaps
+            float mx = fmax_fin(s[0][0], s[0][1]);
+#pragma unroll
+            for (int e = 2; e < 16; e += 2) mx = fmaxf(fmaxf(mx, s[e >> 2][e & 3]), s[e >> 2][(e & 3) + 1]);
+            mx = swap_max<32>(swap_max<16>(mx));
+            // lazy rescaling, as in decode: the row's sum and accumulators move to a new max only
+            // when some row of the wave saw its max grow by more than 8 (log2 units); until then
+            // exponents are taken against the older max and stay below 2^8
+            const float mn = fmax_fin(m[j], mx * qmul);
+            if (__any(mn > m[j] + 8.f)) {
+                const float alpha = fast_exp2(m[j] - mn);
+                lsum[j] *= alpha;
+#pragma unroll
+                for (int dg = 0; dg < 4; ++dg)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[j][dg][r] *= alpha;
+                m[j] = mn;
+            }
+            const float mref = m[j];
+            float psum = 0.f;
+            uint32_t pk[4][2];
+#pragma unroll
+            for (int kg = 0; kg < 4; ++kg) {
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    p[r] = fast_exp2(__builtin_fmaf(s[kg][r], qmul, -mref));
+                    psum += p[r];
+                }
+                if constexpr (I8) { // P^T carries p sv (the page's V scale), so O needs none
+                    const float sv = ssc[buf][kg][1];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) p[r] *= sv;
+                }
+                pk[kg][0] = pack_bf16(p[0], p[1]);
+                pk[kg][1] = pack_bf16(p[2], p[3]);
+            }
+            lsum[j] += psum;
+#pragma unroll
+            for (int kp = 0; kp < 2; ++kp) {
+                // k slots: keys 32 kp + 4 g .. +3 (elements 0-3) and 32 kp + 16 + 4 g .. +3 (4-7)
+                const bf16x8_t pb =
+                    as_bf16x8(make_uint4(pk[2 * kp][0], pk[2 * kp][1], pk[2 * kp + 1][0], pk[2 * kp + 1][1]));
+#pragma unroll
+                for (int dg = 0; dg < 4; ++dg) {
+                    // V^T: lane gets dim 16 dg + l16 of the same eight keys, by two transposed reads
+                    const uint16_t *vp = &vs[lb + 32 * kp + 4 * g + (l16 >> 2)][16 * dg + 4 * (l16 & 3)];
+                    const uint2 lo = lds_read_tr16(vp), hi = lds_read_tr16(vp + 16 * kPfLd);
+                    const bf16x8_t a = as_bf16x8(make_uint4(lo.x, lo.y, hi.x, hi.y));
+                    o[j][dg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, o[j][dg], 0, 0, 0);
+                }
+            }
+        }
+    };
+    for (int c = 0; c < nch; ++c) step(c, st);
+    __syncthreads(); // every wave is done with both buffers
+
+    // out[row][h][..] = O / l, the row's sum reduced over its 4 lanes.  The lane holds dims
+    // 16 dg + 4 g .. +3 of row l16; through rows 16 w .. 16 w + 15 of ks (free after the barrier
+    // above), each store instruction writes 8 whole 128-byte rows, so the non-temporal stores go
+    // out as full lines.
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (tile[j] < 0) continue;
+        const float l = swap_sum<32>(swap_sum<16>(lsum[j]));
+        const float inv = 1.0f / l;
+        uint16_t(*st)[kPfLd] = &ks[16 * w];
+#pragma unroll
+        for (int dg = 0; dg < 4; ++dg)
+            *(uint2 *)&st[l16][16 * dg + 4 * g] = make_uint2(pack_bf16(o[j][dg][0] * inv, o[j][dg][1] * inv),
+                                                             pack_bf16(o[j][dg][2] * inv, o[j][dg][3] * inv));
+        // the lane index recomputed here (lane_here): hoisted out of the chunk loop, the output's
+        // address pieces were held across it and spilled
+        const int ln = lane_here(lane);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = (ln >> 3) + 8 * i, unit = ln & 7, qrow = 16 * tile[j] + r;
+            const uint4 v = *(const uint4 *)&st[r][8 * unit];
+            if (qrow < t) st_stream((uint16_t *)out + (((size_t)b * t + qrow) * pv.H + h) * kHeadDim + 8 * unit, v);
+        }
     }
 }
 
@@ -1411,6 +1409,8 @@ hipError_t launch_decode_gqa(const PoolView &pv, const BatchView &bv, int layer,
     return hipGetLastError();
 }
 
+static int prefill_rounds(int t) { return (t + kPfRound - 1) / kPfRound; }
+
 hipError_t launch_prefill_mfma(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
                                const void *v, void *out, float scale, bool fused, bool window, hipStream_t stream,
                                const LaunchTiming &tm) {
@@ -1426,7 +1426,7 @@ hipError_t launch_prefill_mfma(const PoolView &pv, const BatchView &bv, int laye
         XNP_LAUNCH(k_prefill_fast<false>, dim3(bv.n * pv.H), dim3(64 * kPfWaves), stream, tm, pv, bv, layer, q, k, v,
                    out, qmul);
     else
-        XNP_LAUNCH(k_prefill_mfma<DT_BF16>, dim3(bv.n * pv.H), dim3(64 * kPfWaves), stream, tm, pv, bv, layer, q, k, v,
+        XNP_LAUNCH(k_prefill_mfma<DT_BF16>, dim3(bv.n * pv.H * prefill_rounds(bv.t)), dim3(64 * kPfWaves), stream, tm, pv, bv, layer, q, k, v,
                    out, qmul, fused ? 1 : 0);
     return hipGetLastError();
 }
@@ -1437,7 +1437,7 @@ hipError_t launch_prefill_mfma_i8(const PoolView &pv, const BatchView &bv, int l
                                   float scale, hipStream_t stream, const LaunchTiming &tm) {
     if (pv.cache_dt != DT_I8 || pv.act_dt != DT_BF16) return hipErrorInvalidValue;
     const float qmul = scale * 1.4426950408889634f;
-    XNP_LAUNCH(k_prefill_mfma<DT_I8>, dim3(bv.n * pv.H), dim3(64 * kPfWaves), stream, tm, pv, bv, layer, q, nullptr,
+    XNP_LAUNCH(k_prefill_mfma<DT_I8>, dim3(bv.n * pv.H * prefill_rounds(bv.t)), dim3(64 * kPfWaves), stream, tm, pv, bv, layer, q, nullptr,
                nullptr, out, qmul, 0);
     return hipGetLastError();
 }
