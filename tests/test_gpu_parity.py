@@ -396,6 +396,25 @@ def test_window_caches_match_mimis_kv_cache(cache, act):
         assert pool.current_end(wids[i]) == contexts[i]  # rows held: the window, full
 
 
+# Steps of a few rows attend them in one launch (up to 4, and no more than the smallest window holds;
+# f32 runs longer steps 4 rows a launch): windows of 1 row, less than a page, a page, a ragged two and
+# a half and seven pages, empty, filling and full, more than 1024 groups (one wave each) and few
+# (eight waves), against the oracle's KvCache.
+@pytest.mark.parametrize("cache,act", [("bf16", "bf16"), ("f32", "f32")])
+@pytest.mark.parametrize("contexts", [(1, 24), (3, 3), (16, 40, 112), (40,) * 130])
+def test_a_few_window_rows_in_one_launch(cache, act, contexts):
+    L, H = 1, 8
+    pool = xnp.KvPool(num_layers=L, num_heads=H, num_blocks=8 * len(contexts), max_streams=len(contexts),
+                      max_blocks_per_stream=7, cache_dtype=cache, act_dtype=act, max_pos=4096, page_seed=4)
+    ids = [pool.init_window(c) for c in contexts]
+    orcs = [oracle.Window(L, H, 64, c, act=act) for c in contexts]
+    rng = np.random.default_rng(57)
+    for t in (2, 3, 4, 2, 1, 4, 3) if len(contexts) > 3 else (2, 3, 4, 2, 1, 3, 4) * 3 + (4,) * 24 + (3, 2, 1, 2):
+        _window_batch(pool, ids, orcs, t, L, H, act, cache, rng)
+    for i in range(0, len(contexts), 29 if len(contexts) > 3 else 1):
+        _assert_window_rows(pool, ids[i], orcs[i], contexts[i], L, H, cache)
+
+
 def test_int8_rows_holding_infinities_quantize_as_the_oracle():
     # An int8 page's scale is its rows' amax / 127, taken with IEEE maxima: a row holding an
     # infinity gives the page an infinite scale, its infinite elements code -127 (rint(inf / inf) is

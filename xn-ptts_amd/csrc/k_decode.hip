@@ -23,23 +23,36 @@ namespace xnp {
 // prompt-row kernel.  `pages` lists the stream's page ids by logical block (a decode record's
 // copy, or the block table).  With GQ > 1 each page is read once for the GQ heads: K is unpacked
 // (or taken by dot2) once per row, V once, and each head keeps its own online softmax.
-template <int CDT, bool ABF, int SPLIT, bool PREFIX, int GQ = 1>
+//
+// ROWS: the GQ queries are rows r0 = bv.wrow .. of a window step, all of query head h (at most
+// bv.wrows of them live), against the rows the window held before row r0 and the step's own.  Row e
+// sees position p = r0's position + e and the window - 1 before it: the held pages less the slots
+// its rows 0 .. e take (which hold the positions that left its window), then the new rows 0 .. e,
+// which go through the loop's arithmetic as one more page built from the inputs.  The rows are
+// appended once every wave has read the pages.
+template <int CDT, bool ABF, int SPLIT, bool PREFIX, int GQ = 1, bool ROWS = false>
 __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView &bv, int layer, const StreamRec &R,
                                             const int32_t *rec_pages, int h, const void *q, const void *knew,
                                             const void *vnew, void *out, float qmul, int fused) {
     using LN = Lanes<CDT>;
     constexpr int DPL = LN::DPL, LPR = LN::LPR, RPP = LN::RPP, NP = LN::NP, DEPTH = LN::DEPTH;
     constexpr int AE = ABF ? 2 : 4;
+    constexpr int NS = ROWS ? GQ : 1; // seen masks: one for every query, or one per window row
+    static_assert(!ROWS || (!PREFIX && CDT != DT_I8), "window rows: no prefix, no int8 (whose append rewrites pages)");
     __shared__ float part[SPLIT][GQ][kPartStride];
 
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int nb = R.nblk > w ? (R.nblk - w + SPLIT - 1) / SPLIT : 0; // this wave's pages
     const int kvh = h / (pv.H / pv.KVH);                               // the tiles the heads read
 
+    // ROWS: the slot of row e (distinct: a launch takes no more rows than the window holds)
+    const int slot0 = ROWS ? R.pos % R.window : 0;
+    auto row_slot = [&](int e) { return slot0 + e >= R.window ? slot0 + e - R.window : slot0 + e; };
+
     // Per-page metadata, lane j holding page w + j * SPLIT: page id, seen rows, int8 scales.
     // Past the wave's last page the lanes hold page 0 with no row seen.
     int my_page = 0, my_ok = 0;
-    uint32_t my_seen = 0;
+    uint32_t my_seen[NS] = {};
     float my_sk = 0.f, my_sv = 0.f;
     // issued with the header load: record slots past nblk hold stale ids and are masked below
     const int pg_raw = w + lane * SPLIT < pv.mbps ? rec_pages[w + lane * SPLIT] : -1;
@@ -55,7 +68,14 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
         if (!ok) seen = 0;
         my_page = ok ? pg : 0;
         my_ok = ok ? 1 : 0;
-        my_seen = seen;
+#pragma unroll
+        for (int e = 0; e < NS; ++e) {
+            if constexpr (ROWS) {
+                const int sl = row_slot(e);
+                if (e < bv.wrows && (sl >> 4) == blk) seen &= ~(1u << (sl & 15));
+            }
+            my_seen[e] = seen;
+        }
     }
 
     const uint4 *kbase = (const uint4 *)((const char *)pv.pages + tile_index(pv, layer, 0, 0, kvh) * (kBlock * kHeadDim * esize<CDT>()));
@@ -115,8 +135,9 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
     float qpow[GQ], ppow[GQ]; // H16: the power of two each query was scaled down by (f16_fit_exponent)
 #pragma unroll
     for (int e = 0; e < GQ; ++e) {
-        const char *qrow = (const char *)q + ((size_t)R.b * pv.H + h + e) * kHeadDim * AE;
-        rotated_q<DPL, ABF>(pv, qrow, c, R.pos, DOT2 || H16 ? 1.f : qmul, qw[e]);
+        const int er = ROWS ? min(e, bv.wrows - 1) : 0; // a dead row repeats the last one
+        const char *qrow = (const char *)q + ((size_t)(R.b + er) * pv.H + h + (ROWS ? 0 : e)) * kHeadDim * AE;
+        rotated_q<DPL, ABF>(pv, qrow, c, R.pos + er, DOT2 || H16 ? 1.f : qmul, qw[e]);
         if (two_q) rotated_q<DPL, ABF>(pv, qrow, c, R.pos_pre, DOT2 || H16 ? 1.f : qmul, qp[e]);
         if constexpr (DOT2) {
 #pragma unroll
@@ -165,8 +186,7 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
     }
 
     // One page's scores and softmax/accumulator update from its K and V registers.
-    auto process = [&](const uint4 (&kr)[NP], const uint4 (&vr)[NP], int j) {
-        const uint32_t seen = __builtin_amdgcn_readlane(my_seen, j);
+    auto process = [&](const uint4 (&kr)[NP], const uint4 (&vr)[NP], int j, const uint32_t (&seen)[NS]) {
         const int base = (w + j * SPLIT) * kBlock;
         float sk = 1.f, sv = 1.f;
         if constexpr (CDT == DT_I8) {
@@ -233,7 +253,7 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
                 if constexpr (CDT == DT_I8) dw[e] *= sk;
                 if constexpr (H16) dw[e] *= pre ? ppow[e] : qpow[e];
                 if constexpr (DOT2 || H16) dw[e] *= qmul;
-                s[e][p] = ((seen >> r) & 1u) ? dw[e] : -INFINITY;
+                s[e][p] = ((seen[ROWS ? e : 0] >> r) & 1u) ? dw[e] : -INFINITY;
             }
         }
         // Lazy rescaling: the accumulators move to a new max only when some lane's max grew by
@@ -267,7 +287,9 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
             // hold what the memory held before): zero them, since 0 * NaN would still be NaN.
             // int8 bytes always convert to finite values (scales start at 0 and are amax / 127),
             // so int8 rows need no zeroing.
-            const bool rs = (seen >> (g + RPP * p)) & 1u;
+            uint32_t any = seen[0];
+            if constexpr (ROWS) any |= seen[NS - 1]; // held pages: row 0's mask holds the others; new rows: the last's
+            const bool rs = (any >> (g + RPP * p)) & 1u;
             const uint4 vv = (CDT == DT_I8 || rs) ? vr[p] : make_uint4(0, 0, 0, 0);
             float x[DPL];
             unpack<CDT>(vv, x);
@@ -314,7 +336,39 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
 #pragma unroll
         for (int u = 0; u <= DEPTH; ++u) {
             load(kb[(u + DEPTH) % (DEPTH + 1)], vb[(u + DEPTH) % (DEPTH + 1)], j + u + DEPTH);
-            process(kb[u], vb[u], j + u);
+            uint32_t seen[NS];
+#pragma unroll
+            for (int e = 0; e < NS; ++e) seen[e] = __builtin_amdgcn_readlane(my_seen[e], j + u);
+            process(kb[u], vb[u], j + u, seen);
+        }
+    }
+    if constexpr (ROWS) {
+        // the step's own rows as one page (row e in tile row e), by the wave whose turn the next page is
+        if (w == R.nblk % SPLIT) {
+            uint4 kr[NP], vr[NP];
+            uint32_t seen[NS];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                const int e = min(g + RPP * p, bv.wrows - 1);
+                const size_t arow = ((size_t)(R.b + e) * pv.KVH + kvh) * kHeadDim * AE;
+                kr[p] = *(const uint4 *)((const char *)knew + arow + 16 * c);
+                vr[p] = *(const uint4 *)((const char *)vnew + arow + 16 * c);
+                if constexpr (CDT == DT_BF16) {
+                    kr[p] = rotate8(kr[p], *(const uint4 *)(pv.rope16 + (size_t)(R.pos + e) * (kHeadDim / 2) + 4 * c));
+                } else { // as append_row_wave rotates it
+                    float *x = (float *)&kr[p];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const float2 cs = pv.rope[(size_t)(R.pos + e) * (kHeadDim / 2) + 2 * c + i];
+                        const float a = x[2 * i] * cs.x, bb = x[2 * i + 1] * cs.y, d = x[2 * i] * cs.y, f = x[2 * i + 1] * cs.x;
+                        x[2 * i] = a - bb;
+                        x[2 * i + 1] = d + f;
+                    }
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < NS; ++e) seen[e] = (2u << min(e, bv.wrows - 1)) - 1u;
+            process(kr, vr, 0, seen);
         }
     }
 
@@ -355,10 +409,24 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
         }
     }
     __syncthreads();
+    if constexpr (ROWS) { // every wave has read the pages: the step's rows go into their slots
+        if (w == SPLIT - 1) {
+#pragma unroll
+            for (int e = 0; e < GQ; ++e) {
+                const int sl = row_slot(e);
+                const int pg = e < bv.wrows ? rec_pages[sl >> 4] : -1;
+                const size_t arow = ((size_t)(R.b + e) * pv.KVH + kvh) * kHeadDim * AE;
+                if (pg >= 0 && pg < pv.NB)
+                    append_row_wave<CDT, ABF>(pv, layer, pg, sl & 15, kvh, R.pos + e, (const char *)knew + arow,
+                                              (const char *)vnew + arow, false);
+            }
+        }
+    }
     if (w != 0) return;
     // wave 0 writes the heads' outputs, lane d owning dim d
 #pragma unroll
     for (int e = 0; e < GQ; ++e) {
+        if (ROWS && e >= bv.wrows) break;
         float M = -1e30f;
 #pragma unroll
         for (int k = 0; k < SPLIT; ++k) M = fmaxf(M, part[k][e][64]);
@@ -370,7 +438,7 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
             A = __builtin_fmaf(part[k][e][lane], a, A);
         }
         const float r = A / L;
-        const size_t o = ((size_t)R.b * pv.H + h + e) * kHeadDim + lane;
+        const size_t o = ((size_t)(R.b + (ROWS ? e : 0)) * pv.H + h + (ROWS ? 0 : e)) * kHeadDim + lane;
         if constexpr (ABF)
             ((uint16_t *)out)[o] = (uint16_t)bf16_bits(r);
         else
@@ -405,6 +473,27 @@ __global__ __launch_bounds__(64 * SPLIT) __attribute__((amdgpu_waves_per_eu(Lane
     if (bv.wrow >= 0) window_row(R, bv.wrow);
     attend_core<CDT, ABF, SPLIT, PREFIX, GQ>(pv, bv, layer, R, (const int32_t *)(rec + sizeof(StreamRec)), slot * GQ,
                                              q, knew, vnew, out, qmul, fused);
+}
+
+// Rows bv.wrow .. bv.wrow + bv.wrows - 1 of a window step (2 to NR of them: Mimi's decoder takes 2 a
+// frame) in one launch, one work group per (stream, head): the window is read once for all of them,
+// where a launch per row read it per row.  500 windows of up to 250 rows, 2 rows, 2 layers:
+// 186 -> 169 us a step, bound by the host then, 104 us since the plan is composed faster.  One query head per kv
+// head only (a group that shares its kv head with another would append while the other reads).
+template <int CDT, bool ABF, int SPLIT, int NR>
+__global__ __launch_bounds__(64 * SPLIT) __attribute__((amdgpu_waves_per_eu(Lanes<CDT>::WAVES))) void k_window_rows(
+    PoolView pv, BatchView bv, int layer, const void *q, const void *knew, const void *vnew, void *out, float qmul) {
+    const int b = blockIdx.x, full = bv.n / 8 * 8; // XCD runs as in k_decode
+    const int sidx = b < full * pv.H ? b / (8 * pv.H) * 8 + b % 8 : full + (b - full * pv.H) / pv.H;
+    const int h = b < full * pv.H ? b % (8 * pv.H) / 8 : (b - full * pv.H) % pv.H;
+    const char *rec = bv.recs + (size_t)sidx * bv.rec_stride;
+    StreamRec R = *(const StreamRec *)rec;
+    R.b += bv.wrow;
+    R.pos += bv.wrow;
+    R.span = min(R.pos, R.window); // the rows held before row bv.wrow
+    R.nblk = (R.span + kBlock - 1) / kBlock;
+    attend_core<CDT, ABF, SPLIT, false, NR, true>(pv, bv, layer, R, (const int32_t *)(rec + sizeof(StreamRec)), h, q, knew,
+                                                  vnew, out, qmul, 0);
 }
 
 // Prompt rows (transformer.rs:231-248), after k_append has written all t rows: row i of a stream
@@ -536,6 +625,37 @@ static hipError_t prefill_rows_impl(const PoolView &pv, const BatchView &bv, int
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+template <int CDT, bool ABF, int NR>
+static hipError_t window_rows_impl(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
+                                   const void *v, void *out, float scale, hipStream_t stream, const LaunchTiming &tm) {
+    const float qmul = scale * 1.4426950408889634f;
+    const dim3 grid(bv.n * pv.H);
+#define XNP_WROWS(S) XNP_LAUNCH((k_window_rows<CDT, ABF, S, NR>), grid, dim3(64 * S), stream, tm, pv, bv, layer, q, k, v, out, qmul)
+    switch (bv.split) {
+    case 1: XNP_WROWS(1); break;
+    case 2: XNP_WROWS(2); break;
+    case 4: XNP_WROWS(4); break;
+    case 8: XNP_WROWS(8); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef XNP_WROWS
+    return hipGetLastError();
+}
+
+int window_rows_max(const PoolView &pv) { return pv.cache_dt == DT_I8 || pv.H != pv.KVH ? 1 : 4; }
+
+hipError_t launch_window_rows(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
+                              const void *v, void *out, float scale, hipStream_t stream, const LaunchTiming &tm) {
+    if (bv.n == 0) return hipSuccess;
+    if (bv.wrows < 1 || bv.wrows > window_rows_max(pv)) return hipErrorInvalidValue;
+    if (bv.wrows == 1) return launch_decode(pv, bv, layer, q, k, v, out, scale, true, stream, tm);
+    if (pv.cache_dt == DT_F32)
+        return bv.wrows == 2 ? window_rows_impl<DT_F32, false, 2>(pv, bv, layer, q, k, v, out, scale, stream, tm)
+                             : window_rows_impl<DT_F32, false, 4>(pv, bv, layer, q, k, v, out, scale, stream, tm);
+    return bv.wrows == 2 ? window_rows_impl<DT_BF16, true, 2>(pv, bv, layer, q, k, v, out, scale, stream, tm)
+                         : window_rows_impl<DT_BF16, true, 4>(pv, bv, layer, q, k, v, out, scale, stream, tm);
 }
 
 hipError_t launch_window_prefill(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,

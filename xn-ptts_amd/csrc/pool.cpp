@@ -77,7 +77,7 @@ struct Stream {
 
 // Window steps of more rows than this on a bf16 pool run as one windowed prefill on MFMA plus an
 // append; shorter ones (Mimi's decoder takes 2 a frame), and every window step on f32 and int8 pools,
-// run row by row through the decode kernel.
+// run a few rows a launch (window_rows_max) through the decode's core.
 constexpr int32_t kWindowRowByRow = 4;
 
 // The window's blocks a step of t rows from position p writes: those of the slots the last
@@ -150,7 +150,8 @@ struct xnp_pool {
         std::vector<int32_t> ids;
         std::vector<std::pair<int32_t, int32_t>> taken; // (stream, block) pages taken by begin
         BatchView bv{};
-        bool wsteps = false; // a step of several rows on window caches: one decode per row
+        bool wsteps = false; // a step of several rows on window caches
+        int32_t wmin = 0;    // its smallest window
     } batch;
 
     PoolView view() const {
@@ -1104,7 +1105,7 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
     }
     if (t > 1 && windows && windows != n)
         return fail(XNP_E_INVALID, "a step of %d rows holds window caches only, or none", t);
-    const bool wsteps = t > 1 && windows; // one decode per row, each over its own records
+    const bool wsteps = t > 1 && windows;
     if (wsteps && pool->d.cache_dtype == XNP_I8 && pool->d.num_kv_heads < pool->d.num_heads)
         return fail(XNP_E_INVALID, "an int8 window cache with grouped heads takes one row a step");
     if (need > (int)pool->free_pages.size())
@@ -1231,7 +1232,8 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
         B.bv.split = std::max(B.bv.split, decode_min_split(pool->view(), B.bv.prefix != 0));
     {
         const int gq = t == 1 ? decode_heads_per_group(pool->view(), B.bv.prefix != 0) : 1;
-        const int64_t groups = (int64_t)n * t * pool->d.num_heads / gq;
+        // (a window step's launch attends its rows together, one group per (stream, head))
+        const int64_t groups = (int64_t)n * (wsteps ? 1 : t) * pool->d.num_heads / gq;
         while (!pool->d.decode_split && B.bv.split < 8 && groups * B.bv.split < 1024)
             B.bv.split *= 2;
     }
@@ -1313,6 +1315,12 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
     B.bv.rec_stride = pool->rec_stride;
     B.bv.masks = (const uint32_t *)(pool->dbatch + o_masks);
     B.bv.wrow = -1;
+    B.bv.wrows = 0;
+    B.wmin = 0;
+    if (wsteps) {
+        B.wmin = pool->streams[ids[0]].window;
+        for (int32_t i = 1; i < n; i++) B.wmin = std::min(B.wmin, pool->streams[ids[i]].window);
+    }
     B.bv.n = n;
     B.bv.t = t;
     B.wsteps = wsteps;
@@ -1375,7 +1383,7 @@ extern "C" xnp_status xnp_attend(xnp_pool *pool, int32_t layer, const void *q, c
                                  void *out, float scale, void *hip_stream) {
     if (!pool) return fail(XNP_E_INVALID, "null argument");
     if (pool->batch.open && pool->batch.wsteps) {
-        // window caches, several rows: row by row, each a fused append + decode over its records
+        // window caches, several rows: up to window_rows_max a launch, each a fused append + decode
         auto &B = pool->batch;
         if (xnp_status st = batch_call(pool, layer, hip_stream, false, true)) return st;
         if (B.n > 0 && (!q || !k || !v || !out)) return fail(XNP_E_INVALID, "null q, k, v or out");
@@ -1389,10 +1397,12 @@ extern "C" xnp_status xnp_attend(xnp_pool *pool, int32_t layer, const void *q, c
             return XNP_OK;
         }
         BatchView bv = B.bv;
-        for (int32_t r = 0; r < B.t; r++) {
-            bv.wrow = r; // the kernel derives row r's record from the step's
-            HIP_TRY(launch_decode(pool->view(), bv, layer, q, k, v, out, scale, true, B.stream,
-                                  r == 0 ? tm : LaunchTiming()),
+        const int32_t most = std::min(window_rows_max(pool->view()), B.wmin); // the rows' slots distinct
+        for (int32_t r = 0; r < B.t; r += bv.wrows) {
+            bv.wrow = r; // the kernel derives the rows' record from the step's
+            bv.wrows = std::min(most, B.t - r);
+            HIP_TRY(launch_window_rows(pool->view(), bv, layer, q, k, v, out, scale, B.stream,
+                                       r == 0 ? tm : LaunchTiming()),
                     "attend");
         }
         return XNP_OK;

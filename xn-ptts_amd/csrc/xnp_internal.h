@@ -67,7 +67,8 @@ struct BatchView {
     int32_t n, t, rec_stride;
     int32_t split;  // waves per (stream, head) work group
     int32_t prefix; // 1 if some stream of the batch is an absolute ring keeping a prefix
-    int32_t wrow;   // a window step run row by row: the row this launch attends (-1 otherwise)
+    int32_t wrow;   // a window step run a few rows a launch: the first row this launch attends (-1 otherwise)
+    int32_t wrows;  // ... and how many it attends
     int32_t kmax;   // a prompt step (t > 1): the most key slots a stream of it attends, write_slot + t
 };
 
@@ -153,6 +154,11 @@ hipError_t launch_prefill(const PoolView &pv, const BatchView &bv, int layer, co
 // append of the last min(t, window) rows into their slots, (p + i) % window.
 hipError_t launch_window_prefill(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
                                  const void *v, void *out, float scale, hipStream_t stream, const LaunchTiming &timing);
+// Rows bv.wrow .. bv.wrow + bv.wrows - 1 of a window step, attended and appended in one launch; at most
+// window_rows_max of them (1 on int8 pools and grouped heads: row by row).
+int window_rows_max(const PoolView &pv);
+hipError_t launch_window_rows(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
+                              const void *v, void *out, float scale, hipStream_t stream, const LaunchTiming &timing);
 hipError_t launch_window_append(const PoolView &pv, const BatchView &bv, int layer, const void *k, const void *v,
                                 hipStream_t stream);
 hipError_t launch_evict_rotate(const PoolView &pv, const EvictRow *rows, int n,
