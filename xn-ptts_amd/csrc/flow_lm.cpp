@@ -172,6 +172,8 @@ struct xnp_flow_lm {
     uint16_t *bh = nullptr, *bh2 = nullptr;
     int32_t *dids = nullptr;
     int32_t *hids = nullptr; // pinned staging of token ids
+    hipEvent_t ids_read = nullptr; // the last upload from hids has completed
+    bool ids_pending = false;
     float *cond_vec = nullptr; // [d_model]: the model's summed conditions (condition_providers)
     bool has_cond = false;     // cond_vec is set
     std::vector<void *> allocs;
@@ -181,6 +183,8 @@ struct xnp_flow_lm {
 static void fl_free(xnp_flow_lm *lm) {
     if (lm->graph.exec) (void)hipGraphExecDestroy(lm->graph.exec);
     for (void *p : lm->allocs) (void)hipFree(p);
+    if (lm->ids_pending) (void)hipEventSynchronize(lm->ids_read);
+    if (lm->ids_read) (void)hipEventDestroy(lm->ids_read);
     if (lm->hids) (void)hipHostFree(lm->hids);
     delete lm;
 }
@@ -253,6 +257,7 @@ extern "C" xnp_status xnp_flow_lm_create(xnp_pool *pool, const xnp_flow_lm_desc 
     if ((e = dalloc((void **)&lm->dids, sizeof(int32_t) * M)) != hipSuccess) return fail_hip(e, "flow LM ids");
     if ((e = hipHostMalloc((void **)&lm->hids, sizeof(int32_t) * M, hipHostMallocDefault)) != hipSuccess)
         return fail_hip(e, "pinned ids");
+    if ((e = hipEventCreateWithFlags(&lm->ids_read, hipEventDisableTiming)) != hipSuccess) return fail_hip(e, "ids event");
     if ((e = hipMemcpy(lm->w, weights, sizeof(float) * L.total, hipMemcpyHostToDevice)) != hipSuccess)
         return fail_hip(e, "weight upload");
     // every block's adaLN_modulation rows, then the final layer's, stacked
@@ -429,10 +434,13 @@ extern "C" xnp_status xnp_flow_lm_prompt_text(xnp_flow_lm *lm, const int32_t *id
                              lm->d.n_bins + 1);
     hipStream_t hs = (hipStream_t)hip_stream;
     FL_TRY(hipSetDevice(pool_desc(lm->pool)->device), "hipSetDevice");
-    // the previous call's upload from the staging buffer has finished once the stream reaches here
-    FL_TRY(hipStreamSynchronize(hs), "staging");
+    // wait for the previous call's upload from the staging buffer alone, not for the stream's work
+    if (lm->ids_pending) FL_TRY(hipEventSynchronize(lm->ids_read), "staging");
+    lm->ids_pending = false;
     std::memcpy(lm->hids, tokens, sizeof(int32_t) * M);
     FL_TRY(hipMemcpyAsync(lm->dids, lm->hids, sizeof(int32_t) * M, hipMemcpyHostToDevice, hs), "token upload");
+    FL_TRY(hipEventRecord(lm->ids_read, hs), "token upload");
+    lm->ids_pending = true;
     if (xnp_status st = xnp_batch_begin(lm->pool, ids, n, t, hip_stream)) return st;
     xnp_status st;
     if (lm->d.precision == XNP_FLOW_Q8) {

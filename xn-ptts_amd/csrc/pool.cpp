@@ -68,8 +68,27 @@ struct Stream {
     int32_t current_end = 0;
     std::vector<int32_t> blocks; // logical block -> page, -1 where none
     int32_t ring = RING_NONE, write = 0, filled = 0, prefix = 0, shift = 0;
-    std::vector<uint8_t> valid;
+    // a ring's valid slots, as the bits the decode's masks are made of (a step's plan copies words)
+    std::vector<uint32_t> valid;
     int32_t nvalid = 0; // valid slots of the ring
+    bool holds(int32_t slot) const { return (valid[slot >> 5] >> (slot & 31)) & 1u; }
+    void set_valid(int32_t s0, int32_t s1) { // slots [s0, s1)
+        for (int32_t sl = s0; sl < s1;) {
+            const int32_t n = std::min(s1 - sl, 32 - (sl & 31));
+            valid[sl >> 5] |= (n == 32 ? ~0u : (1u << n) - 1u) << (sl & 31);
+            sl += n;
+        }
+    }
+    void clear_valid(int32_t slot) { valid[slot >> 5] &= ~(1u << (slot & 31)); }
+    int32_t count_valid(int32_t s0, int32_t s1) const { // of slots [s0, s1)
+        int32_t c = 0;
+        for (int32_t sl = s0; sl < s1;) {
+            const int32_t n = std::min(s1 - sl, 32 - (sl & 31));
+            c += __builtin_popcount(valid[sl >> 5] >> (sl & 31) & (n == 32 ? ~0u : (1u << n) - 1u));
+            sl += n;
+        }
+        return c;
+    }
     // Mimi's KvCache (transformer.rs:257-318): an absolute ring of `window` slots that places its
     // rows itself, row p in slot p % window, each overwriting the row that just left the window
     int32_t window = 0;
@@ -82,16 +101,14 @@ constexpr int32_t kWindowRowByRow = 4;
 
 // The window's blocks a step of t rows from position p writes: those of the slots the last
 // min(t, window) rows land in, (p + i) % window (an earlier row's slot is taken again by a later one).
+// In row order: those slots are one cyclic run, so the blocks from its first slot's on, then, past the
+// window's end, the ones from 0 that the first stretch did not visit.
 template <class F> void window_blocks(const Stream &s, int64_t p, int32_t t, F &&each) {
-    const int32_t nb = (s.window + kBlock - 1) / kBlock;
-    std::vector<uint8_t> hit(nb, 0);
-    for (int64_t r = std::max<int64_t>(0, t - s.window); r < t; r++) {
-        const int32_t b = (int32_t)((p + r) % s.window) / kBlock;
-        if (!hit[b]) {
-            hit[b] = 1;
-            each(b);
-        }
-    }
+    const int32_t n = std::min(t, s.window), first = (int32_t)((p + t - n) % s.window), end = first + n;
+    const int32_t b0 = first / kBlock;
+    for (int32_t b = b0; b <= (std::min(end, s.window) - 1) / kBlock; b++) each(b);
+    if (end > s.window)
+        for (int32_t b = 0; b <= std::min((end - s.window - 1) / kBlock, b0 - 1); b++) each(b);
 }
 
 // A pinned host buffer an upload is composed in; reused once its copy has completed.
@@ -766,8 +783,7 @@ extern "C" xnp_status xnp_stream_info_get(const xnp_pool *pool, int32_t id, xnp_
     out->ring_prefix = s->prefix;
     out->window = s->window;
     out->ring_shift = s->shift;
-    int32_t in_view = 0, blocks = 0, shared = 0;
-    for (uint8_t v : s->valid) in_view += v;
+    int32_t in_view = s->nvalid, blocks = 0, shared = 0;
     for (int32_t p : s->blocks)
         if (p >= 0) {
             blocks++;
@@ -795,7 +811,7 @@ extern "C" xnp_status xnp_ring_valid(const xnp_pool *pool, int32_t id, uint8_t *
     const Stream *s = pool->get(id);
     if (!s) return fail(XNP_E_STREAM, "no open stream %d", id);
     for (int32_t i = 0; i < std::min(cap, s->capacity); i++)
-        valid[i] = s->ring == RING_NONE ? (i < s->current_end) : s->valid[i];
+        valid[i] = s->ring == RING_NONE ? (i < s->current_end) : s->holds(i);
     return XNP_OK;
 }
 
@@ -922,8 +938,8 @@ extern "C" xnp_status xnp_ring_start(xnp_pool *pool, int32_t id, int32_t mode, i
     if (!pool->host_only) HIP_TRY(hipSetDevice(pool->d.device), "hipSetDevice");
     if (xnp_status st = pool->unshare(id, (hipStream_t)hip_stream)) return st;
     const int32_t used = s->current_end;
-    s->valid.assign(s->capacity, 0);
-    for (int32_t i = 0; i < used; i++) s->valid[i] = 1;
+    s->valid.assign((s->capacity + 31) / 32, 0u);
+    s->set_valid(0, used);
     s->nvalid = used;
     s->ring = mode;
     s->write = used;
@@ -962,7 +978,7 @@ extern "C" xnp_status xnp_ring_evict(xnp_pool *pool, int32_t id, int32_t prefix,
     // Every slot is checked before any change (transformer.rs:896-901).
     for (int32_t j = 0; j < count; j++) {
         const int32_t sl = slots[j];
-        if (sl < prefix || sl < 0 || sl >= s->capacity || !s->valid[sl])
+        if (sl < prefix || sl < 0 || sl >= s->capacity || !s->holds(sl))
             return fail(XNP_E_EVICT, "slot %d holds no row past the prefix", sl);
     }
     std::vector<EvictRow> rows;
@@ -970,7 +986,7 @@ extern "C" xnp_status xnp_ring_evict(xnp_pool *pool, int32_t id, int32_t prefix,
         for (int32_t sl = prefix; sl < s->filled; sl++) {
             bool evicted = false;
             for (int32_t j = 0; j < count && !evicted; j++) evicted = slots[j] == sl;
-            if (s->valid[sl] && !evicted) rows.push_back({id, sl});
+            if (s->holds(sl) && !evicted) rows.push_back({id, sl});
         }
         // The rows must fit one upload (max_blocks_per_stream * 16 of them always do).
         if (!pool->host_only && !rows.empty()) {
@@ -993,8 +1009,8 @@ extern "C" xnp_status xnp_ring_evict(xnp_pool *pool, int32_t id, int32_t prefix,
         }
     }
     for (int32_t j = 0; j < count; j++)
-        if (s->valid[slots[j]]) {
-            s->valid[slots[j]] = 0;
+        if (s->holds(slots[j])) {
+            s->clear_valid(slots[j]);
             s->nvalid--;
         }
     if (s->ring == RING_ABSOLUTE) s->shift += count;
@@ -1014,9 +1030,7 @@ extern "C" xnp_status xnp_ring_slide(xnp_pool *pool, int32_t id, int32_t prefix,
         return fail(XNP_E_INVALID, "slide over %d slots past %d with a window of %d, dropping %d, at step %lld",
                     span, prefix, window, drop, (long long)step);
     // valid slots in [prefix, prefix + span): the ring's count less those outside the window
-    int32_t in_view = s->nvalid;
-    for (int32_t sl = 0; sl < prefix; sl++) in_view -= s->valid[sl];
-    for (int32_t sl = prefix + span; sl < s->capacity; sl++) in_view -= s->valid[sl];
+    const int32_t in_view = s->nvalid - s->count_valid(0, prefix) - s->count_valid(prefix + span, s->capacity);
     if (in_view == window) {
         // s2s.rs:324-332: frames take the slots after the prefix in turn, so the oldest are the
         // next ones round.
@@ -1089,7 +1103,7 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
             windows++;
         } else if (s->ring != RING_NONE) {
             if (t != 1) return fail(XNP_E_RING, "a ring cache takes one row at a time, not %d", t);
-            if (s->valid[s->write]) return fail(XNP_E_RING, "ring slot %d still holds a row, evict it first", s->write);
+            if (s->holds(s->write)) return fail(XNP_E_RING, "ring slot %d still holds a row, evict it first", s->write);
             need += s->blocks[s->write / kBlock] < 0;
             last_pos = s->current_end + (s->ring == RING_ABSOLUTE ? s->shift : 0);
         } else {
@@ -1196,15 +1210,14 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
             P.span = std::max(s.filled, s.write + 1);
             P.ring = 1;
             // RingSlots::decode_mask (transformer.rs:42-52): valid slots and the write slot.
-            P.mask_off = (int32_t)masks.size();
-            const int words = (P.span + 31) / 32;
-            masks.resize(masks.size() + words, 0u);
-            for (int32_t sl = 0; sl < P.span; sl++)
-                if (s.valid[sl] || sl == s.write) masks[P.mask_off + sl / 32] |= 1u << (sl % 32);
-            const int32_t b0 = s.write / kBlock * kBlock, b1 = std::min(b0 + kBlock, s.capacity);
-            int other = 0;
-            for (int32_t sl = b0; sl < b1; sl++) other |= (sl != s.write && s.valid[sl]);
-            P.fresh = !other;
+            // Bits past the span are no valid slot's.  A step of several rows attends without masks.
+            if (t == 1) {
+                P.mask_off = (int32_t)masks.size();
+                masks.insert(masks.end(), s.valid.begin(), s.valid.begin() + (P.span + 31) / 32);
+                masks[P.mask_off + s.write / 32] |= 1u << (s.write % 32);
+            }
+            const int32_t b0 = s.write / kBlock * kBlock;
+            P.fresh = s.count_valid(b0, std::min(b0 + kBlock, s.capacity)) == (s.holds(s.write) ? 1 : 0);
             if (s.window) {
                 // the held rows are positions p - held .. p - 1, the oldest in slot (p - held) % window
                 P.window = s.window;
@@ -1215,8 +1228,13 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
     // decode order: longest streams first, so the short ones fill the tail of the launch
     std::vector<int32_t> order(n);
     for (int32_t i = 0; i < n; i++) order[i] = i;
-    if (t == 1)
-        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return plans[a].span > plans[b].span; });
+    if (t == 1) { // by counting the spans, equal ones in the batch's order
+        std::vector<int32_t> at(pool->d.max_blocks_per_stream * kBlock + 2, 0);
+        for (int32_t i = 0; i < n; i++) at[plans[i].span]++;
+        int32_t before = 0;
+        for (size_t sp = at.size(); sp-- > 0;) before += std::exchange(at[sp], before);
+        for (int32_t i = 0; i < n; i++) order[at[plans[i].span]++] = i;
+    }
     // waves per decode work group, unless the caller fixed them: the pool's default (the fewest
     // whose lanes index a stream's pages), at least two on MFMA; and a batch of few groups fills
     // few CUs, so give each group more waves (a larger split only raises the pages a group can
@@ -1448,13 +1466,13 @@ extern "C" xnp_status xnp_batch_end(xnp_pool *pool) {
             // newest in slot p % window
             const int64_t p = (int64_t)s.current_end + s.shift + B.t;
             const int32_t held = (int32_t)std::min<int64_t>(p, s.window);
-            for (int32_t sl = s.filled; sl < held; sl++) s.valid[sl] = 1;
+            s.set_valid(std::min(s.filled, held), held);
             s.nvalid = s.filled = s.current_end = held;
             s.shift = (int32_t)(p - held);
             s.write = (int32_t)(p % s.window);
         } else if (s.ring != RING_NONE) {
             // complete_kv's ring branch, transformer.rs:74-79 (begin refused a valid write slot)
-            s.valid[s.write] = 1;
+            s.set_valid(s.write, s.write + 1);
             s.nvalid++;
             s.filled = std::max(s.filled, s.write + 1);
             s.current_end += 1;

@@ -15,7 +15,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
-from .kv import _check, _ptr, _stream, load_library
+from .kv import _check, _int_array, _ptr, _stream, load_library
 
 FREQ_DIM = 256  # the time embedders' frequency embedding (mlp.rs:186-193)
 
@@ -179,7 +179,7 @@ class FlowLM:
         latent_out [n][ldim], eos_out [n], conditions [n][d_model] (each stream's
         FlowLMState::conditions; None: the model's, if set) -- f32 device tensors.  graph: replay a
         recording of the frame's launches (xnp_flow_lm_step_graph; needs a non-null stream)."""
-        arr = (ctypes.c_int32 * len(ids))(*ids)
+        _, arr = _int_array(ids, "i", ctypes.c_int32)
         fn = self._lib.xnp_flow_lm_step_graph if graph else self._lib.xnp_flow_lm_step
         _check(fn(self._h, arr, len(ids), _ptr(latent_in), _ptr(conditions), _ptr(noise), _ptr(latent_out),
                   _ptr(eos_out), _stream(stream)))

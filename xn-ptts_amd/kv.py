@@ -16,6 +16,7 @@ kernels).  A refused call raises XnpError carrying the library's status and mess
 """
 from __future__ import annotations
 
+import array
 import ctypes
 import os
 from typing import Iterable, Optional, Sequence
@@ -216,6 +217,21 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
+def _int_array(values, code: str, ctype):
+    """values (whole numbers, a sequence or an array) as a C array for one call: the array object to
+    keep alive, and what ctypes passes.  array.array converts a list several times as fast as ctypes
+    does; what it refuses (a number out of range, an empty list's address) goes the ctypes way."""
+    try:
+        a = array.array(code, values)
+        if len(a):
+            return a, (ctype * len(a)).from_buffer(a)
+    except (OverflowError, TypeError):
+        values = [int(x) for x in values] if code == "q" else values
+        a = values
+    c = (ctype * max(len(a), 1))(*a)
+    return c, c
+
+
 def _stream(stream) -> Optional[int]:
     if stream is not None:
         return stream
@@ -386,8 +402,9 @@ class KvPool:
         """slide() over many streams, stream i at steps[i], in one call."""
         ids = list(ids)
         n = len(ids)
-        arr = (_i32 * max(n, 1))(*ids)
-        st = (ctypes.c_int64 * max(n, 1))(*[int(x) for x in steps])
+        _, arr = _int_array(ids, "i", _i32)
+        steps = steps.tolist() if hasattr(steps, "tolist") else list(steps)
+        _, st = _int_array(steps, "q", ctypes.c_int64)
         failed = _i32(-1)
         _check(self._lib.xnp_ring_slide_batch(self._h, arr, n, prefix, span, window, drop, st,
                                               ctypes.byref(failed), _stream(stream)))
@@ -395,7 +412,7 @@ class KvPool:
     # -- a batched step -----------------------------------------------------------------------
     def begin(self, ids: Iterable[int], t: int = 1, stream=None):
         ids = list(ids)
-        arr = (_i32 * max(len(ids), 1))(*ids)
+        _, arr = _int_array(ids, "i", _i32)
         self._stream_h = _stream(stream)
         _check(self._lib.xnp_batch_begin(self._h, arr, len(ids), t, self._stream_h))
 
