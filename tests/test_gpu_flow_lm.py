@@ -87,6 +87,30 @@ def test_flow_lm_prompt_and_frames_match_the_oracle():
                 assert rel_err(rows.cpu().numpy(), vals) <= 1e-5, (i, layer, kv)
 
 
+# From 16 rows a prompt's f32 linears run on 16- and 32-row MFMA tiles, the LayerNorms inside them: prompts
+# of one row less than a tile, a tile, one more, ragged two and a half (two streams), and 400 rows (two
+# row tiles a group), with K of 256, 512, 1024 and one that no slice divides (the flow LM's FF 1500), and
+# N of ragged column tiles, against the oracle: the rows every layer's cache got and the frame after.
+@pytest.mark.parametrize("n,t,ff,dm", [(1, 15, 1024, 512), (1, 16, 1500, 512), (1, 17, 256, 256), (2, 20, 2044, 512),
+                                       (2, 200, 1024, 256)])
+def test_f32_prompts_on_row_tiles_match_the_oracle(n, t, ff, dm):
+    cfg = fl.FlowLMConfig(d_model=dm, num_heads=dm // 64, num_layers=2, flow_depth=1, flow_dim=256, dim_feedforward=ff,
+                          n_bins=100)
+    blob = fl.random_weights(cfg, 98 + t, std=0.04, unit_norms=False)
+    rng = np.random.default_rng(99 + t)
+    tokens = rng.integers(0, cfg.n_bins + 1, (n, t)).astype(np.int32)
+    noise = (0.5 * rng.standard_normal((1, n, cfg.ldim))).astype(np.float32)
+    pool, ids, sts, _ = run_pair(cfg, blob, tokens, 1, noise, t + 4)
+    for i in range(n):
+        for layer in range(cfg.num_layers):
+            for kv in (0, 1):
+                rows = torch.empty((t + 1, cfg.num_heads, 64), dtype=torch.float32, device=DEV)
+                pool.read_rows(ids[i], layer, kv, 0, rows)
+                torch.cuda.synchronize()
+                vals, _, _ = sts[i].read_rows(layer, kv, 0, t + 1)
+                assert rel_err(rows.cpu().numpy(), vals) <= 1e-5, (i, layer, kv)
+
+
 def test_phonon_31m_shape_64_tokens_then_200_frames_at_temperature_0():
     # the single-stream configuration: 6 layers x 512, 8 heads, FF 2048, ldim 32, 4001-row LUT,
     # flow net 512 x 6, 1 LSD step; N(0, 0.02) linears, unit norms; 64 tokens, 200 greedy frames

@@ -603,6 +603,29 @@ hipError_t launch_gemm_q8(const void *A, int M, int K, const int8_t *W, const fl
 // that the norm's operands load together with x instead of behind a branch after the reductions.
 constexpr int kNormLn = 1, kNormAffine = 2, kNormMod = 4;
 
+// y (bias added) to the output value: eo the auxiliary operand, er the output's old value
+template <int EPI> __device__ __forceinline__ float linear_epilogue(float y, float eo, float er, float alpha) {
+    if constexpr (EPI == kLinStore) {
+        return y;
+    } else if constexpr (EPI == kLinGeluErf) {
+        return 0.5f * y * (1.0f + erff(y * 0.7071067811865476f));
+    } else if constexpr (EPI == kLinGeluTanh) {
+        const float c = 0.7978845608028654f;
+        return 0.5f * y * (1.0f + tanhf(c * (y + 0.044715f * y * y * y)));
+    } else if constexpr (EPI == kLinSilu) {
+        return y / (1.0f + expf(-y));
+    } else if constexpr (EPI == kLinSiluAddVec) {
+        const float z = y + eo;
+        return z / (1.0f + expf(-z));
+    } else if constexpr (EPI == kLinResidual) {
+        return er + y;
+    } else if constexpr (EPI == kLinGated) {
+        return er + eo * y;
+    } else { // kLinAxpy
+        return eo + y * alpha;
+    }
+}
+
 template <int KC, int EPI, int NORM>
 __global__ __launch_bounds__(256) void k_linear_f32(const float *x, int ldx, int M, int K, const float *W,
                                                     const float *bias, int N, LinOut lo, LinNorm ln) {
@@ -681,27 +704,187 @@ __global__ __launch_bounds__(256) void k_linear_f32(const float *x, int ldx, int
         for (int c = 0; c < KC; ++c) acc = __builtin_fmaf(w[c], c * 64 + lane < K ? xv[c] : 0.f, acc);
         acc = wave_sum(acc);
         if (lane != 0) continue;
-        const float y = acc + b;
-        if constexpr (EPI == kLinStore) {
-            *o = y;
-        } else if constexpr (EPI == kLinGeluErf) {
-            *o = 0.5f * y * (1.0f + erff(y * 0.7071067811865476f));
-        } else if constexpr (EPI == kLinGeluTanh) {
-            const float c = 0.7978845608028654f;
-            *o = 0.5f * y * (1.0f + tanhf(c * (y + 0.044715f * y * y * y)));
-        } else if constexpr (EPI == kLinSilu) {
-            *o = y / (1.0f + expf(-y));
-        } else if constexpr (EPI == kLinSiluAddVec) {
-            const float z = y + eo;
-            *o = z / (1.0f + expf(-z));
-        } else if constexpr (EPI == kLinResidual) {
-            *o = er + y;
-        } else if constexpr (EPI == kLinGated) {
-            *o = er + eo * y;
-        } else { // kLinAxpy
-            *o = eo + y * lo.alpha;
+        *o = linear_epilogue<EPI>(acc + b, eo, er, lo.alpha);
+    }
+}
+
+// The same product for several rows (prompts, batches of f32 streams), on v_mfma_f32_16x16x4_f32: one
+// work group of 8 waves per 16 MT rows x 16 columns, the waves splitting K.  A wave's whole share of x
+// and W is loaded at once, 16 bytes a lane: lane (l16, g) holds row (column) l16 at k = 16 i + 4 g .. + 3,
+// whose four values go to four products of 4 k each (x and W in the same (g, value) slot, so every k
+// meets its own).  Four sums a tile, one per value, then the waves' shares through LDS in a fixed
+// order: chains of NST additions, as short as k_linear_f32's.  The LayerNorm's moments are taken the same way
+// (the lane's values, its row's 4 lanes, the 8 waves), in two passes over the registers.
+//
+// At prompt sizes this is bound by the launch and one round trip to memory; k_linear_f32 took the rows
+// one after another, a round trip and three wave sums each (64 rows of 512: 15-27 us a launch, here
+// 4-10).
+template <int NST, int MT, int EPI, int NORM>
+__global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx, int M, int K, const float *W,
+                                                         const float *bias, int N, LinOut lo, LinNorm ln) {
+    typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4))); // rows need word alignment only
+    __shared__ float red[8][MT][16][17];
+    __shared__ float mom[2][8][MT * 16];
+    const int ntn = (N + 15) / 16, m0 = (int)blockIdx.x / ntn * (16 * MT), n0 = (int)blockIdx.x % ntn * 16;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
+    // every load is unconditional, its row and k clamped; values past K are zeroed on the x side
+    f32x4_a4 xv[MT][NST], wv[NST], sh[MT][NST], sc[MT][NST], nw[NST], nb[NST];
+    int k[NST];
+    const float *wr = W + (size_t)min(n0 + l16, N - 1) * K;
+#pragma unroll
+    for (int i = 0; i < NST; ++i) {
+        k[i] = 16 * (w * NST + i) + 4 * g;
+        const int kk = min(k[i], K - 4);
+        wv[i] = *(const f32x4_a4 *)(wr + kk);
+        if constexpr ((NORM & kNormAffine) != 0) {
+            nw[i] = *(const f32x4_a4 *)(ln.w + kk);
+            nb[i] = *(const f32x4_a4 *)(ln.b + kk);
+        }
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const size_t m = min(m0 + 16 * j + l16, M - 1);
+            xv[j][i] = *(const f32x4_a4 *)(x + m * ldx + kk);
+            if constexpr ((NORM & kNormMod) != 0) {
+                sh[j][i] = *(const f32x4_a4 *)(ln.shift + m * ln.ld_mod + kk);
+                sc[j][i] = *(const f32x4_a4 *)(ln.scale + m * ln.ld_mod + kk);
+            }
         }
     }
+    // the output this thread finishes (tile row er of row tile ej, column n0 + en) and its operands
+    const int ej = threadIdx.x >> 8, er_ = (threadIdx.x >> 4) & 15, en = threadIdx.x & 15;
+    const int om = m0 + 16 * ej + er_, on = n0 + en;
+    const bool mine = ej < MT && om < M && on < N;
+    float *o = nullptr;
+    float eo = 0.f, er = 0.f, b = 0.f;
+    if (mine) {
+        o = lo.out[0] + (size_t)om * lo.ld[0] + (on - lo.col0[0]);
+        if (lo.nseg > 1 && on >= lo.col0[1]) {
+            if (lo.nseg > 2 && on >= lo.col0[2])
+                o = lo.out[2] + (size_t)om * lo.ld[2] + (on - lo.col0[2]);
+            else
+                o = lo.out[1] + (size_t)om * lo.ld[1] + (on - lo.col0[1]);
+        }
+        if (bias) b = bias[on];
+        if constexpr (EPI == kLinResidual || EPI == kLinGated) er = *o;
+        if constexpr (EPI == kLinSiluAddVec)
+            eo = lo.aux[on];
+        else if constexpr (EPI == kLinGated || EPI == kLinAxpy)
+            eo = lo.aux[(size_t)om * lo.ld_aux + on];
+    }
+    __builtin_amdgcn_sched_barrier(0); // the loads above go out together
+    if constexpr ((NORM & kNormLn) != 0) {
+        // a row's moment from every lane that holds a share of it: rows 16 j + l16
+        auto moment = [&](float (&v)[MT], int which, float (&out)[MT]) {
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                const float s = swap_sum<32>(swap_sum<16>(v[j]));
+                if (g == 0) mom[which][w][16 * j + l16] = s;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                float p[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) p[q] = mom[which][q][16 * j + l16];
+                out[j] = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+            }
+        };
+        float v[MT], sum[MT], sq[MT];
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            v[j] = 0.f;
+#pragma unroll
+            for (int i = 0; i < NST; ++i)
+                if (k[i] < K) v[j] += (xv[j][i].x + xv[j][i].y) + (xv[j][i].z + xv[j][i].w);
+        }
+        moment(v, 0, sum);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const float mean = sum[j] / (float)K;
+            v[j] = 0.f;
+#pragma unroll
+            for (int i = 0; i < NST; ++i) {
+                xv[j][i] -= mean;
+                const f32x4_a4 d = xv[j][i] * xv[j][i];
+                if (k[i] < K) v[j] += (d.x + d.y) + (d.z + d.w);
+            }
+        }
+        moment(v, 1, sq);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const float rstd = 1.0f / __builtin_sqrtf(sq[j] / (float)K + ln.eps);
+#pragma unroll
+            for (int i = 0; i < NST; ++i) {
+                xv[j][i] *= rstd;
+                if constexpr ((NORM & kNormAffine) != 0) xv[j][i] = xv[j][i] * nw[i] + nb[i];
+                if constexpr ((NORM & kNormMod) != 0) xv[j][i] = xv[j][i] * (sc[j][i] + 1.0f) + sh[j][i];
+            }
+        }
+    }
+    f32x4_t acc[MT][4];
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[j][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NST; ++i) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const bool in = k[i] < K;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                acc[j][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? xv[j][i][c] : 0.f, wv[i][c], acc[j][c], 0, 0, 0);
+        }
+    }
+    // lane: column l16, rows 4 g + r of each row tile
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            red[w][j][4 * g + r][l16] = (acc[j][0][r] + acc[j][1][r]) + (acc[j][2][r] + acc[j][3][r]);
+    __syncthreads();
+    if (!mine) return;
+    float p[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) p[q] = red[q][ej][er_][en];
+    const float y = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])) + b;
+    *o = linear_epilogue<EPI>(y, eo, er, lo.alpha);
+}
+
+// Rows from which k_linear_f32_rows is taken: a whole row tile.  A prompt of the 6-layer model with its
+// first frame (row by row, then on row tiles): 4 tokens 391 and 365 us, 8 tokens 431 and 373, 16 tokens
+// 560 and 387, 64 tokens 1231 and 424.  Below 16 the gain is small, and the other order of the sums there
+// takes a model that feeds its latents back (5 frames from two 5-token prompts) past the 1e-5 its f32
+// results are held to (1.1e-5).
+constexpr int kLinRows = 16;
+
+template <int NST, int MT, int NORM>
+static hipError_t linear_f32_rows_mt(const float *x, int ldx, int M, int K, const float *W, const float *b, int N, int epi,
+                                     const LinOut &lo, const LinNorm &ln, hipStream_t stream) {
+    const dim3 grid((N + 15) / 16 * ((M + 16 * MT - 1) / (16 * MT))), block(512);
+#define XNP_LIN(E) hipLaunchKernelGGL((k_linear_f32_rows<NST, MT, E, NORM>), grid, block, 0, stream, x, ldx, M, K, W, b, N, lo, ln)
+    switch (epi) {
+    case kLinStore: XNP_LIN(kLinStore); break;
+    case kLinGeluErf: XNP_LIN(kLinGeluErf); break;
+    case kLinGeluTanh: XNP_LIN(kLinGeluTanh); break;
+    case kLinSilu: XNP_LIN(kLinSilu); break;
+    case kLinSiluAddVec: XNP_LIN(kLinSiluAddVec); break;
+    case kLinResidual: XNP_LIN(kLinResidual); break;
+    case kLinGated: XNP_LIN(kLinGated); break;
+    case kLinAxpy: XNP_LIN(kLinAxpy); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef XNP_LIN
+    return hipGetLastError();
+}
+
+template <int NST, int NORM>
+static hipError_t linear_f32_rows(const float *x, int ldx, int M, int K, const float *W, const float *b, int N, int epi,
+                                  const LinOut &lo, const LinNorm &ln, hipStream_t stream) {
+    // two row tiles a group (W read once for both) once one-tile groups fill the chip twice over
+    if ((int64_t)((N + 15) / 16) * ((M + 15) / 16) >= 1024)
+        return linear_f32_rows_mt<NST, 2, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
+    return linear_f32_rows_mt<NST, 1, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
 }
 
 template <int KC, int NORM>
@@ -728,6 +911,12 @@ template <int NORM>
 static hipError_t linear_f32_norm(const float *x, int ldx, int M, int K, const float *W, const float *b, int N, int epi,
                                   const LinOut &lo, const LinNorm &ln, hipStream_t stream) {
     const int kc = (K + 63) / 64;
+    if (M >= kLinRows && K % 4 == 0 && K >= 128) {
+        if (K <= 256) return linear_f32_rows<2, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
+        if (K <= 512) return linear_f32_rows<4, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
+        if (K <= 1024) return linear_f32_rows<8, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
+        if (K <= 2048) return linear_f32_rows<16, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
+    }
     if (kc <= 1) return linear_f32_kc<1, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
     if (kc <= 4) return linear_f32_kc<4, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
     if (kc <= 8) return linear_f32_kc<8, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
