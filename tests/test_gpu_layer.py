@@ -53,6 +53,32 @@ def test_linear_q8_on_128_row_tiles_matches_the_oracle(epi):
     check_linear_q8(129, 512, 16448, epi)
 
 
+@pytest.mark.parametrize("rows,n,epi", [(3265, 1032, "store"), (2721, 1536, "gelu_erf"), (2721, 1536, "gelu_tanh")])
+def test_linear_q8_with_w_in_registers_matches_the_oracle(rows, n, epi):
+    # K = 512, 1024 columns and more, at least three 32-row tiles a run (85 tiles of 1536 columns, 102 of
+    # 1032): W held in registers, rows streamed.  The last tile holds one row; 1032 columns leave the last
+    # column group one 8-column piece.  linear_q8 takes n a multiple of 64, the flow entry any n.
+    if n % 64 == 0:
+        check_linear_q8(rows, 512, n, epi)
+        return
+    rng = np.random.default_rng(rows)
+    x = normal(rng, (rows, 512), "bf16")
+    q, s = xnp.quantize_rows(rng.standard_normal((n, 512)).astype(np.float32) * 0.02)
+    b = (0.1 * rng.standard_normal(n)).astype(np.float32)
+    y = dev(np.full((rows, n + 8), 7.0, np.float32))
+    xnp.flow_linear_q8(dev(x), dev(q, torch.int8), dev(s, torch.float32), y, epi, bias=dev(b, torch.float32))
+    torch.cuda.synchronize()
+    assert rel_err(host(y)[:, :n], oracle.flow_linear_q8(x, q, s, epi, bias=b)) <= TOL
+    assert (host(y)[:, n:] == 7.0).all()  # nothing past the columns
+
+
+@pytest.mark.parametrize("n,epi", [(512, "residual"), (4096, "gelu_erf")])
+def test_linear_q8_on_128_column_tiles_matches_the_oracle(n, epi):
+    # 128 x 128 tiles where they fill whole rounds of 512 groups: K = 2048 (two halves a group) and 1024,
+    # the last row tile one row
+    check_linear_q8(13057 if n == 512 else 1665, 2048 if n == 512 else 1024, n, epi)
+
+
 def check_linear_q8(rows, k, n, epi):
     rng = np.random.default_rng(rows * 7 + n)
     x = normal(rng, (rows, k), "bf16")

@@ -2,6 +2,8 @@
 // MFMA with its epilogues, the f32 linears of batch-1 frames, and the row gathers.
 #include "kernels_common.h"
 
+#include <type_traits>
+
 namespace xnp {
 
 // ---------------------------------------------------------------------------------------------
@@ -148,6 +150,29 @@ hipError_t launch_layer_norm(const void *x, int rows, int dim, const float *w, c
 // when given) into X and rounds: X + layer_scale(linear(..)) as transformer.rs:612-633 does; the
 // flow net's epilogues are listed with their enum.  N may be any width (columns past N are
 // neither loaded nor stored) and K any multiple of 16 (the last chunk's loads past K read zeros).
+// gelu(y) = y Phi(y) for the bf16 epilogues (the erf form), from the tail Q(a) = 1 - Phi(a) = exp(-a^2 / 2)
+// p(t), t = 1 / (1 + 0.3 a), p a polynomial of degree 8 fitted to exp(a^2 / 2) Q(a) (the scaled
+// complementary error function) over a in [0, 13.5], 5.7e-8 relative at most; 17 VALU instructions in
+// one path, where 0.5 y (1 + erff(y / sqrt 2)) took 38 (linear1 at 16384 rows: 20 of its 75 us).  For
+// every finite bf16 y the result rounds to the bf16 nearest the exact value; the erff form, whose
+// 1 + erff cancels on the negative side, missed it for 197 of them.  Infinities and NaN as in the
+// erff form.
+__device__ __forceinline__ float gelu_erf(float y) {
+    const float a = fminf(fabsf(y), 40.f);
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(a, 0.3f, 1.f));
+    float p = 0.03833426907658577f;
+    p = __builtin_fmaf(p, t, -0.16895195841789246f);
+    p = __builtin_fmaf(p, t, 0.22821731865406036f);
+    p = __builtin_fmaf(p, t, -0.07599961757659912f);
+    p = __builtin_fmaf(p, t, 0.14218507707118988f);
+    p = __builtin_fmaf(p, t, 0.09483297169208527f);
+    p = __builtin_fmaf(p, t, 0.12188205868005753f);
+    p = __builtin_fmaf(p, t, 0.11949305981397629f);
+    p = __builtin_fmaf(p, t, 6.8529375312209595e-06f);
+    const float q = p * fast_exp2(a * (a * -0.72134752f));
+    return y * (y < 0.f ? q : 1.f - q);
+}
+
 constexpr int kGmT = 64;  // tile rows and columns
 constexpr int kGmK = 64;  // K chunk
 constexpr int kGmLd = 72; // LDS row length in bf16
@@ -170,42 +195,144 @@ constexpr int kGmPD = 3;  // K chunks of loads in flight
 // NKC: K is exactly NKC x KS chunks (8 or 16 per half: the flow LM's 512-2048 wide projections),
 // so the rounds run unrolled whole and without the past-K clamps and masks; 0: any K, in a loop.
 // Tiles go to the XCDs in contiguous runs (xcd_tile), so each XCD's L2 holds about an eighth of A.
-constexpr int kGsLd = 72; // the staged epilogue's LDS row in bf16
 
-template <int EPI, bool AF32, int MI, int KS, bool STG, int NKC>
-__global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, int K, const int8_t *W, const float *s,
+// The staged epilogue: a thread takes 8 consecutive columns of a row (y rounded to bf16), with the
+// operands of that piece (epi_load) and of its columns (epi_cols), and writes 16 bytes (32 for f32 rows).
+struct EpiPiece {
+    uint4 x, gate; // kResidual, kGated: the output's old values; kGated: the gate
+    float4 ax[2];  // kAxpyF32, kAddF32: the auxiliary row
+};
+struct EpiCols {
+    float4 v[2]; // kResidual: the layer scale (ones without); kSiluAddVec: the vector
+    char *out;   // row 0 of the output at these columns
+    int ld;      // its row stride in values
+};
+template <int EPI> __device__ __forceinline__ void epi_load(const GemmOut &go, int m, int n, EpiPiece &p) {
+    if constexpr (EPI == kResidual || EPI == kGated)
+        p.x = *(const uint4 *)((const uint16_t *)go.out[0] + (size_t)m * go.ld[0] + n);
+    if constexpr (EPI == kGated) p.gate = *(const uint4 *)((const uint16_t *)go.aux + (size_t)m * go.ld_aux + n);
+    if constexpr (EPI == kAxpyF32 || EPI == kAddF32) {
+        p.ax[0] = *(const float4 *)((const float *)go.aux + (size_t)m * go.ld_aux + n);
+        p.ax[1] = *(const float4 *)((const float *)go.aux + (size_t)m * go.ld_aux + n + 4);
+    }
+}
+template <int EPI> __device__ __forceinline__ void epi_cols(const GemmOut &go, int n, EpiCols &c) {
+    constexpr int ES = EPI == kAxpyF32 || EPI == kStoreF32 ? 4 : 2;
+    c.out = (char *)go.out[0] + (size_t)n * ES;
+    c.ld = go.ld[0];
+    if constexpr (EPI == kStore) { // constant indices: the kernel's arguments stay scalars
+        if (go.nseg > 1 && n >= go.col0[1]) c.out = (char *)go.out[1] + (size_t)(n - go.col0[1]) * ES, c.ld = go.ld[1];
+        if (go.nseg > 2 && n >= go.col0[2]) c.out = (char *)go.out[2] + (size_t)(n - go.col0[2]) * ES, c.ld = go.ld[2];
+    }
+    if constexpr (EPI == kResidual) {
+        c.v[0] = c.v[1] = make_float4(1.f, 1.f, 1.f, 1.f);
+        if (go.ls) {
+            c.v[0] = *(const float4 *)(go.ls + n);
+            c.v[1] = *(const float4 *)(go.ls + n + 4);
+        }
+    }
+    if constexpr (EPI == kSiluAddVec) {
+        c.v[0] = *(const float4 *)((const float *)go.aux + n);
+        c.v[1] = *(const float4 *)((const float *)go.aux + n + 4);
+    }
+}
+// one value: y to the output value, i its place in the piece
+template <int EPI>
+__device__ __forceinline__ float epi_value(float y, int i, const EpiPiece &p, const EpiCols &c, const GemmOut &go) {
+    const uint32_t *xw = (const uint32_t *)&p.x, *gw = (const uint32_t *)&p.gate;
+    const float *ax = (const float *)&p.ax[0], *cv = (const float *)&c.v[0];
+    if constexpr (EPI == kGeluErf) {
+        return gelu_erf(y);
+    } else if constexpr (EPI == kGeluTanh) {
+        const float cc = 0.7978845608028654f;
+        return 0.5f * y * (1.0f + tanhf(cc * (y + 0.044715f * y * y * y)));
+    } else if constexpr (EPI == kResidual) {
+        const float a = go.ls ? bf16_value(bf16_bits(y * cv[i])) : y;
+        return bf16_value((i & 1) ? xw[i >> 1] >> 16 : xw[i >> 1] & 0xffffu) + a;
+    } else if constexpr (EPI == kSilu) {
+        return y / (1.0f + expf(-y));
+    } else if constexpr (EPI == kSiluAddVec) {
+        const float z = bf16_value(bf16_bits(y + cv[i]));
+        return z / (1.0f + expf(-z));
+    } else if constexpr (EPI == kGated) {
+        const float gate = bf16_value((i & 1) ? gw[i >> 1] >> 16 : gw[i >> 1] & 0xffffu);
+        return bf16_value((i & 1) ? xw[i >> 1] >> 16 : xw[i >> 1] & 0xffffu) + bf16_value(bf16_bits(gate * y));
+    } else if constexpr (EPI == kAxpyF32) {
+        return bf16_value(bf16_bits(bf16_value(bf16_bits(ax[i])) + bf16_value(bf16_bits(y * go.alpha))));
+    } else if constexpr (EPI == kAddF32) {
+        return bf16_value(bf16_bits(ax[i])) + y;
+    } else { // kStore, kStoreF32
+        return y;
+    }
+}
+// the piece's 8 output values to row m
+template <int EPI> __device__ __forceinline__ void epi_write(const float (&r)[8], int m, const EpiCols &c) {
+    if constexpr (EPI == kAxpyF32 || EPI == kStoreF32) {
+        float *o = (float *)c.out + (size_t)m * c.ld;
+        *(float4 *)o = make_float4(r[0], r[1], r[2], r[3]);
+        *(float4 *)(o + 4) = make_float4(r[4], r[5], r[6], r[7]);
+    } else {
+        st_stream((uint16_t *)c.out + (size_t)m * c.ld,
+                  make_uint4(pack_bf16(r[0], r[1]), pack_bf16(r[2], r[3]), pack_bf16(r[4], r[5]), pack_bf16(r[6], r[7])));
+    }
+}
+__device__ __forceinline__ float epi_y(const uint4 &yv, int i) { // value i of the staged y
+    const uint32_t u = ((const uint32_t *)&yv)[i >> 1];
+    return bf16_value((i & 1) ? u >> 16 : u & 0xffffu);
+}
+template <int EPI>
+__device__ __forceinline__ void epi_store(const GemmOut &go, int m, const uint4 &yv, const EpiPiece &p, const EpiCols &c) {
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = epi_value<EPI>(epi_y(yv, i), i, p, c, go);
+    epi_write<EPI>(r, m, c);
+}
+
+template <int EPI, bool AF32, int MI, int NI, int KS, bool STG, int NKC>
+__global__ __launch_bounds__(256 * KS, NI > 2 ? 2 : 1) void k_gemm_q8(const uint16_t *A, int M, int K, const int8_t *W, const float *s,
                                                       int N, GemmOut go) {
-    constexpr int BM = 32 * MI;
+    constexpr int BM = 32 * MI, BN = 32 * NI;
+    constexpr int KC = kGmK, LD = kGmLd; // K chunk, LDS row length in bf16
+    // K chunks of loads in flight (a wide tile's round is twice as long; its registers are full)
+    constexpr int PD = NI > 2 ? 2 : kGmPD;
+    static_assert(NI == 2 || STG, "wide tiles come with the staged epilogue");
     static_assert(KS == 1 || KS == 2, "one or two halves");
-    __shared__ __attribute__((aligned(16))) uint16_t As[KS][2][BM][kGmLd];
-    __shared__ __attribute__((aligned(16))) uint16_t Ws[KS][2][kGmT][kGmLd];
-    const int ntn = (N + kGmT - 1) / kGmT, tile = xcd_tile(blockIdx.x, gridDim.x);
-    const int m0 = (tile / ntn) * BM, n0 = (tile % ntn) * kGmT;
+    struct Tiles {
+        uint16_t A[KS][2][BM][LD], W[KS][2][BN][LD];
+    };
+    __shared__ __attribute__((aligned(16))) Tiles smem;
+    auto &As = smem.A;
+    auto &Ws = smem.W;
+    const int ntn = (N + BN - 1) / BN, tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int m0 = (tile / ntn) * BM, n0 = (tile % ntn) * BN;
     const int tid = threadIdx.x & 255, h = KS > 1 ? (int)(threadIdx.x >> 8) : 0;
     const int w = tid >> 6, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
     const int wm = w & 1, wn = w >> 1;
 
-    // staging: A rows a_r + 32 i, i < MI (the tile's 32 MI rows), 8 values at k 8 a_k; W row w_r, 16
-    // int8 at k 16 w_k.
-    // kGmPD chunks of loads are in flight: set c % kGmPD holds chunk c from its load until it is
+    // staging: A rows a_r + RA i (the tile's 32 MI rows), 8 values at k 8 a_k; W rows w_r + RW i,
+    // 16 int8 at k 16 w_k.
+    // PD chunks of loads are in flight: set c % PD holds chunk c from its load until it is
     // written to LDS.  The words stay as loaded until then -- zeroing past K, rounding f32 A rows
     // and widening W happen at the LDS store, since any use at the load would make the wave wait
     // for it there.
-    constexpr int NA = MI; // A rows a thread stages
-    const int a_r = tid >> 3, a_k = tid & 7, w_r = tid >> 2, w_k = tid & 3;
+    constexpr int UA = KC / 8, UW = KC / 16, RA = 256 / UA, RW = 256 / UW; // pieces a row, rows a pass
+    constexpr int NA = BM / RA, NW = BN / RW;                                // A and W rows a thread stages
+    const int a_r = tid / UA, a_k = tid % UA, w_r = tid / UW, w_k = tid % UW;
     int ar[NA];
 #pragma unroll
-    for (int i = 0; i < NA; ++i) ar[i] = min(m0 + a_r + 32 * i, M - 1);
-    const int wr = min(n0 + w_r, N - 1);
+    for (int i = 0; i < NA; ++i) ar[i] = min(m0 + a_r + RA * i, M - 1);
+    int wr[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) wr[i] = min(n0 + w_r + RW * i, N - 1);
     constexpr int AW = AF32 ? 2 : 1; // uint4 per 8 A values
-    uint4 ra[NA][kGmPD][AW], rw[kGmPD];
+    uint4 ra[NA][PD][AW], rw[NW][PD];
     // NKC > 0: K is a whole number of chunks, so nothing reaches past it and the clamps and masks
     // below drop out (they were 14-18 of a round's 47-51 VALU instructions)
     constexpr bool kWhole = NKC > 0;
     auto load = [&](int kc, int set) {
         // past K (K % 16 == 0, so no 16-byte load straddles it): an in-bounds address, zeroed at
         // the store
-        const int k0 = kc * kGmK;
+        const int k0 = kc * KC;
         const int ka = kWhole || k0 + 8 * a_k < K ? k0 + 8 * a_k : 0, kw = kWhole || k0 + 16 * w_k < K ? k0 + 16 * w_k : 0;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
@@ -217,7 +344,8 @@ __global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, 
                 ra[i][set][0] = *(const uint4 *)(A + (size_t)ar[i] * K + ka);
             }
         }
-        rw[set] = *(const uint4 *)(W + (size_t)wr * K + kw);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) rw[i][set] = *(const uint4 *)(W + (size_t)wr[i] * K + kw);
     };
     auto masked = [](const uint4 &u, uint32_t m) { return make_uint4(u.x & m, u.y & m, u.z & m, u.w & m); };
     auto bf16_row = [&](const uint4 (&u)[AW]) { // 8 A values as bf16 pairs
@@ -234,73 +362,63 @@ __global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, 
         return pack_bf16((float)(int8_t)((u >> sh) & 0xffu), (float)(int8_t)((u >> (sh + 8)) & 0xffu));
     };
     auto store = [&](int buf, int set, int kc) {
-        uint4 av[NA], wq = rw[set];
+        uint4 av[NA], wq[NW];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) wq[i] = rw[i][set];
 #pragma unroll
         for (int i = 0; i < NA; ++i) av[i] = bf16_row(ra[i][set]);
         // words past K zeroed with masks rather than under a branch: a branch here splits the
         // loop, and past the join the compiler no longer knows which loads are still in flight
         // (it then waits for all of them before the next load)
         if constexpr (!kWhole) {
-            const int k0 = kc * kGmK;
+            const int k0 = kc * KC;
             const uint32_t ma = k0 + 8 * a_k < K ? ~0u : 0u, mw = k0 + 16 * w_k < K ? ~0u : 0u;
 #pragma unroll
             for (int i = 0; i < NA; ++i) av[i] = masked(av[i], ma);
-            wq = masked(wq, mw);
+#pragma unroll
+            for (int i = 0; i < NW; ++i) wq[i] = masked(wq[i], mw);
         }
 #pragma unroll
-        for (int i = 0; i < NA; ++i) *(uint4 *)&As[h][buf][a_r + 32 * i][8 * a_k] = av[i];
-        *(uint4 *)&Ws[h][buf][w_r][16 * w_k] = make_uint4(widen2(wq.x, 0), widen2(wq.x, 16), widen2(wq.y, 0), widen2(wq.y, 16));
-        *(uint4 *)&Ws[h][buf][w_r][16 * w_k + 8] =
-            make_uint4(widen2(wq.z, 0), widen2(wq.z, 16), widen2(wq.w, 0), widen2(wq.w, 16));
+        for (int i = 0; i < NA; ++i) *(uint4 *)&As[h][buf][a_r + RA * i][8 * a_k] = av[i];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const uint4 q = wq[i];
+            uint16_t *ws = &Ws[h][buf][w_r + RW * i][16 * w_k];
+            *(uint4 *)ws = make_uint4(widen2(q.x, 0), widen2(q.x, 16), widen2(q.y, 0), widen2(q.y, 16));
+            *(uint4 *)(ws + 8) = make_uint4(widen2(q.z, 0), widen2(q.z, 16), widen2(q.w, 0), widen2(q.w, 16));
+        }
     };
 
     // the epilogue's per-column operands, loaded before the loop so that they arrive with it
-    float sc[2], bn[2], lsn[2];
+    float sc[NI], bn[NI], lsn[NI];
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-        const int n = min(n0 + 32 * wn + 16 * ni + l16, N - 1);
+    for (int ni = 0; ni < NI; ++ni) {
+        const int n = min(n0 + 16 * NI * wn + 16 * ni + l16, N - 1);
         sc[ni] = s[n];
         bn[ni] = go.bias ? go.bias[n] : 0.f;
         lsn[ni] = (EPI == kResidual && go.ls) ? go.ls[n] : 1.f;
     }
 
-    // the staged epilogue's pieces (rows er + 32 e, columns n0 + ec ..) and their operands
-    const int er = tid >> 3, ec = 8 * (tid & 7), ne = n0 + ec;
-    uint4 xo[MI], gt[MI];
-    float4 ax[MI][2], lv[2];
-    if constexpr (STG) {
+    // the staged epilogue's pieces (rows er + ER e, columns n0 + ec ..) and their operands (wide tiles:
+    // loaded after the K loop, whose registers they would take)
+    constexpr int PR = BN / 8, ER = 256 / PR, NE = BM / ER; // pieces a row, rows a pass, passes
+    const int er = tid / PR, ec = 8 * (tid % PR), ne = n0 + ec;
+    EpiPiece piece[NE];
+    auto operands = [&] {
         if (h == 0) {
 #pragma unroll
-            for (int e = 0; e < MI; ++e) {
-                const int mm = min(m0 + er + 32 * e, M - 1), nn = ne < N ? ne : 0;
-                if constexpr (EPI == kResidual || EPI == kGated)
-                    xo[e] = *(const uint4 *)((const uint16_t *)go.out[0] + (size_t)mm * go.ld[0] + nn);
-                if constexpr (EPI == kGated)
-                    gt[e] = *(const uint4 *)((const uint16_t *)go.aux + (size_t)mm * go.ld_aux + nn);
-                if constexpr (EPI == kAxpyF32 || EPI == kAddF32) {
-                    ax[e][0] = *(const float4 *)((const float *)go.aux + (size_t)mm * go.ld_aux + nn);
-                    ax[e][1] = *(const float4 *)((const float *)go.aux + (size_t)mm * go.ld_aux + nn + 4);
-                }
-            }
-            if constexpr (EPI == kResidual) {
-                lv[0] = lv[1] = make_float4(1.f, 1.f, 1.f, 1.f);
-                if (go.ls && ne < N) {
-                    lv[0] = *(const float4 *)(go.ls + ne);
-                    lv[1] = *(const float4 *)(go.ls + ne + 4);
-                }
-            }
-            if constexpr (EPI == kSiluAddVec) {
-                lv[0] = *(const float4 *)((const float *)go.aux + (ne < N ? ne : 0));
-                lv[1] = *(const float4 *)((const float *)go.aux + (ne < N ? ne : 0) + 4);
-            }
+            for (int e = 0; e < NE; ++e) epi_load<EPI>(go, min(m0 + er + ER * e, M - 1), ne < N ? ne : 0, piece[e]);
         }
-    }
+    };
+    EpiCols cols;
+    if constexpr (STG) epi_cols<EPI>(go, ne < N ? ne : 0, cols);
+    if constexpr (STG && NI == 2) operands();
 
-    f32x4_t acc[MI][2];
+    f32x4_t acc[MI][NI];
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     // this half's chunks: c = 0 .. nkh - 1 is chunk h + KS c.  Both halves run nkmax rounds, one
     // barrier each, whatever their own count (the launcher takes KS = 2 only when nk >= 2 KS).
@@ -309,44 +427,44 @@ __global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, 
     // are in flight after it, and it then drains them all before the next one.  NKC > 0: K is
     // NKC x KS chunks exactly, and the rounds are unrolled whole -- the back edge of a loop makes
     // the compiler copy load registers still in flight, which waits for them.
-    const int nk = NKC > 0 ? NKC * KS : (K + kGmK - 1) / kGmK;
+    const int nk = NKC > 0 ? NKC * KS : (K + KC - 1) / KC;
     const int nkh = NKC > 0 ? NKC : (nk - h + KS - 1) / KS, nkmax = NKC > 0 ? NKC : (nk + KS - 1) / KS;
     auto chunk = [&](int c) { return h + KS * min(c, nkh - 1); };
-    auto round = [&](int c, int u) { // u = c % kGmPD: set indices stay constants
+    auto round = [&](int c, int u) { // u = c % PD: set indices stay constants
         const int buf = c & 1;
-        load(chunk(c + kGmPD), u); // set u held chunk c, already in LDS
+        load(chunk(c + PD), u); // set u held chunk c, already in LDS
         if (c < nkh) {
 #pragma unroll
-            for (int ks = 0; ks < kGmK / 32; ++ks) {
-                bf16x8_t a[MI], bw[2];
+            for (int ks = 0; ks < KC / 32; ++ks) {
+                bf16x8_t a[MI], bw[NI];
 #pragma unroll
                 for (int i = 0; i < MI; ++i)
                     a[i] = as_bf16x8(*(const uint4 *)&As[h][buf][16 * MI * wm + 16 * i + l16][32 * ks + 8 * g]);
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    bw[i] = as_bf16x8(*(const uint4 *)&Ws[h][buf][32 * wn + 16 * i + l16][32 * ks + 8 * g]);
+                for (int i = 0; i < NI; ++i)
+                    bw[i] = as_bf16x8(*(const uint4 *)&Ws[h][buf][16 * NI * wn + 16 * i + l16][32 * ks + 8 * g]);
 #pragma unroll
                 for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-                    for (int ni = 0; ni < 2; ++ni)
+                    for (int ni = 0; ni < NI; ++ni)
                         acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mi], bw[ni], acc[mi][ni], 0, 0, 0);
             }
         }
         // buffer buf ^ 1's last readers finished before the previous barrier
-        store(buf ^ 1, (u + 1) % kGmPD, chunk(c + 1));
+        store(buf ^ 1, (u + 1) % PD, chunk(c + 1));
         __syncthreads();
     };
 #pragma unroll
-    for (int c = 0; c < kGmPD; ++c) load(chunk(c), c);
+    for (int c = 0; c < PD; ++c) load(chunk(c), c);
     store(0, 0, h);
     __syncthreads();
     if constexpr (NKC > 0) {
 #pragma unroll
-        for (int c = 0; c < NKC; ++c) round(c, c % kGmPD);
+        for (int c = 0; c < NKC; ++c) round(c, c % PD);
     } else {
-        for (int cb = 0; cb < nkmax; cb += kGmPD) {
+        for (int cb = 0; cb < nkmax; cb += PD) {
 #pragma unroll
-            for (int u = 0; u < kGmPD; ++u) {
+            for (int u = 0; u < PD; ++u) {
                 if (cb + u >= nkmax) break; // uniform over the group
                 round(cb + u, u);
             }
@@ -355,15 +473,15 @@ __global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, 
     if constexpr (KS > 1) {
         // half 1's sums to half 0 through LDS (the tiles are free: every half passed the loop's
         // last barrier after its last read); half 0 adds them, in the same order in every group
-        static_assert(sizeof(As) >= 256 * MI * 8 * sizeof(float), "room for half 1's sums");
-        float *red = (float *)&As[0][0][0][0];
+        static_assert(sizeof(smem) >= 256 * MI * NI * 4 * sizeof(float), "room for half 1's sums");
+        float *red = (float *)&smem;
         if (h == 1) {
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < 2; ++ni)
+                for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) red[((mi * 2 + ni) * 4 + r) * 256 + tid] = acc[mi][ni][r];
+                    for (int r = 0; r < 4; ++r) red[((mi * NI + ni) * 4 + r) * 256 + tid] = acc[mi][ni][r];
         }
         __syncthreads();
         if (!STG && h == 1) return;
@@ -371,106 +489,46 @@ __global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, 
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < 2; ++ni)
+                for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[mi][ni][r] += red[((mi * 2 + ni) * 4 + r) * 256 + tid];
+                    for (int r = 0; r < 4; ++r) acc[mi][ni][r] += red[((mi * NI + ni) * 4 + r) * 256 + tid];
         }
     }
 
     if constexpr (STG) {
-        // y into LDS (lane: column 32 wn + 16 ni + l16, rows 16 MI wm + 16 mi + 4 g + r); both halves
+        // y into LDS (lane: column 16 NI wn + 16 ni + l16, rows 16 MI wm + 16 mi + 4 g + r); both halves
         // meet at the barriers, half 1 with nothing to store
-        static_assert(sizeof(As) >= 32 * MI * kGsLd * sizeof(uint16_t), "room for the tile");
-        uint16_t(*st)[kGsLd] = (uint16_t(*)[kGsLd]) & As[0][0][0][0];
+        constexpr int kGsLd = BN + 8; // the staged epilogue's LDS row in bf16
+        static_assert(sizeof(smem) >= BM * kGsLd * sizeof(uint16_t), "room for the tile");
+        uint16_t(*st)[kGsLd] = (uint16_t(*)[kGsLd]) & smem;
+        if constexpr (NI > 2) operands();
         if constexpr (KS > 1) __syncthreads(); // half 0 has read half 1's sums
         if (h == 0) {
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < 2; ++ni)
+                for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float v = go.bias ? acc[mi][ni][r] * sc[ni] + bn[ni] : acc[mi][ni][r] * sc[ni];
-                        st[16 * MI * wm + 16 * mi + 4 * g + r][32 * wn + 16 * ni + l16] = (uint16_t)bf16_bits(v);
+                        st[16 * MI * wm + 16 * mi + 4 * g + r][16 * NI * wn + 16 * ni + l16] = (uint16_t)bf16_bits(v);
                     }
         }
         __syncthreads();
         if (h != 0) return;
 #pragma unroll
-        for (int e = 0; e < MI; ++e) {
-            const int m = m0 + er + 32 * e;
+        for (int e = 0; e < NE; ++e) {
+            const int m = m0 + er + ER * e;
             if (m >= M || ne >= N) continue;
-            const uint4 yv = *(const uint4 *)&st[er + 32 * e][ec];
-            const uint32_t *yw = (const uint32_t *)&yv;
-            float y[8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                y[2 * i] = bf16_value(yw[i] & 0xffffu);
-                y[2 * i + 1] = bf16_value(yw[i] >> 16);
-            }
-            if constexpr (EPI == kStore) {
-                int seg = 0;
-                if (go.nseg > 1 && ne >= go.col0[1]) seg = (go.nseg > 2 && ne >= go.col0[2]) ? 2 : 1;
-                st_stream((uint16_t *)go.out[seg] + (size_t)m * go.ld[seg] + (ne - go.col0[seg]), yv);
-            } else if constexpr (EPI == kStoreF32) {
-                float *o = (float *)go.out[0] + (size_t)m * go.ld[0] + ne;
-                *(float4 *)o = make_float4(y[0], y[1], y[2], y[3]);
-                *(float4 *)(o + 4) = make_float4(y[4], y[5], y[6], y[7]);
-            } else if constexpr (EPI == kAxpyF32) {
-                const float cu[8] = {ax[e][0].x, ax[e][0].y, ax[e][0].z, ax[e][0].w,
-                                     ax[e][1].x, ax[e][1].y, ax[e][1].z, ax[e][1].w};
-                float r8[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    r8[i] = bf16_value(bf16_bits(bf16_value(bf16_bits(cu[i])) + bf16_value(bf16_bits(y[i] * go.alpha))));
-                float *o = (float *)go.out[0] + (size_t)m * go.ld[0] + ne;
-                *(float4 *)o = make_float4(r8[0], r8[1], r8[2], r8[3]);
-                *(float4 *)(o + 4) = make_float4(r8[4], r8[5], r8[6], r8[7]);
-            } else if constexpr (EPI == kAddF32) {
-                const float cu[8] = {ax[e][0].x, ax[e][0].y, ax[e][0].z, ax[e][0].w,
-                                     ax[e][1].x, ax[e][1].y, ax[e][1].z, ax[e][1].w};
-                float r8[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) r8[i] = bf16_value(bf16_bits(cu[i])) + y[i];
-                st_stream((uint16_t *)go.out[0] + (size_t)m * go.ld[0] + ne,
-                          make_uint4(pack_bf16(r8[0], r8[1]), pack_bf16(r8[2], r8[3]), pack_bf16(r8[4], r8[5]), pack_bf16(r8[6], r8[7])));
-            } else {
-                float r8[8];
-                const uint32_t *xw = (const uint32_t *)&xo[e], *gw = (const uint32_t *)&gt[e];
-                const float l8[8] = {lv[0].x, lv[0].y, lv[0].z, lv[0].w, lv[1].x, lv[1].y, lv[1].z, lv[1].w};
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float yi = y[i];
-                    if constexpr (EPI == kGeluErf) {
-                        r8[i] = 0.5f * yi * (1.0f + erff(yi * 0.7071067811865476f));
-                    } else if constexpr (EPI == kGeluTanh) {
-                        const float cc = 0.7978845608028654f;
-                        r8[i] = 0.5f * yi * (1.0f + tanhf(cc * (yi + 0.044715f * yi * yi * yi)));
-                    } else if constexpr (EPI == kResidual) {
-                        const float a = go.ls ? bf16_value(bf16_bits(yi * l8[i])) : yi;
-                        r8[i] = bf16_value((i & 1) ? xw[i >> 1] >> 16 : xw[i >> 1] & 0xffffu) + a;
-                    } else if constexpr (EPI == kSilu) {
-                        r8[i] = yi / (1.0f + expf(-yi));
-                    } else if constexpr (EPI == kSiluAddVec) {
-                        const float z = bf16_value(bf16_bits(yi + l8[i]));
-                        r8[i] = z / (1.0f + expf(-z));
-                    } else { // kGated
-                        const float gate = bf16_value((i & 1) ? gw[i >> 1] >> 16 : gw[i >> 1] & 0xffffu);
-                        r8[i] = bf16_value((i & 1) ? xw[i >> 1] >> 16 : xw[i >> 1] & 0xffffu) +
-                                bf16_value(bf16_bits(gate * yi));
-                    }
-                }
-                st_stream((uint16_t *)go.out[0] + (size_t)m * go.ld[0] + ne,
-                          make_uint4(pack_bf16(r8[0], r8[1]), pack_bf16(r8[2], r8[3]), pack_bf16(r8[4], r8[5]), pack_bf16(r8[6], r8[7])));
-            }
+            epi_store<EPI>(go, m, *(const uint4 *)&st[er + ER * e][ec], piece[e], cols);
         }
         return;
     }
 
-    // lane: column n0 + 32 wn + 16 ni + l16, rows m0 + 16 MI wm + 16 mi + 4 g + r
+    // lane: column n0 + 16 NI wn + 16 ni + l16, rows m0 + 16 MI wm + 16 mi + 4 g + r
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-        const int n = n0 + 32 * wn + 16 * ni + l16;
+    for (int ni = 0; ni < NI; ++ni) {
+        const int n = n0 + 16 * NI * wn + 16 * ni + l16;
         if (n >= N) continue;
         int seg = 0;
         if constexpr (EPI == kStore) {
@@ -488,7 +546,7 @@ __global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, 
                 } else if constexpr (EPI == kGeluErf || EPI == kGeluTanh) {
                     float gv;
                     if constexpr (EPI == kGeluErf) {
-                        gv = 0.5f * y * (1.0f + erff(y * 0.7071067811865476f));
+                        gv = gelu_erf(y);
                     } else {
                         const float c = 0.7978845608028654f;
                         gv = 0.5f * y * (1.0f + tanhf(c * (y + 0.044715f * y * y * y)));
@@ -521,6 +579,147 @@ __global__ __launch_bounds__(256 * KS) void k_gemm_q8(const uint16_t *A, int M, 
     }
 }
 
+// The same product for K = 512 and many rows, with W in registers: one work group of 8 waves per CU
+// holds 256 columns of W for a run of 32-row tiles, each wave 32 columns over all of K as the 32 A
+// operands of v_mfma_f32_32x32x16_bf16 (128 registers, widened once).  The rows stream through a
+// ring of 3 LDS slots (32 KB, loaded straight into LDS two tiles ahead), and a wave's inner loop is one
+// 16-byte LDS read per MFMA: k_gemm_q8's tiles pay a barrier, the W widening and an LDS round trip of
+// both operands per 64 k, and no unit of theirs was busy half the time (16384 rows, qkv: MFMA 28 %, LDS
+// 50 %, VALU 32 %), whatever their size or prefetch.  16384 rows: qkv 48.7 (128 x 64 tiles), 41 (128 x 128),
+// here 31.5 us (818 TFLOP/s); linear1 with its GELU 83, 65, 51.4 us, bound by the GELU's VALU work.
+//
+// The k order is the same for both operands and otherwise free: lane (col, hi) of W loads 16
+// consecutive k (32 j + 16 hi ..), its halves the operands of steps 2 j and 2 j + 1, so row unit (8 k)
+// 4 j + 2 hi + b is read at step 2 j + b.  Units sit at unit ^ (row & 15): a read's 8 rows fall in
+// distinct banks, and a row of a tile is one 1 KB load.
+// D = W A^T holds, per lane, row l % 32 and columns 8 (r / 4) + 4 (l / 32) + r % 4: rounded to bf16 they
+// go through LDS as [row][col], and 8 columns a thread leave by the staged epilogue one tile later.
+constexpr int kWrK = 512, kWrRows = 32, kWrCols = 256, kWrSlots = 3;
+
+template <int EPI>
+__global__ __launch_bounds__(512, 2) void k_gemm_q8_wres(const uint16_t *A, int M, const int8_t *W, const float *s, int N,
+                                                         GemmOut go, int per) {
+    __shared__ __attribute__((aligned(16))) uint16_t As[kWrSlots][kWrRows][kWrK];
+    __shared__ __attribute__((aligned(16))) uint16_t st[2][kWrRows][kWrCols + 8]; // rows 16 bytes further apart in banks
+    const int ntn = (N + kWrCols - 1) / kWrCols, tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int n0 = tile % ntn * kWrCols, t0 = tile / ntn * per, t1 = min(t0 + per, (M + kWrRows - 1) / kWrRows);
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, hi = lane >> 5, col = lane & 31;
+    const uint32_t as_at = lds_addr(&As[0][0][0]);
+    // tile t's rows 4 w .. 4 w + 3 into slot: lane l's 16 bytes are unit l ^ (row & 15) of the row
+    auto issue = [&](int t, int slot) {
+        const int ln = lane_here(lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = 4 * w + i, m = min(t * kWrRows + row, M - 1);
+            dma16_at(A + (size_t)m * kWrK + 8 * (ln ^ (row & 15)), as_at + (uint32_t)((slot * kWrRows + row) * kWrK * 2));
+        }
+    };
+    // W, then the first two tiles behind it
+    const int nw = n0 + 32 * w; // the wave's columns
+    bf16x8_t wf[32];
+    {
+        const int8_t *wr = W + (size_t)min(nw + col, N - 1) * kWrK + 16 * hi;
+        uint4 raw[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) raw[j] = *(const uint4 *)(wr + 32 * j);
+        __builtin_amdgcn_sched_barrier(0);
+        issue(t0, 0);
+        if (t0 + 1 < t1) issue(t0 + 1, 1);
+        auto widen2 = [](uint32_t u, int sh) { // two int8 -> a bf16 pair (exact: |q| <= 127)
+            return pack_bf16((float)(int8_t)((u >> sh) & 0xffu), (float)(int8_t)((u >> (sh + 8)) & 0xffu));
+        };
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            wf[2 * j] = as_bf16x8(make_uint4(widen2(raw[j].x, 0), widen2(raw[j].x, 16), widen2(raw[j].y, 0), widen2(raw[j].y, 16)));
+            wf[2 * j + 1] = as_bf16x8(make_uint4(widen2(raw[j].z, 0), widen2(raw[j].z, 16), widen2(raw[j].w, 0), widen2(raw[j].w, 16)));
+        }
+    }
+    float sc[16], bn[16]; // of columns nw + 8 (r / 4) + 4 hi + r % 4
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int n = min(nw + 8 * (r >> 2) + 4 * hi + (r & 3), N - 1);
+        sc[r] = s[n];
+        bn[r] = go.bias ? go.bias[n] : 0.f;
+    }
+    // the pieces this thread stores: rows er and er + 16, 8 columns.  Past the last row or column the
+    // last one again, bit for bit what its own thread stores: no branch parts the products below
+    const int er = tid >> 5, ne = min(n0 + 8 * (tid & 31), N - 8), ec = ne - n0;
+    static_assert(EPI == kStore || EPI == kGeluErf || EPI == kGeluTanh, "epilogues without operands of their own");
+    EpiCols cols;
+    epi_cols<EPI>(go, ne, cols);
+    auto row_of = [&](int t, int e) { return min(t * kWrRows + er + 16 * e, M - 1); };
+    auto store_tile = [&](int t) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int m = row_of(t, e);
+            epi_store<EPI>(go, m, *(const uint4 *)&st[t & 1][m - t * kWrRows][ec], EpiPiece(), cols);
+        }
+    };
+    // the lane's LDS offsets within a slot for steps 0 .. 7 (steps 8 i + .. lie 256 i bytes further: a
+    // row's units 16 i .. keep their place in 16s)
+    uint32_t aofs[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) aofs[k] = col * (kWrK * 2) + 16 * ((4 * (k >> 1) + 2 * hi + (k & 1)) ^ (col & 15));
+    constexpr int FD = 6; // LDS reads ahead
+    auto tile_body = [&](int t, int slot, auto FIRST) {
+        // this lane's loads of tile t have landed: tile t + 1's 4 went out after them, last of all (the
+        // stores of the iteration before are older)
+        if (t + 1 < t1)
+            asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier(); // tile t is in LDS; every wave is done with tile t - 1's slot and has staged its outputs
+        const char *base = (const char *)&As[slot][0][0];
+        auto frag = [&](int k) { return as_bf16x8(*(const uint4 *)(base + aofs[k & 7] + 256 * (k >> 3))); };
+        f32x16_t acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+        bf16x8_t f[FD];
+#pragma unroll
+        for (int k = 0; k < FD; ++k) f[k] = frag(k);
+        uint4 yv[2];
+        float o8[8];
+        if constexpr (!decltype(FIRST)::value) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) yv[e] = *(const uint4 *)&st[(t - 1) & 1][row_of(t - 1, e) - (t - 1) * kWrRows][ec];
+        }
+        // FD LDS reads stay ahead of the products, one issued after each, and the previous tile's outputs
+        // are finished a value a product and leave between them: the waves of a SIMD are in the same
+        // phase (one barrier a tile), so nothing else would run beside the matrix pipe.  The scheduling
+        // barriers hold that order (VALU instructions may cross them); left alone, the compiler reads
+        // each operand right before its product, an LDS round trip each.
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[k], f[k % FD], acc, 0, 0, 0);
+            if (k + FD < 32) f[k % FD] = frag(k + FD);
+            __builtin_amdgcn_sched_barrier(0x6);
+            if constexpr (!decltype(FIRST)::value) {
+                if (k >= 4 && k < 20) {
+                    const int e = (k - 4) >> 3, i = (k - 4) & 7;
+                    o8[i] = epi_value<EPI>(epi_y(yv[e], i), i, EpiPiece(), cols, go);
+                    if (i == 7) epi_write<EPI>(o8, row_of(t - 1, e), cols);
+                }
+            }
+            if (k == 21 && t + 2 < t1) issue(t + 2, slot == 0 ? 2 : slot - 1);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float y[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = acc[4 * q + r] * sc[4 * q + r] + bn[4 * q + r];
+            *(uint2 *)&st[t & 1][col][32 * w + 8 * q + 4 * hi] = make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
+        }
+    };
+    tile_body(t0, 0, std::true_type{});
+    int slot = 1;
+    for (int t = t0 + 1; t < t1; ++t) {
+        tile_body(t, slot, std::false_type{});
+        slot = slot == 2 ? 0 : slot + 1;
+    }
+    lds_barrier();
+    store_tile(t1 - 1);
+}
+
 // The staged epilogue's conditions: 8-column pieces that stay inside N and inside one kStore segment,
 // and 16-byte aligned accesses to every output and operand row.
 static bool gemm_staged(int N, int epi, const GemmOut &go) {
@@ -534,19 +733,23 @@ static bool gemm_staged(int N, int epi, const GemmOut &go) {
     return true;
 }
 
-template <int MI, int KS, bool STG, int NKC>
+template <int MI, int NI, int KS, bool STG, int NKC>
 static hipError_t gemm_q8_stg(const void *A, int M, int K, const int8_t *W, const float *s, int N, int epi,
                               const GemmOut &go, hipStream_t stream) {
-    const dim3 grid(((N + kGmT - 1) / kGmT) * ((M + 32 * MI - 1) / (32 * MI))), block(256 * KS);
+    const dim3 grid(((N + 32 * NI - 1) / (32 * NI)) * ((M + 32 * MI - 1) / (32 * MI))), block(256 * KS);
     const uint16_t *a = (const uint16_t *)A;
-#define XNP_GEMM(E) hipLaunchKernelGGL((k_gemm_q8<E, false, MI, KS, STG, NKC>), grid, block, 0, stream, a, M, K, W, s, N, go)
+#define XNP_GEMM(E) hipLaunchKernelGGL((k_gemm_q8<E, false, MI, NI, KS, STG, NKC>), grid, block, 0, stream, a, M, K, W, s, N, go)
     if (go.a_f32) {
-        if ((epi != kStore && epi != kAddF32) || NKC != 0) return hipErrorInvalidValue;
-        if (epi == kStore)
-            hipLaunchKernelGGL((k_gemm_q8<kStore, true, MI, KS, STG, 0>), grid, block, 0, stream, a, M, K, W, s, N, go);
-        else
-            hipLaunchKernelGGL((k_gemm_q8<kAddF32, true, MI, KS, STG, 0>), grid, block, 0, stream, a, M, K, W, s, N, go);
-        return hipGetLastError();
+        if constexpr (NKC == 0) {
+            if (epi == kStore)
+                hipLaunchKernelGGL((k_gemm_q8<kStore, true, MI, NI, KS, STG, 0>), grid, block, 0, stream, a, M, K, W, s, N, go);
+            else if (epi == kAddF32)
+                hipLaunchKernelGGL((k_gemm_q8<kAddF32, true, MI, NI, KS, STG, 0>), grid, block, 0, stream, a, M, K, W, s, N, go);
+            else
+                return hipErrorInvalidValue;
+            return hipGetLastError();
+        }
+        return hipErrorInvalidValue;
     }
     switch (epi) {
     case kStore: XNP_GEMM(kStore); break;
@@ -565,15 +768,42 @@ static hipError_t gemm_q8_stg(const void *A, int M, int K, const int8_t *W, cons
     return hipGetLastError();
 }
 
+// Runs of row tiles the 256-column groups of k_gemm_q8_wres split M into (a group per CU), or 0 where it
+// is not taken: a group's start (its 128 KB of W loaded and widened) costs about 4 us, so it wants three
+// tiles and more to a run.  2048 rows (two tiles): qkv 10.2 against 9.7 us, linear1 12.5 against 12.8; 5000
+// rows: 14.0 against 17.7 and 20.7 against 26.5; 512 columns (out_proj) 18.8 against 17.6 even at 16384
+// rows.  The epilogues with operands of their own would not fit its registers.
+static int gemm_wres_runs(int M, int K, int N, int epi, const GemmOut &go) {
+    if (K != kWrK || N < 1024 || go.a_f32 || (epi != kStore && epi != kGeluErf && epi != kGeluTanh)) return 0;
+    const int ntn = (N + kWrCols - 1) / kWrCols, tiles = (M + kWrRows - 1) / kWrRows;
+    const int runs = std::min(tiles, std::max(1, 256 / ntn));
+    return (tiles + runs - 1) / runs >= 3 && gemm_staged(N, epi, go) ? runs : 0;
+}
+
+static hipError_t gemm_q8_wres(const void *A, int M, const int8_t *W, const float *s, int N, int epi, const GemmOut &go,
+                               hipStream_t stream) {
+    const int ntn = (N + kWrCols - 1) / kWrCols, tiles = (M + kWrRows - 1) / kWrRows;
+    const int runs = gemm_wres_runs(M, kWrK, N, epi, go), per = (tiles + runs - 1) / runs;
+    const dim3 grid(ntn * ((tiles + per - 1) / per)), block(512);
+    const uint16_t *a = (const uint16_t *)A;
+    switch (epi) {
+    case kStore: hipLaunchKernelGGL(k_gemm_q8_wres<kStore>, grid, block, 0, stream, a, M, W, s, N, go, per); break;
+    case kGeluErf: hipLaunchKernelGGL(k_gemm_q8_wres<kGeluErf>, grid, block, 0, stream, a, M, W, s, N, go, per); break;
+    case kGeluTanh: hipLaunchKernelGGL(k_gemm_q8_wres<kGeluTanh>, grid, block, 0, stream, a, M, W, s, N, go, per); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 // The staged epilogue's kernels come unrolled whole for K of 8 or 16 chunks per half (the flow
 // LM's 512-2048 wide projections); others run the rounds in a loop.
 template <int MI, int KS>
 static hipError_t gemm_q8_mi(const void *A, int M, int K, const int8_t *W, const float *s, int N, int epi,
                              const GemmOut &go, hipStream_t stream) {
-    if (!gemm_staged(N, epi, go)) return gemm_q8_stg<MI, KS, false, 0>(A, M, K, W, s, N, epi, go, stream);
-    if (!go.a_f32 && K == 8 * KS * kGmK) return gemm_q8_stg<MI, KS, true, 8>(A, M, K, W, s, N, epi, go, stream);
-    if (!go.a_f32 && K == 16 * KS * kGmK) return gemm_q8_stg<MI, KS, true, 16>(A, M, K, W, s, N, epi, go, stream);
-    return gemm_q8_stg<MI, KS, true, 0>(A, M, K, W, s, N, epi, go, stream);
+    if (!gemm_staged(N, epi, go)) return gemm_q8_stg<MI, 2, KS, false, 0>(A, M, K, W, s, N, epi, go, stream);
+    if (!go.a_f32 && K == 8 * KS * kGmK) return gemm_q8_stg<MI, 2, KS, true, 8>(A, M, K, W, s, N, epi, go, stream);
+    if (!go.a_f32 && K == 16 * KS * kGmK) return gemm_q8_stg<MI, 2, KS, true, 16>(A, M, K, W, s, N, epi, go, stream);
+    return gemm_q8_stg<MI, 2, KS, true, 0>(A, M, K, W, s, N, epi, go, stream);
 }
 
 hipError_t launch_gemm_q8(const void *A, int M, int K, const int8_t *W, const float *s, int N, int epi,
@@ -585,6 +815,16 @@ hipError_t launch_gemm_q8(const void *A, int M, int K, const int8_t *W, const fl
     const int64_t ntn = (N + kGmT - 1) / kGmT;
     const int64_t groups64 = ntn * ((M + kGmT - 1) / kGmT), groups128 = ntn * ((M + 127) / 128);
     const bool mi1 = groups64 < 512;
+    if (gemm_wres_runs(M, K, N, epi, go) > 0) return gemm_q8_wres(A, M, W, s, N, epi, go, stream);
+    // 128 x 128 tiles (twice the products per barrier and per byte staged of 128 x 64) where they fill the
+    // chip's 512 places (two groups a CU) in nearly whole rounds: 16384 rows, linear2 65 -> 49 us, out_proj
+    // 20.4 -> 17.6; at 5000 rows linear1 (640 groups, the second round of 128) took 33.9 against 30.4.
+    const int64_t wide = (N + 127) / 128 * (int64_t)((M + 127) / 128), rounds = (wide + 511) / 512;
+    if (5 * wide >= 4 * 512 * rounds && !go.a_f32 && gemm_staged(N, epi, go)) {
+        if (K == 8 * kGmK) return gemm_q8_stg<4, 4, 1, true, 8>(A, M, K, W, s, N, epi, go, stream);
+        if (K == 16 * kGmK) return gemm_q8_stg<4, 4, 1, true, 16>(A, M, K, W, s, N, epi, go, stream);
+        if (K == 32 * kGmK) return gemm_q8_stg<4, 4, 2, true, 16>(A, M, K, W, s, N, epi, go, stream);
+    }
     // two halves per group on alternate K chunks when K is long (32 chunks and more)
     if (K >= 32 * kGmK)
         return mi1 ? gemm_q8_mi<1, 2>(A, M, K, W, s, N, epi, go, stream) : gemm_q8_mi<2, 2>(A, M, K, W, s, N, epi, go, stream);

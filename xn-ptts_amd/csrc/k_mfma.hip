@@ -746,7 +746,7 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
 // A and B always hold the same key (or dim) in the same (lane / 32, element) slot, so each
 // contraction is right whatever order the instruction walks k in.
 
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
+
 
 constexpr int kWpChunk = 64;  // keys of a chunk
 constexpr int kWpSlots = 3;   // chunk slots of the LDS ring: 2 chunks load while one is attended

@@ -399,6 +399,7 @@ __device__ __forceinline__ float pow2i(int x) { return __uint_as_float((uint32_t
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(const uint4 &u) {
     bf16x8_t r;
