@@ -79,6 +79,35 @@ def test_linear_q8_on_128_column_tiles_matches_the_oracle(n, epi):
     check_linear_q8(13057 if n == 512 else 1665, 2048 if n == 512 else 1024, n, epi)
 
 
+# Few rows (up to 256) run in one pass per 16 or 32 rows x 32 columns, K of 512, 1024 and 2048: one row, a
+# tile, one more, the most rows and one past them (which takes k_gemm_q8), ragged columns (the flow
+# entry: 40 and 264), every epilogue the flow LM uses there with and without a LayerNorm in front.
+@pytest.mark.parametrize("rows", [1, 16, 17, 130, 256, 257])
+@pytest.mark.parametrize("k,n,epi", [(512, 40, "store"), (512, 264, "silu"), (1024, 520, "gated"), (2048, 512, "axpy_f32"),
+                                     (512, 32, "store_f32"), (2048, 64, "silu_add")])
+def test_flow_linear_q8_of_few_rows_matches_the_oracle(rows, k, n, epi):
+    rng = np.random.default_rng(rows * 11 + k + n)
+    x = normal(rng, (rows, k), "bf16")
+    q, s = xnp.quantize_rows(rng.standard_normal((n, k)).astype(np.float32) * 0.03)
+    b = (0.1 * rng.standard_normal(n)).astype(np.float32)
+    aux = out0 = None
+    if epi == "silu_add":
+        aux = normal(rng, n, "bf16")
+    elif epi == "gated":
+        aux, out0 = normal(rng, (rows, n), "bf16"), normal(rng, (rows, n), "bf16")
+    elif epi == "axpy_f32":
+        aux = rng.standard_normal((rows, n)).astype(np.float32)
+    f32_out = epi in ("axpy_f32", "store_f32")
+    y = (torch.zeros((rows, n), dtype=torch.float32, device=DEV) if f32_out
+         else (dev(out0) if out0 is not None else torch.zeros((rows, n), dtype=torch.bfloat16, device=DEV)))
+    a = None if aux is None else (dev(aux) if epi == "gated" else dev(aux, torch.float32))
+    xnp.flow_linear_q8(dev(x), dev(q, torch.int8), dev(s, torch.float32), y, epi, bias=dev(b, torch.float32), aux=a,
+                       alpha=0.5)
+    torch.cuda.synchronize()
+    want = oracle.flow_linear_q8(x, q, s, epi, bias=b, aux=aux, out=out0, alpha=0.5)
+    assert rel_err(host(y), want) <= TOL
+
+
 def check_linear_q8(rows, k, n, epi):
     rng = np.random.default_rng(rows * 7 + n)
     x = normal(rng, (rows, k), "bf16")

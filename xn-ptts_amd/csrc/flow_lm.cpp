@@ -587,22 +587,23 @@ static xnp_status fl_frame_q8(xnp_flow_lm *lm, int M, const float *latent_in, co
         FL_Q(gemm(lm->bya, false, F, lm->adaq, lm->adab, na, kStore, lm->bada, na, nullptr, 0, 1.f, "adaLN_modulation"));
         for (int r = 0; r < d.flow_depth; r++) { // ResBlock (mlp.rs:113-131)
             const uint16_t *mod = lm->bada + (size_t)r * 3 * F;
-            FL_TRY(launch_layer_norm_mod(lm->bxf, M, F, lm->W(L.rb_lnw[r]), lm->W(L.rb_lnb[r]), 1e-6f, mod, mod + F, na,
-                                         lm->bh, hs),
-                   "in_ln");
-            FL_Q(gemm(lm->bh, false, F, lm->rb1[r], lm->W(L.rb_b1[r]), F, kSilu, lm->bh2, F, nullptr, 0, 1.f, "mlp.0"));
+            RowNorm in;
+            in.w = lm->W(L.rb_lnw[r]), in.b = lm->W(L.rb_lnb[r]), in.eps = 1e-6f, in.shift = mod, in.scale = mod + F, in.ld_mod = na;
+            GemmOut h2;
+            h2.out[0] = lm->bh2, h2.ld[0] = F, h2.bias = lm->W(L.rb_b1[r]);
+            FL_TRY(launch_norm_gemm_q8(lm->bxf, M, F, in, lm->bh, lm->rb1[r].q, lm->rb1[r].s, F, kSilu, h2, hs), "in_ln and mlp.0");
             FL_Q(gemm(lm->bh2, false, F, lm->rb2[r], lm->W(L.rb_b2[r]), F, kGated, lm->bxf, F, mod + 2 * F, na, 1.f,
                       "mlp.2"));
         }
         const uint16_t *fmod = lm->bada + (size_t)d.flow_depth * 3 * F; // FinalLayer (mlp.rs:155-163)
-        FL_TRY(launch_layer_norm_mod(lm->bxf, M, F, nullptr, nullptr, 1e-6f, fmod, fmod + F, na, lm->bh, hs),
-               "norm_final");
-        if (d.flow_type == XNP_FLOW_DRIFTING)
-            FL_Q(gemm(lm->bh, false, F, lm->finw, lm->W(L.fin_b), ld, kStoreF32, latent_out, ld, nullptr, 0, 1.f,
-                      "final linear"));
-        else
-            FL_Q(gemm(lm->bh, false, F, lm->finw, lm->W(L.fin_b), ld, kAxpyF32, latent_out, ld, cur, ld,
-                      lsd ? 1.0f / (float)steps : 1.0f, "final linear"));
+        RowNorm nf;
+        nf.eps = 1e-6f, nf.shift = fmod, nf.scale = fmod + F, nf.ld_mod = na;
+        const bool drift = d.flow_type == XNP_FLOW_DRIFTING;
+        GemmOut o;
+        o.out[0] = latent_out, o.ld[0] = ld, o.bias = lm->W(L.fin_b);
+        if (!drift) o.aux = cur, o.ld_aux = ld, o.alpha = lsd ? 1.0f / (float)steps : 1.0f;
+        FL_TRY(launch_norm_gemm_q8(lm->bxf, M, F, nf, lm->bh, lm->finw.q, lm->finw.s, ld, drift ? kStoreF32 : kAxpyF32, o, hs),
+               "norm_final and final linear");
     }
 #undef FL_Q
     return XNP_OK;

@@ -720,6 +720,190 @@ __global__ __launch_bounds__(512, 2) void k_gemm_q8_wres(const uint16_t *A, int 
     store_tile(t1 - 1);
 }
 
+// The same product for few rows (K of 512, 1024 or 2048), with a LayerNorm of the rows in front when
+// LNM is not 0 (K = 512; LNM - 1 is k_layer_norm's MODE).  At these sizes a launch is a chain of round
+// trips, not work: k_gemm_q8 stages K chunk by chunk and the LayerNorm was a launch of its own.  Here one
+// work group of 8 waves takes 16 MT rows x 32 columns, wave w the K slice from w K / 8, and loads its
+// whole share of A and W at once, straight into the MFMA's operand layout (lane (l16, g): row or column
+// l16, 16 consecutive k from 64 i + 16 g, whose halves are the operands of two products; the k order is
+// the same for both).  D = W A^T (lane: row l16, columns 4 g + r) goes to LDS, the waves' shares are
+// added in k order, y leaves by the staged epilogue.
+//
+// The LayerNorm is k_layer_norm's to the bit: its lane j holds k 8 j .. + 7, here the two halves of
+// lane (l16, g) of wave w (j = 8 w + 2 g, + 1), and its reduction pairs j over bits 0, 1, .. 5: the
+// halves, g's two bits by row swaps, the waves' three through LDS.  (Rows and both sides' times: the
+// rule at gemm_small.)
+struct LnIn {
+    const float *w = nullptr, *b = nullptr;
+    float eps = 1e-5f;
+    const uint16_t *shift = nullptr, *scale = nullptr;
+    int ld_mod = 0;
+};
+
+template <int EPI, int NS, int MT, int LNM>
+__global__ __launch_bounds__(512) void k_gemm_q8_small(const uint16_t *A, int M, const int8_t *W, const float *s, int N,
+                                                       GemmOut go, LnIn ln) {
+    static_assert(LNM == 0 || NS == 1, "the LayerNorm takes rows of 512");
+    constexpr int K = 512 * NS, MODE = LNM - 1;
+    __shared__ __attribute__((aligned(16))) float red[8][16 * MT][36];
+    __shared__ __attribute__((aligned(16))) uint16_t yt[16 * MT][40];
+    __shared__ float mom[2][8][16 * MT];
+    // row tiles fastest: an XCD's run of groups shares its columns of W
+    const int mts = (M + 16 * MT - 1) / (16 * MT), tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int m0 = tile % mts * (16 * MT), n0 = tile / mts * 32;
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
+    const int k0 = 64 * NS * w + 16 * g;
+    uint4 wr[2][NS], ar[MT][NS][2];
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wr[j][i] = *(const uint4 *)(W + (size_t)min(n0 + 16 * j + l16, N - 1) * K + k0 + 64 * i);
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                ar[j][i][b] = *(const uint4 *)(A + (size_t)min(m0 + 16 * j + l16, M - 1) * K + k0 + 64 * i + 8 * b);
+    }
+    float4 aw[4], ab[4];
+    uint4 rsh[MT][2], rsc[MT][2];
+    if constexpr (LNM > 0) {
+        if constexpr ((MODE & kLnAffine) != 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                aw[i] = *(const float4 *)(ln.w + k0 + 4 * i);
+                ab[i] = *(const float4 *)(ln.b + k0 + 4 * i);
+            }
+        }
+        if constexpr ((MODE & kLnMod) != 0) {
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    const size_t o = (size_t)min(m0 + 16 * j + l16, M - 1) * ln.ld_mod + k0 + 8 * b;
+                    rsh[j][b] = *(const uint4 *)(ln.shift + o);
+                    rsc[j][b] = *(const uint4 *)(ln.scale + o);
+                }
+        }
+    }
+    // what the tail needs: this thread's sum is row tid / 32 (+ 16 j), column tid % 32; the first 64 MT
+    // threads store 8 columns of a row
+    const int sn = min(n0 + (tid & 31), N - 1);
+    const float sc = s[sn], bn = go.bias ? go.bias[sn] : 0.f;
+    const int er = tid >> 2, ec = 8 * (tid & 3), em = m0 + er, ne = n0 + ec;
+    const bool mine = tid < 64 * MT && em < M && ne < N;
+    EpiPiece piece;
+    EpiCols cols;
+    if (mine) {
+        epi_load<EPI>(go, em, ne, piece);
+        epi_cols<EPI>(go, ne, cols);
+    }
+    __builtin_amdgcn_sched_barrier(0); // the loads above go out together
+
+    if constexpr (LNM > 0) {
+        float v[MT][2][8];
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[j][b][i] = epi_y(ar[j][0][b], i);
+        auto moment = [&](float (&p)[MT], int which) {
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                p[j] = swap_sum<32>(swap_sum<16>(p[j]));
+                if (g == 0) mom[which][w][16 * j + l16] = p[j];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                float q[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) q[i] = mom[which][i][16 * j + l16];
+                p[j] = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+            }
+        };
+        float sum[MT], sq[MT];
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            float p[2] = {0.f, 0.f};
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) p[b] += v[j][b][i];
+            sum[j] = p[0] + p[1];
+        }
+        moment(sum, 0);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            sum[j] = sum[j] / (float)K; // the mean
+            float p[2] = {0.f, 0.f};
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float d = v[j][b][i] - sum[j];
+                    p[b] = __builtin_fmaf(d, d, p[b]);
+                }
+            sq[j] = p[0] + p[1];
+        }
+        moment(sq, 1);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const float rstd = 1.0f / __builtin_sqrtf(sq[j] / (float)K + ln.eps);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                float y[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    y[i] = (v[j][b][i] - sum[j]) * rstd;
+                    if constexpr ((MODE & kLnAffine) != 0)
+                        y[i] = y[i] * ((const float *)&aw[2 * b])[i] + ((const float *)&ab[2 * b])[i];
+                    if constexpr ((MODE & kLnMod) != 0) {
+                        const float sc1 = bf16_value(bf16_bits(epi_y(rsc[j][b], i) + 1.0f));
+                        y[i] = bf16_value(bf16_bits(bf16_value(bf16_bits(y[i])) * sc1)) + epi_y(rsh[j][b], i);
+                    }
+                }
+                ar[j][0][b] = make_uint4(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]), pack_bf16(y[4], y[5]), pack_bf16(y[6], y[7]));
+            }
+        }
+    }
+    f32x4_t acc[MT][2];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[j][0] = acc[j][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto widen4 = [](uint32_t a, uint32_t b) { // 8 int8 -> bf16 (exact: |q| <= 127)
+        auto two = [](uint32_t u, int sh) {
+            return pack_bf16((float)(int8_t)((u >> sh) & 0xffu), (float)(int8_t)((u >> (sh + 8)) & 0xffu));
+        };
+        return as_bf16x8(make_uint4(two(a, 0), two(a, 16), two(b, 0), two(b, 16)));
+    };
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const bf16x8_t w0 = widen4(wr[n][i].x, wr[n][i].y), w1 = widen4(wr[n][i].z, wr[n][i].w);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, as_bf16x8(ar[j][i][0]), acc[j][n], 0, 0, 0);
+                acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, as_bf16x8(ar[j][i][1]), acc[j][n], 0, 0, 0);
+            }
+        }
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) *(f32x4_t *)&red[w][16 * j + l16][16 * n + 4 * g] = acc[j][n];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const int row = 16 * j + (tid >> 5), col = tid & 31;
+        float v = red[0][row][col];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) v += red[i][row][col]; // in k order
+        yt[row][col] = (uint16_t)bf16_bits(go.bias ? v * sc + bn : v * sc);
+    }
+    __syncthreads();
+    if (mine) epi_store<EPI>(go, em, *(const uint4 *)&yt[er][ec], piece, cols);
+}
+
 // The staged epilogue's conditions: 8-column pieces that stay inside N and inside one kStore segment,
 // and 16-byte aligned accesses to every output and operand row.
 static bool gemm_staged(int N, int epi, const GemmOut &go) {
@@ -806,10 +990,80 @@ static hipError_t gemm_q8_mi(const void *A, int M, int K, const int8_t *W, const
     return gemm_q8_stg<MI, 2, KS, true, 0>(A, M, K, W, s, N, epi, go, stream);
 }
 
+// Rows up to which k_gemm_q8_small is taken: each of its groups reads its rows and columns over all of K
+// (no tile larger than 32 x 32), which the larger tiles of k_gemm_q8 overtake.  A step of 9 layers (512
+// wide, FF 2048, caches of up to 800 rows; k_gemm_q8 with the LayerNorms apart, then here): 32 rows 360 and
+// 272 us, 128 rows 472 and 408, 256 rows 625 and 597, 300 rows 685 and 696.  The four projections alone,
+// warm: 40 rows 20.7 and 15.1 us, 256 rows 21.4 and 19.4, 600 rows 26.1 and 36.8.
+constexpr int kSmallRows = 256;
+static bool gemm_small(int M, int K, int N, int epi, const GemmOut &go) {
+    return M <= kSmallRows && (K == 512 || K == 1024 || K == 2048) && !go.a_f32 && gemm_staged(N, epi, go);
+}
+
+template <int EPI, int NS, int LNM>
+static hipError_t gemm_q8_small(const void *A, int M, const int8_t *W, const float *s, int N, const GemmOut &go,
+                                const LnIn &ln, hipStream_t stream) {
+    // two row tiles a group (its columns of W read and widened for both) once one-tile groups are more than
+    // the CUs: linear1 at 128 rows 4.3 -> 4.0 us, linear2 at 331 rows 9.2 -> 7.9
+    const int ntn = (N + 31) / 32, mts = (M + 15) / 16;
+    const uint16_t *a = (const uint16_t *)A;
+    if (ntn * mts > 256)
+        hipLaunchKernelGGL((k_gemm_q8_small<EPI, NS, 2, LNM>), dim3(ntn * ((M + 31) / 32)), dim3(512), 0, stream, a, M, W, s, N, go, ln);
+    else
+        hipLaunchKernelGGL((k_gemm_q8_small<EPI, NS, 1, LNM>), dim3(ntn * mts), dim3(512), 0, stream, a, M, W, s, N, go, ln);
+    return hipGetLastError();
+}
+
+template <int NS>
+static hipError_t gemm_q8_small_epi(const void *A, int M, const int8_t *W, const float *s, int N, int epi, const GemmOut &go,
+                                    hipStream_t stream) {
+    switch (epi) {
+    case kStore: return gemm_q8_small<kStore, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kGeluErf: return gemm_q8_small<kGeluErf, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kGeluTanh: return gemm_q8_small<kGeluTanh, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kResidual: return gemm_q8_small<kResidual, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kSilu: return gemm_q8_small<kSilu, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kSiluAddVec: return gemm_q8_small<kSiluAddVec, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kGated: return gemm_q8_small<kGated, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kAxpyF32: return gemm_q8_small<kAxpyF32, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kStoreF32: return gemm_q8_small<kStoreF32, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    case kAddF32: return gemm_q8_small<kAddF32, NS, 0>(A, M, W, s, N, go, LnIn(), stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+// LayerNorm (norm: the affine, the modulation) then the projection; h: M x K bf16 of scratch, taken where
+// the two run apart.  Fused for few rows of 512 with the epilogues the flow LM pairs with a norm.
+hipError_t launch_norm_gemm_q8(const void *x, int M, int K, const RowNorm &norm, void *h, const int8_t *W, const float *s,
+                               int N, int epi, const GemmOut &go, hipStream_t stream) {
+    if (M <= 0) return hipSuccess;
+    if (K == 512 && gemm_small(M, K, N, epi, go) && (norm.w == nullptr) == (norm.b == nullptr) &&
+        (norm.shift == nullptr) == (norm.scale == nullptr) && (!norm.shift || norm.ld_mod % 8 == 0)) {
+        LnIn ln;
+        ln.w = norm.w, ln.b = norm.b, ln.eps = norm.eps;
+        ln.shift = (const uint16_t *)norm.shift, ln.scale = (const uint16_t *)norm.scale, ln.ld_mod = norm.ld_mod;
+        const int mode = (norm.w ? kLnAffine : 0) | (norm.shift ? kLnMod : 0);
+        if (mode == kLnAffine && epi == kStore) return gemm_q8_small<kStore, 1, 1 + kLnAffine>(x, M, W, s, N, go, ln, stream);
+        if (mode == kLnAffine && epi == kGeluErf) return gemm_q8_small<kGeluErf, 1, 1 + kLnAffine>(x, M, W, s, N, go, ln, stream);
+        if (mode == kLnAffine && epi == kGeluTanh) return gemm_q8_small<kGeluTanh, 1, 1 + kLnAffine>(x, M, W, s, N, go, ln, stream);
+        if (mode == (kLnAffine | kLnMod) && epi == kSilu)
+            return gemm_q8_small<kSilu, 1, 1 + (kLnAffine | kLnMod)>(x, M, W, s, N, go, ln, stream);
+        if (mode == kLnMod && epi == kAxpyF32) return gemm_q8_small<kAxpyF32, 1, 1 + kLnMod>(x, M, W, s, N, go, ln, stream);
+        if (mode == kLnMod && epi == kStoreF32) return gemm_q8_small<kStoreF32, 1, 1 + kLnMod>(x, M, W, s, N, go, ln, stream);
+    }
+    const hipError_t e = launch_layer_norm_mod(x, M, K, norm.w, norm.b, norm.eps, norm.shift, norm.scale, norm.ld_mod, h, stream);
+    return e != hipSuccess ? e : launch_gemm_q8(h, M, K, W, s, N, epi, go, stream);
+}
+
 hipError_t launch_gemm_q8(const void *A, int M, int K, const int8_t *W, const float *s, int N, int epi,
                           const GemmOut &go, hipStream_t stream) {
     if (M <= 0) return hipSuccess;
     if (N <= 0 || K <= 0 || K % 16) return hipErrorInvalidValue;
+    if (gemm_small(M, K, N, epi, go)) {
+        if (K == 512) return gemm_q8_small_epi<1>(A, M, W, s, N, epi, go, stream);
+        if (K == 1024) return gemm_q8_small_epi<2>(A, M, W, s, N, epi, go, stream);
+        return gemm_q8_small_epi<4>(A, M, W, s, N, epi, go, stream);
+    }
     // 32-row tiles when 64-row ones would leave the chip's 1024 SIMDs under two waves each; 128-row
     // tiles when those still give 512 groups (two per CU)
     const int64_t ntn = (N + kGmT - 1) / kGmT;

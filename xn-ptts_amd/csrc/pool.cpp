@@ -1640,24 +1640,25 @@ static xnp_status layer_step_impl(xnp_pool *pool, int32_t layer, const xnp_layer
     hipStream_t hs = pool->batch.stream;
     const int M = (int)rows;
     // self-attention block: x + layer_scale_1(out_proj(attn(in_proj(norm1(x)))))
-    HIP_TRY(launch_layer_norm(x, M, dm, w->ln1_w, w->ln1_b, 1e-5f, S.h, hs), "norm1");
+    RowNorm norm;
+    norm.w = w->ln1_w, norm.b = w->ln1_b;
     GemmOut qkv;
     qkv.nseg = 3;
     qkv.out[0] = S.q, qkv.ld[0] = qd, qkv.col0[0] = 0;
     qkv.out[1] = S.k, qkv.ld[1] = kd, qkv.col0[1] = qd;
     qkv.out[2] = S.v, qkv.ld[2] = kd, qkv.col0[2] = qd + kd;
-    HIP_TRY(launch_gemm_q8(S.h, M, dm, w->wqkv, w->sqkv, nqkv, kStore, qkv, hs), "in_proj");
+    HIP_TRY(launch_norm_gemm_q8(x, M, dm, norm, S.h, w->wqkv, w->sqkv, nqkv, kStore, qkv, hs), "norm1 and in_proj");
     if (xnp_status st = xnp_attend(pool, layer, S.q, S.k, S.v, S.att, 1.0f / std::sqrt((float)D), hip_stream))
         return st;
     GemmOut res;
     res.out[0] = x, res.ld[0] = dm, res.ls = w->ls1;
     HIP_TRY(launch_gemm_q8(S.att, M, qd, w->wout, w->sout, dm, kResidual, res, hs), "out_proj");
     // feed-forward block: x + layer_scale_2(linear2(gelu(linear1(norm2(x)))))
-    HIP_TRY(launch_layer_norm(x, M, dm, w->ln2_w, w->ln2_b, 1e-5f, S.h, hs), "norm2");
+    norm.w = w->ln2_w, norm.b = w->ln2_b;
     GemmOut hid;
     hid.out[0] = S.f, hid.ld[0] = ff;
-    HIP_TRY(launch_gemm_q8(S.h, M, dm, w->w1, w->s1, ff, w->gelu == XNP_GELU_ERF ? kGeluErf : kGeluTanh, hid, hs),
-            "linear1");
+    HIP_TRY(launch_norm_gemm_q8(x, M, dm, norm, S.h, w->w1, w->s1, ff, w->gelu == XNP_GELU_ERF ? kGeluErf : kGeluTanh, hid, hs),
+            "norm2 and linear1");
     res.ls = w->ls2;
     HIP_TRY(launch_gemm_q8(S.f, M, ff, w->w2, w->s2, dm, kResidual, res, hs), "linear2");
     return XNP_OK;

@@ -201,6 +201,17 @@ hipError_t launch_layer_norm_mod(const void *x, int rows, int dim, const float *
                                  const void *shift, const void *scale, int ld_mod, void *out, hipStream_t stream);
 hipError_t launch_gemm_q8(const void *A, int M, int K, const int8_t *W, const float *s, int N, int epi,
                           const GemmOut &go, hipStream_t stream);
+// A LayerNorm of bf16 rows in front of a projection: launch_layer_norm_mod's operands.
+struct RowNorm {
+    const float *w = nullptr, *b = nullptr;
+    float eps = 1e-5f;
+    const void *shift = nullptr, *scale = nullptr;
+    int32_t ld_mod = 0;
+};
+// launch_layer_norm_mod into h then launch_gemm_q8 of h, to the bit; in one launch for few rows (h is
+// then left as it is).  x and the outputs are different buffers.
+hipError_t launch_norm_gemm_q8(const void *x, int M, int K, const RowNorm &norm, void *h, const int8_t *W, const float *s,
+                               int N, int epi, const GemmOut &go, hipStream_t stream);
 // Epilogues of the f32 linear (launch_linear_f32), y = x W^T + b:
 //   kLinStore out = y; kLinGelu* out = gelu(y); kLinSilu out = silu(y); kLinSiluAddVec
 //   out = silu(y + aux[n]); kLinResidual out += y; kLinGated out += aux[m][n] * y; kLinAxpy
