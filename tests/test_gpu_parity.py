@@ -396,6 +396,26 @@ def test_window_caches_match_mimis_kv_cache(cache, act):
         assert pool.current_end(wids[i]) == contexts[i]  # rows held: the window, full
 
 
+# A bf16 window step of more than 4 rows writes its rows from the attention's own launch: over fresh windows
+# (every 256-row round a work group), over held rows when the window has 192 and more rows and no heads
+# share a kv head; otherwise an append runs after.  Windows of 40, 191, 192 and 250 rows: a fresh chunk
+# shorter than the window or of several rounds, chunks over held rows shorter and longer than the window
+# and than a round, single and few rows between, every held row bit for bit after each.
+@pytest.mark.parametrize("context", [40, 191, 192, 250])
+@pytest.mark.parametrize("steps", [(7, 300, 30, 2, 64, 5), (300, 1, 257, 513, 100), (600, 250, 8)])
+def test_window_chunks_write_their_rows(context, steps):
+    L, H = 1, 2
+    pool = xnp.KvPool(num_layers=L, num_heads=H, num_blocks=80, max_streams=4, max_blocks_per_stream=16,
+                      cache_dtype="bf16", act_dtype="bf16", max_pos=4096, page_seed=8)
+    ids = [pool.init_window(context) for _ in range(2)]
+    orcs = [oracle.Window(L, H, 64, context, rows_max=600, act="bf16") for _ in range(2)]
+    rng = np.random.default_rng(59)
+    for t in steps:
+        _window_batch(pool, ids, orcs, t, L, H, "bf16", "bf16", rng)
+        for i in range(2):
+            _assert_window_rows(pool, ids[i], orcs[i], context, L, H, "bf16")
+
+
 # Steps of a few rows attend them in one launch (up to 4, and no more than the smallest window holds;
 # f32 runs longer steps 4 rows a launch): windows of 1 row, less than a page, a page, a ragged two and
 # a half and seven pages, empty, filling and full, more than 1024 groups (one wave each) and few

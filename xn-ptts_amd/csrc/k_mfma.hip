@@ -720,7 +720,9 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
 // virtually: the window's held rows first (j < ncache, oldest first, at slot (wbase + j) mod W),
 // then the chunk's rows (j = ncache + i: input row i, rotated at its position and rounded to bf16).
 // Query row i has virtual index ncache + i and sees key j when ncache + i - W < j <= ncache + i.
-// The chunk's rows reach the window by their own append (k_window_append); this kernel only reads.
+// The rows that stay are written by the group of the last round as they pass through its LDS, where that
+// cannot race with a read (window_append_fused); k_window_append read and wrote them again in 30 us of the
+// 139 a layer took.  Fresh windows take a group per round.  160 clips of 375 rows, 2 layers: 282 -> 226 us.
 //
 // Query rows are taken in rounds of 256: 8 pairs of 16-row tiles, pair i rows 32 i .. 32 i + 31 of
 // the round, wave w owning pair w.  A round's keys (from the window of its first row to
@@ -787,13 +789,16 @@ __device__ __forceinline__ void wait_chunks(int ahead) {
 }
 
 __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_prefill_window(
-    PoolView pv, BatchView bv, int layer, const void *q, const void *knew, const void *vnew, void *out, float qmul) {
+    PoolView pv, BatchView bv, int layer, const void *q, const void *knew, const void *vnew, void *out, float qmul,
+    int append) {
     __shared__ __attribute__((aligned(16))) uint16_t ks[kWpSlots][kWpChunk][kHeadDim]; // K, [key][unit ^ swz]
     __shared__ __attribute__((aligned(16))) uint16_t vs[kWpSlots][kWpChunk][kHeadDim]; // V, [key][unit ^ swz]
     __shared__ __attribute__((aligned(16))) uint4 rs[kWpSlots][kWpWaves][kWpLoadsC][64]; // the lanes' rope pieces
     __shared__ int32_t spages[kPfMaxPages];
     const int t = bv.t;
-    const int h = blockIdx.x % pv.H, b = blockIdx.x / pv.H;
+    // one group for every round of a (stream, head), or (a grid of several rounds, the last first) one each
+    const int per = bv.n * pv.H, rounds = (int)gridDim.x / per, round = rounds - 1 - (int)blockIdx.x / per;
+    const int h = (int)blockIdx.x % per % pv.H, b = (int)blockIdx.x % per / pv.H;
     const StreamPlan P = bv.plans[b];
     const int32_t *tab = pv.tables + (size_t)P.sid * pv.mbps;
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, hi = lane >> 5, col = lane & 31;
@@ -848,20 +853,38 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
             dma16(pv.rope16 + (size_t)(P.key_pos + r) * (kHeadDim / 2) + 4 * unit, &rs[slot][w][i][0]);
         }
     };
+    // the rows that stay (KvCache::trim): the step's last min(t, W), the first of them in slot s0; with
+    // `append` the group of the last round writes them as they pass through its LDS, whole rows of 128
+    // bytes, from the lanes that hold them (one query head per kv head writes)
+    const int keep = min(t, W), s0 = (P.pos + t - keep) % W;
+    const bool writes = append && h % (pv.H / pv.KVH) == 0;
     // ...then, once they have landed, the step's own keys rotated in place by the lane that loaded
     // them
-    auto settle = [&](int j0, int khi, int slot) {
+    auto settle = [&](int j0, int khi, int slot, bool last) {
         const int ln = lane_here(lane);
 #pragma unroll
         for (int i = 0; i < kWpLoadsC; ++i) {
             const int key = kWpKeysW * w + 8 * i + (ln >> 3), j = j0 + key;
             if (j >= khi || j < nfrom) continue;
             uint4 *kp = (uint4 *)&ks[slot][key][8 * (ln & 7)]; // this lane's own pieces
-            *kp = rotate8(*kp, rs[slot][w][i][ln]);
+            const uint4 kk = rotate8(*kp, rs[slot][w][i][ln]);
+            *kp = kk;
+            const int r = j - ncache - (t - keep); // the row's place among those that stay
+            if (last && writes && r >= 0) {
+                int s = s0 + r;
+                if (s >= W) s -= W;
+                const int pg = spages[s >> 4];
+                if (pg >= 0 && pg < pv.NB) {
+                    const size_t poff = (size_t)pg * page_elems + (s & 15) * kHeadDim + 8 * ((ln & 7) ^ swz(key));
+                    st_stream(kpages + poff, kk);
+                    st_stream(vpages + poff, *(const uint4 *)&vs[slot][key][8 * (ln & 7)]);
+                }
+            }
         }
     };
-    const int nqt = (t + 15) / 16;
-    for (int tq0 = 0; tq0 < nqt; tq0 += kWpRound / 16) {
+    const int nqt = (t + 15) / 16, tq_first = rounds > 1 ? round * (kWpRound / 16) : 0;
+    const int tq_end = rounds > 1 ? min(nqt, tq_first + kWpRound / 16) : nqt;
+    for (int tq0 = tq_first; tq0 < tq_end; tq0 += kWpRound / 16) {
         const int nq = min(kWpRound / 16, nqt - tq0);
         // the round's keys: from the window of its first row to its last row
         const int khi = ncache + min(t, 16 * (tq0 + nq));
@@ -876,7 +899,7 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
         // chunk loads write LDS, so a later round's wait until every reader of the previous round is
         // done.  The round's first chunk goes out ahead of the queries when it reads no page (keys of
         // the step itself), the rest of the ring once the queries are in.
-        if (tq0 > 0) __syncthreads();
+        if (tq0 > tq_first) __syncthreads();
         const bool early = klo >= nfrom;
         if (early) issue(klo, khi, 0);
         {
@@ -942,7 +965,7 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
                 // this lane's loads of chunk c have landed: after them it issued chunk c + 1 (chunks
                 // 0 .. 2 went out first, then one a step)
                 wait_chunks(min(c == 0 ? kWpSlots - 1 : kWpSlots - 2, nch - 1 - c));
-                settle(j0, khi, u);
+                settle(j0, khi, u, tq0 + nq == nqt);
                 lds_barrier(); // chunk c is in LDS; every wave is done with chunk c - 1's slot
                 if (c > 0 && c + kWpSlots - 1 < nch)
                     issue(j0 + kWpChunk * (kWpSlots - 1), khi, (u + kWpSlots - 1) % kWpSlots);
@@ -1410,6 +1433,17 @@ hipError_t launch_decode_gqa(const PoolView &pv, const BatchView &bv, int layer,
 }
 
 static int prefill_rounds(int t) { return (t + kPfRound - 1) / kPfRound; }
+static_assert(kPfRound == kWpRound, "prefill_rounds counts both kernels' rounds");
+
+// The window's rows written by the attention itself.  A row that stays takes the slot of the position W
+// before it, which may be held and read by the same launch.  Without held rows nothing reads the pages
+// (and the rounds may be groups of their own).  With them, a (stream, head) must be one group (no query
+// head shares its kv head), which loads that position's key W keys before the row: with 192 and more,
+// at least two chunks earlier, so every wave's load of it has landed, the barrier of the chunk before
+// the row's being past.  Otherwise k_window_append runs after.
+bool window_append_fused(const PoolView &pv, const BatchView &bv) {
+    return bv.wheld == 0 || (pv.H == pv.KVH && bv.wmin >= 192);
+}
 
 hipError_t launch_prefill_mfma(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
                                const void *v, void *out, float scale, bool fused, bool window, hipStream_t stream,
@@ -1417,8 +1451,8 @@ hipError_t launch_prefill_mfma(const PoolView &pv, const BatchView &bv, int laye
     if ((fused || window) && (!k || !v)) return hipErrorInvalidValue; // the step's own rows are read from k, v
     const float qmul = scale * 1.4426950408889634f;
     if (window)
-        XNP_LAUNCH(k_prefill_window, dim3(bv.n * pv.H), dim3(64 * kWpWaves), stream, tm, pv, bv, layer, q, k, v, out,
-                   qmul);
+        XNP_LAUNCH(k_prefill_window, dim3(bv.n * pv.H * (bv.wheld == 0 ? prefill_rounds(bv.t) : 1)), dim3(64 * kWpWaves), stream, tm,
+                   pv, bv, layer, q, k, v, out, qmul, window_append_fused(pv, bv) ? 1 : 0);
     else if (bv.kmax <= kPfFastKeys && fused)
         XNP_LAUNCH(k_prefill_fast<true>, dim3(bv.n * pv.H), dim3(64 * kPfWaves), stream, tm, pv, bv, layer, q, k, v,
                    out, qmul);

@@ -168,7 +168,6 @@ struct xnp_pool {
         std::vector<std::pair<int32_t, int32_t>> taken; // (stream, block) pages taken by begin
         BatchView bv{};
         bool wsteps = false; // a step of several rows on window caches
-        int32_t wmin = 0;    // its smallest window
     } batch;
 
     PoolView view() const {
@@ -1334,10 +1333,13 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
     B.bv.masks = (const uint32_t *)(pool->dbatch + o_masks);
     B.bv.wrow = -1;
     B.bv.wrows = 0;
-    B.wmin = 0;
+    B.bv.wheld = B.bv.wmin = 0;
     if (wsteps) {
-        B.wmin = pool->streams[ids[0]].window;
-        for (int32_t i = 1; i < n; i++) B.wmin = std::min(B.wmin, pool->streams[ids[i]].window);
+        B.bv.wmin = pool->streams[ids[0]].window;
+        for (int32_t i = 0; i < n; i++) {
+            B.bv.wmin = std::min(B.bv.wmin, pool->streams[ids[i]].window);
+            B.bv.wheld = std::max(B.bv.wheld, pool->streams[ids[i]].current_end);
+        }
     }
     B.bv.n = n;
     B.bv.t = t;
@@ -1411,11 +1413,12 @@ extern "C" xnp_status xnp_attend(xnp_pool *pool, int32_t layer, const void *q, c
             // every row's windowed attention in one MFMA launch (the held rows from the pages, the
             // step's own from k and v), then the rows that stay into their slots
             HIP_TRY(launch_window_prefill(pool->view(), B.bv, layer, q, k, v, out, scale, B.stream, tm), "window attend");
-            HIP_TRY(launch_window_append(pool->view(), B.bv, layer, k, v, B.stream), "window append");
+            if (!window_append_fused(pool->view(), B.bv))
+                HIP_TRY(launch_window_append(pool->view(), B.bv, layer, k, v, B.stream), "window append");
             return XNP_OK;
         }
         BatchView bv = B.bv;
-        const int32_t most = std::min(window_rows_max(pool->view()), B.wmin); // the rows' slots distinct
+        const int32_t most = std::min(window_rows_max(pool->view()), bv.wmin); // the rows' slots distinct
         for (int32_t r = 0; r < B.t; r += bv.wrows) {
             bv.wrow = r; // the kernel derives the rows' record from the step's
             bv.wrows = std::min(most, B.t - r);

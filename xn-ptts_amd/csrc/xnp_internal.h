@@ -69,6 +69,7 @@ struct BatchView {
     int32_t prefix; // 1 if some stream of the batch is an absolute ring keeping a prefix
     int32_t wrow;   // a window step run a few rows a launch: the first row this launch attends (-1 otherwise)
     int32_t wrows;  // ... and how many it attends
+    int32_t wheld, wmin; // a window step of several rows: the most rows a window holds, the smallest window
     int32_t kmax;   // a prompt step (t > 1): the most key slots a stream of it attends, write_slot + t
 };
 
@@ -159,6 +160,7 @@ hipError_t launch_window_prefill(const PoolView &pv, const BatchView &bv, int la
 int window_rows_max(const PoolView &pv);
 hipError_t launch_window_rows(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
                               const void *v, void *out, float scale, hipStream_t stream, const LaunchTiming &timing);
+bool window_append_fused(const PoolView &pv, const BatchView &bv); // launch_window_prefill writes the rows itself
 hipError_t launch_window_append(const PoolView &pv, const BatchView &bv, int layer, const void *k, const void *v,
                                 hipStream_t stream);
 hipError_t launch_evict_rotate(const PoolView &pv, const EvictRow *rows, int n,
