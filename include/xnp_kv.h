@@ -191,9 +191,9 @@ xnp_status xnp_stream_load_kv(xnp_pool *pool, int32_t id, int32_t layer, const f
  * number of rows t, more than the window included (Mimi's encoder over a whole voice clip,
  * tts_model.rs:509-515; its decoder takes 2 a frame): with t > 1 every stream of the batch must be
  * a window cache, and xnp_attend is the only per-layer call such a batch takes.  On a bf16 pool a
- * step of more than 4 rows runs every row's windowed attention in one MFMA launch, then writes the
- * last min(t, window) rows into their slots; shorter steps, and every step on f32 and int8 pools,
- * run row by row.  xnp_stream_fork clones a window as it is, every page copied
+ * step of more than 4 rows runs every row's windowed attention in one MFMA launch and writes the
+ * last min(t, window) rows into their slots; shorter steps, and f32 pools, run up to 4 rows a launch,
+ * int8 pools and grouped heads row by row.  xnp_stream_fork clones a window as it is, every page copied
  * (transformer.rs:348-354). */
 xnp_status xnp_window_open(xnp_pool *pool, int32_t window, int32_t *id);
 

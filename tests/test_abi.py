@@ -561,3 +561,20 @@ def test_random_stream_lifecycles_keep_the_page_accounting():
     for sid in list(model):
         p.close(sid)
     assert p.stats()["free_blocks"] == NB
+
+
+def test_a_ring_started_full_needs_a_write_slot():
+    # a ring's write slot starts after the rows it holds: past the last slot when it is full, where a
+    # step is refused (it would read the slot map past its end) until a slot is evicted and set
+    p = xnp.KvPool(num_layers=1, num_heads=2, num_blocks=4, max_streams=1, max_blocks_per_stream=2, host_only=True)
+    sid = p.init_state(32)
+    p.advance(sid, 32)
+    p.start_ring(sid, "absolute", prefix=0)
+    with pytest.raises(xnp.XnpError) as e:
+        p.begin([sid])
+    assert e.value.name == "XNP_E_RING"
+    p.evict(sid, 0, [3])
+    p.set_ring_slot(sid, 3)
+    p.begin([sid])
+    p.end()
+    assert all(p.valid(sid))

@@ -1102,6 +1102,8 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
             windows++;
         } else if (s->ring != RING_NONE) {
             if (t != 1) return fail(XNP_E_RING, "a ring cache takes one row at a time, not %d", t);
+            if (s->write >= s->capacity) // a ring started full, its write slot not set yet
+                return fail(XNP_E_RING, "slot %d of a %d-slot ring", s->write, s->capacity);
             if (s->holds(s->write)) return fail(XNP_E_RING, "ring slot %d still holds a row, evict it first", s->write);
             need += s->blocks[s->write / kBlock] < 0;
             last_pos = s->current_end + (s->ring == RING_ABSOLUTE ? s->shift : 0);
