@@ -37,8 +37,8 @@
 
 --workload mimi: Mimi's windowed attention (2 layers x 8 heads x 64, context 250, bf16): 256 streams,
   each step a 250-row chunk (a 10 s voice clip at 25 Hz) into a window that already holds 249 rows.
-  Value: positions/s over the whole step (the windowed attention and the window append).  Roofline:
-  the windowed attention launch (q, out, the chunk's k and v, the held rows it sees) against 8 TB/s.
+  Value: positions/s over the whole step.  Roofline: the windowed attention launch (q, out, the chunk's
+  k and v, the held rows it sees, the rows that stay written) against 8 TB/s.
 
 --workload vendor_gemm: not this library -- the vendor library's bf16 GEMMs (hipBLASLt through torch)
   at the layer step's four projection shapes and torch's LayerNorm, replayed from a graph, for
@@ -490,7 +490,7 @@ def run_mimi(args, xnp, torch):
     ms, kern, pct = timed_steps(step, args.steps, args.warmup, L, span=False)
     avg_ms = float(kern.mean())
     held = mimi_held(C)
-    hbm = mimi_bytes(S, T, held)
+    hbm = mimi_bytes(S, T, held) + S * min(T, C) * 2 * H * D * 2  # ... and the rows that stay, which the launch writes
     gbs = hbm / (avg_ms * 1e-3) / 1e9
     # every query row sees `context` keys (its own and the context - 1 before it) once the window is full
     flops = 4.0 * D * T * min(C, held + T) * H * S
@@ -503,8 +503,8 @@ def run_mimi(args, xnp, torch):
             "frac": round(gbs / HBM_PEAK_GBS, 4),
             "traffic": traffic_of("mimi", {"streams": S, "chunk": T}, hbm),
             "kernel": "k_prefill_window (RoPE + windowed attention on v_mfma_f32_32x32x16_bf16, the held rows from "
-                      "the pages and the chunk's own from k and v), one launch per layer; the step's k_window_append "
-                      "(the rows that stay into their slots) is in the step time, not here",
+                      "the pages and the chunk's own from k and v; the rows that stay written into their slots), one "
+                      "launch per layer",
             "avg_kernel_us": round(avg_ms * 1000.0, 2), "bytes_per_launch": hbm,
             "mfma": {"achieved": round(tflops, 2), "peak": BF16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / BF16_MFMA_PEAK_TFLOPS, 4), "flops_per_launch": flops}}
