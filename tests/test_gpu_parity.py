@@ -435,6 +435,43 @@ def test_a_few_window_rows_in_one_launch(cache, act, contexts):
         _assert_window_rows(pool, ids[i], orcs[i], contexts[i], L, H, cache)
 
 
+# A step's rows run up to 4 a launch, yet each sees its own window only: a value that is not finite, in
+# position 29's v, reaches the rows at 29 .. 29 + 23 and no other -- neither earlier rows of its own step nor
+# rows after it left the window, bit for bit those of a twin that holds a finite value there.  Steps of 3
+# and 4 rows (with bad_row 29 the last of its step, or not), and longer f32 ones.
+@pytest.mark.parametrize("cache,act,steps", [("bf16", "bf16", (3,) * 20), ("bf16", "bf16", (4,) * 15), ("bf16", "bf16", (2,) * 30),
+                                             ("f32", "f32", (3,) * 20), ("f32", "f32", (6,) * 10)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_rows_a_window_row_does_not_see_stay_out_of_it(cache, act, steps, bad):
+    H, context, at = 8, 24, 29
+    pools = [xnp.KvPool(num_layers=1, num_heads=H, num_blocks=8, max_streams=2, max_blocks_per_stream=4,
+                        cache_dtype=cache, act_dtype=act, max_pos=256, page_seed=4) for _ in range(2)]
+    ids = [[pool.init_window(context)] for pool in pools]
+    rng = np.random.default_rng(58)
+    p = 0
+    for t in steps:
+        q, k, v = (rng.standard_normal((1, t, H, 64)).astype(np.float32) for _ in range(3))
+        outs = []
+        for which, pool in enumerate(pools):
+            if which == 0 and p <= at < p + t:
+                v = v.copy()
+                v[0, at - p, :, 5] = bad
+            elif p <= at < p + t:
+                v[0, at - p, :, 5] = 1.0
+            pool.begin(ids[which], t=t)
+            out = torch.empty((1, t, H, 64), dtype=TORCH_DT[act], device=DEV)
+            pool.attend(0, dev(q, act), dev(k, act), dev(v, act), out, 0.125)
+            torch.cuda.synchronize()
+            pool.end()
+            outs.append(host(out)[0])
+        for i in range(t):
+            if at <= p + i < at + context:
+                assert not np.isfinite(outs[0][i, :, 5]).any(), p + i
+            else:
+                assert np.array_equal(outs[0][i], outs[1][i]), p + i
+        p += t
+
+
 def test_int8_rows_holding_infinities_quantize_as_the_oracle():
     # An int8 page's scale is its rows' amax / 127, taken with IEEE maxima: a row holding an
     # infinity gives the page an infinite scale, its infinite elements code -127 (rint(inf / inf) is

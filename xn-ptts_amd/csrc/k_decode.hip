@@ -287,10 +287,10 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
             // hold what the memory held before): zero them, since 0 * NaN would still be NaN.
             // int8 bytes always convert to finite values (scales start at 0 and are amax / 127),
             // so int8 rows need no zeroing.
-            uint32_t any = seen[0];
-            if constexpr (ROWS) any |= seen[NS - 1]; // held pages: row 0's mask holds the others; new rows: the last's
-            const bool rs = (any >> (g + RPP * p)) & 1u;
-            const uint4 vv = (CDT == DT_I8 || rs) ? vr[p] : make_uint4(0, 0, 0, 0);
+            // ROWS: a row may be one query's and not another's (the step's own rows, and the held ones its
+            // rows take the slots of), so each query's sum skips the rows it does not see.
+            const int r = g + RPP * p;
+            const uint4 vv = (CDT == DT_I8 || ROWS || ((seen[0] >> r) & 1u)) ? vr[p] : make_uint4(0, 0, 0, 0);
             float x[DPL];
             unpack<CDT>(vv, x);
 #pragma unroll
@@ -299,6 +299,7 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
                 l[e] += pe;
                 const float ev = (CDT == DT_I8) ? pe * sv : pe;
                 if constexpr (CDT == DT_I8) vbias[e] += ev;
+                if (ROWS && !((seen[ROWS ? e : 0] >> r) & 1u)) continue;
 #pragma unroll
                 for (int i = 0; i < DPL; ++i) acc[e][i] = __builtin_fmaf(ev, x[i], acc[e][i]);
             }
