@@ -193,7 +193,8 @@ xnp_status xnp_stream_load_kv(xnp_pool *pool, int32_t id, int32_t layer, const f
  * a window cache, and xnp_attend is the only per-layer call such a batch takes.  On a bf16 pool a
  * step of more than 4 rows runs every row's windowed attention in one MFMA launch and writes the
  * last min(t, window) rows into their slots; shorter steps, and f32 pools, run up to 4 rows a launch,
- * int8 pools and grouped heads row by row.  xnp_stream_fork clones a window as it is, every page copied
+ * int8 pools and grouped heads row by row.  The launches of a step depend on the number of streams, t
+ * and the pool alone, so a graph of them replays over other windows, empty or not.  xnp_stream_fork clones a window as it is, every page copied
  * (transformer.rs:348-354). */
 xnp_status xnp_window_open(xnp_pool *pool, int32_t window, int32_t *id);
 

@@ -397,8 +397,8 @@ def test_window_caches_match_mimis_kv_cache(cache, act):
 
 
 # A bf16 window step of more than 4 rows writes its rows from the attention's own launch: over fresh windows
-# (every 256-row round a work group), over held rows when the window has 192 and more rows and no heads
-# share a kv head; otherwise an append runs after.  Windows of 40, 191, 192 and 250 rows: a fresh chunk
+# (every 256-row round a work group) and over held rows (as the rows pass where the window has 192 and more,
+# else at the end); where heads share a kv head an append runs after.  Windows of 40, 191, 192 and 250 rows: a fresh chunk
 # shorter than the window or of several rounds, chunks over held rows shorter and longer than the window
 # and than a round, single and few rows between, every held row bit for bit after each.
 @pytest.mark.parametrize("context", [40, 191, 192, 250])
@@ -416,8 +416,8 @@ def test_window_chunks_write_their_rows(context, steps):
             _assert_window_rows(pool, ids[i], orcs[i], context, L, H, "bf16")
 
 
-# Steps of a few rows attend them in one launch (up to 4, and no more than the smallest window holds;
-# f32 runs longer steps 4 rows a launch): windows of 1 row, less than a page, a page, a ragged two and
+# Steps of a few rows attend them in one launch (up to 4, more than the smallest windows hold; f32 runs longer
+# steps 4 rows a launch): windows of 1 row, less than a page, a page, a ragged two and
 # a half and seven pages, empty, filling and full, more than 1024 groups (one wave each) and few
 # (eight waves), against the oracle's KvCache.
 @pytest.mark.parametrize("cache,act", [("bf16", "bf16"), ("f32", "f32")])
@@ -470,6 +470,49 @@ def test_rows_a_window_row_does_not_see_stay_out_of_it(cache, act, steps, bad):
             else:
                 assert np.array_equal(outs[0][i], outs[1][i]), p + i
         p += t
+
+
+# The launches of a window step captured once and replayed over other windows than they were recorded on: empty
+# ones when recorded, then the same ones holding rows, then others, larger and smaller, against a twin pool
+# that runs every step eagerly -- outputs and rows bit for bit.  Chunks of two rounds and of less than one,
+# with and without shared kv heads, and steps of a few rows (f32: 4 and 2 a step of 6).
+@pytest.mark.parametrize("cache,act,h,kvh,t", [("bf16", "bf16", 2, 2, 300), ("bf16", "bf16", 4, 2, 300), ("bf16", "bf16", 2, 2, 30),
+                                               ("bf16", "bf16", 2, 2, 4), ("bf16", "bf16", 4, 2, 3), ("f32", "f32", 2, 2, 6)])
+@pytest.mark.parametrize("recorded,others", [((250, 250), (40, 191)), ((24, 40), (1, 3)), ((3, 16), (250, 192))])
+def test_window_steps_captured_in_a_hip_graph_replay_over_other_windows(cache, act, h, kvh, t, recorded, others):
+    pools = [xnp.KvPool(num_layers=1, num_heads=h, num_kv_heads=kvh, num_blocks=72, max_streams=4, max_blocks_per_stream=16,
+                        cache_dtype=cache, act_dtype=act, max_pos=4096, page_seed=9) for _ in range(2)]
+    sets = [[[pool.init_window(c) for c in cs] for cs in (recorded, others)] for pool in pools]
+    rng = np.random.default_rng(60 + t)
+    q, k, v = (torch.empty((2, t, n, 64), dtype=TORCH_DT[act], device=DEV) for n in (h, kvh, kvh))
+    outs = [torch.empty_like(q) for _ in range(2)]
+    g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    for step, which in enumerate((0, 0, 1, 1, 0, 1)):
+        for x in (q, k, v):
+            x.copy_(dev(rng.standard_normal(tuple(x.shape)).astype(np.float32), act))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            for p, pool in enumerate(pools):
+                pool.begin(sets[p][which], t=t, stream=s.cuda_stream)
+                if p == 0:
+                    pool.attend(0, q, k, v, outs[0], 0.125)
+                elif step == 0:
+                    with torch.cuda.graph(g, stream=s):
+                        pool.attend(0, q, k, v, outs[1], 0.125)
+                    g.replay()
+                else:
+                    g.replay()
+                pool.end()
+        s.synchronize()
+        assert torch.equal(outs[0], outs[1]), step
+        for i, c in enumerate((recorded, others)[which]):
+            n = pools[0].current_end(sets[0][which][i])
+            for kv in (0, 1):
+                rows = [torch.empty((n, kvh, 64), dtype=CACHE_TORCH[cache], device=DEV) for _ in range(2)]
+                for p, pool in enumerate(pools):
+                    pool.read_rows(sets[p][which][i], 0, kv, 0, rows[p])
+                torch.cuda.synchronize()
+                assert torch.equal(rows[0], rows[1]), (step, c, kv)
 
 
 def test_int8_rows_holding_infinities_quantize_as_the_oracle():

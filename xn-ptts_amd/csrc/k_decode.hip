@@ -29,7 +29,8 @@ namespace xnp {
 // sees position p = r0's position + e and the window - 1 before it: the held pages less the slots
 // its rows 0 .. e take (which hold the positions that left its window), then the new rows 0 .. e,
 // which go through the loop's arithmetic as one more page built from the inputs.  The rows are
-// appended once every wave has read the pages.
+// appended once every wave has read the pages; of rows that share a slot (a window of fewer rows than
+// the launch takes) the last.
 template <int CDT, bool ABF, int SPLIT, bool PREFIX, int GQ = 1, bool ROWS = false>
 __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView &bv, int layer, const StreamRec &R,
                                             const int32_t *rec_pages, int h, const void *q, const void *knew,
@@ -45,9 +46,13 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
     const int nb = R.nblk > w ? (R.nblk - w + SPLIT - 1) / SPLIT : 0; // this wave's pages
     const int kvh = h / (pv.H / pv.KVH);                               // the tiles the heads read
 
-    // ROWS: the slot of row e (distinct: a launch takes no more rows than the window holds)
+    // ROWS: the slot of row e
     const int slot0 = ROWS ? R.pos % R.window : 0;
-    auto row_slot = [&](int e) { return slot0 + e >= R.window ? slot0 + e - R.window : slot0 + e; };
+    auto row_slot = [&](int e) {
+        int s = slot0 + e;
+        while (s >= R.window) s -= R.window;
+        return s;
+    };
 
     // Per-page metadata, lane j holding page w + j * SPLIT: page id, seen rows, int8 scales.
     // Past the wave's last page the lanes hold page 0 with no row seen.
@@ -368,7 +373,10 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
                 }
             }
 #pragma unroll
-            for (int e = 0; e < NS; ++e) seen[e] = (2u << min(e, bv.wrows - 1)) - 1u;
+            for (int e = 0; e < NS; ++e) { // rows max(0, er - window + 1) .. er
+                const int er = min(e, bv.wrows - 1);
+                seen[e] = (2u << er) - (1u << max(0, er - R.window + 1));
+            }
             process(kr, vr, 0, seen);
         }
     }
@@ -415,7 +423,7 @@ __device__ __forceinline__ void attend_core(const PoolView &pv, const BatchView 
 #pragma unroll
             for (int e = 0; e < GQ; ++e) {
                 const int sl = row_slot(e);
-                const int pg = e < bv.wrows ? rec_pages[sl >> 4] : -1;
+                const int pg = e < bv.wrows && e + R.window >= bv.wrows ? rec_pages[sl >> 4] : -1;
                 const size_t arow = ((size_t)(R.b + e) * pv.KVH + kvh) * kHeadDim * AE;
                 if (pg >= 0 && pg < pv.NB)
                     append_row_wave<CDT, ABF>(pv, layer, pg, sl & 15, kvh, R.pos + e, (const char *)knew + arow,

@@ -720,9 +720,19 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
 // virtually: the window's held rows first (j < ncache, oldest first, at slot (wbase + j) mod W),
 // then the chunk's rows (j = ncache + i: input row i, rotated at its position and rounded to bf16).
 // Query row i has virtual index ncache + i and sees key j when ncache + i - W < j <= ncache + i.
-// The rows that stay are written by the group of the last round as they pass through its LDS, where that
-// cannot race with a read (window_append_fused); k_window_append read and wrote them again in 30 us of the
-// 139 a layer took.  Fresh windows take a group per round.  160 clips of 375 rows, 2 layers: 282 -> 226 us.
+//
+// The rows that stay are written here too, where no other group reads the slots they take (k_window_append
+// read and wrote them again in 30 us of the 139 a layer took).  A row takes the slot of the position W before
+// it, which may be held and read by this launch:
+//   - a fresh window (no held rows): nothing reads the pages, so every round is a group of its own, and the
+//     last one's writes the rows as they pass through its LDS.  160 clips of 375 rows, 2 layers: 282 -> 226 us;
+//   - held rows, one query head per kv head: one group runs every round in turn (the other rounds' groups
+//     end at once) and writes the rows as they pass in the last.  The slot's old key lies W keys before the
+//     row: with W >= kWpPassRows at least two chunks earlier, so every wave's load of it has landed, the
+//     barrier of the chunk before the row's being past.  Smaller windows write them after the last round;
+//   - held rows, query heads that share a kv head: k_window_append writes them after this launch.
+// Each group takes this from its stream's plan, not from the launch, which depends on the batch's streams, its
+// rows and the heads alone: a launch recorded in a graph serves any windows it is replayed over.
 //
 // Query rows are taken in rounds of 256: 8 pairs of 16-row tiles, pair i rows 32 i .. 32 i + 31 of
 // the round, wave w owning pair w.  A round's keys (from the window of its first row to
@@ -755,6 +765,7 @@ constexpr int kWpSlots = 3;   // chunk slots of the LDS ring: 2 chunks load whil
 constexpr int kWpWaves = 8;   // waves per work group
 constexpr int kWpPairs = 1;   // tile pairs per wave
 constexpr int kWpRound = 256; // query rows per round: 8 waves x 1 pair x 32 rows
+constexpr int kWpPassRows = 3 * kWpChunk; // windows from which held rows' slots are taken while the rounds run
 // A chunk is 24 direct loads of 1 KB (8 keys each), 3 a wave: one each of K, V and K's rope pieces.
 constexpr int kWpLoadsC = kWpChunk / 8 / kWpWaves; // loads of K (of V, of rope pieces) per wave per chunk
 constexpr int kWpKeysW = kWpChunk / kWpWaves;      // keys of a chunk each wave loads
@@ -789,17 +800,18 @@ __device__ __forceinline__ void wait_chunks(int ahead) {
 }
 
 __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_prefill_window(
-    PoolView pv, BatchView bv, int layer, const void *q, const void *knew, const void *vnew, void *out, float qmul,
-    int append) {
+    PoolView pv, BatchView bv, int layer, const void *q, const void *knew, const void *vnew, void *out, float qmul) {
     __shared__ __attribute__((aligned(16))) uint16_t ks[kWpSlots][kWpChunk][kHeadDim]; // K, [key][unit ^ swz]
     __shared__ __attribute__((aligned(16))) uint16_t vs[kWpSlots][kWpChunk][kHeadDim]; // V, [key][unit ^ swz]
     __shared__ __attribute__((aligned(16))) uint4 rs[kWpSlots][kWpWaves][kWpLoadsC][64]; // the lanes' rope pieces
     __shared__ int32_t spages[kPfMaxPages];
     const int t = bv.t;
-    // one group for every round of a (stream, head), or (a grid of several rounds, the last first) one each
-    const int per = bv.n * pv.H, rounds = (int)gridDim.x / per, round = rounds - 1 - (int)blockIdx.x / per;
+    // a group for every (stream, head, round), the last round first
+    const int per = bv.n * pv.H, back = (int)blockIdx.x / per; // rounds after this one
     const int h = (int)blockIdx.x % per % pv.H, b = (int)blockIdx.x % per / pv.H;
     const StreamPlan P = bv.plans[b];
+    const bool held = P.pos_pre > 0, alone = pv.H == pv.KVH;
+    if (held && back > 0) return; // the last round's group runs them all
     const int32_t *tab = pv.tables + (size_t)P.sid * pv.mbps;
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, hi = lane >> 5, col = lane & 31;
     const int W = P.window;
@@ -853,11 +865,10 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
             dma16(pv.rope16 + (size_t)(P.key_pos + r) * (kHeadDim / 2) + 4 * unit, &rs[slot][w][i][0]);
         }
     };
-    // the rows that stay (KvCache::trim): the step's last min(t, W), the first of them in slot s0; with
-    // `append` the group of the last round writes them as they pass through its LDS, whole rows of 128
-    // bytes, from the lanes that hold them (one query head per kv head writes)
+    // the rows that stay (KvCache::trim): the step's last min(t, W), the first of them in slot s0; written as
+    // they pass in whole rows of 128 bytes, from the lanes that hold them (one query head per kv head writes)
     const int keep = min(t, W), s0 = (P.pos + t - keep) % W;
-    const bool writes = append && h % (pv.H / pv.KVH) == 0;
+    const bool writes = held ? alone && W >= kWpPassRows : h % (pv.H / pv.KVH) == 0;
     // ...then, once they have landed, the step's own keys rotated in place by the lane that loaded
     // them
     auto settle = [&](int j0, int khi, int slot, bool last) {
@@ -882,8 +893,9 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
             }
         }
     };
-    const int nqt = (t + 15) / 16, tq_first = rounds > 1 ? round * (kWpRound / 16) : 0;
-    const int tq_end = rounds > 1 ? min(nqt, tq_first + kWpRound / 16) : nqt;
+    const int nqt = (t + 15) / 16, rounds = (int)gridDim.x / per;
+    const int tq_first = held ? 0 : (rounds - 1 - back) * (kWpRound / 16);
+    const int tq_end = held ? nqt : min(nqt, tq_first + kWpRound / 16);
     for (int tq0 = tq_first; tq0 < tq_end; tq0 += kWpRound / 16) {
         const int nq = min(kWpRound / 16, nqt - tq0);
         // the round's keys: from the window of its first row to its last row
@@ -1079,6 +1091,22 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
             if (act[p] && qrow < t)
                 st_stream((uint16_t *)out + (((size_t)P.out_row * t + qrow) * pv.H + h) * kHeadDim + 8 * unit,
                           *(const uint4 *)(stage + row * kHeadDim + 8 * (unit ^ (row & 7))));
+        }
+    }
+    // Smaller held windows' rows, every wave's loads of the pages having landed before the last barrier.  The
+    // plan is read again, so that nothing of this is kept through the rounds.
+    const StreamPlan &L = bv.plans[b];
+    if (L.pos_pre > 0 && L.window < kWpPassRows && pv.H == pv.KVH) {
+        const int Wl = L.window, n = min(t, Wl), first = (L.pos + t - n) % Wl;
+        for (int e = tid; e < 8 * n; e += 64 * kWpWaves) {
+            const int r = e >> 3, unit = e & 7, i = t - n + r, s = first + r >= Wl ? first + r - Wl : first + r;
+            const int pg = spages[s >> 4];
+            if (pg < 0 || pg >= pv.NB) continue;
+            const size_t arow = (((size_t)L.out_row * t + i) * pv.KVH + h) * kHeadDim + 8 * unit;
+            const size_t poff = (size_t)pg * page_elems + (s & 15) * kHeadDim + 8 * unit;
+            const uint4 cs = *(const uint4 *)(pv.rope16 + (size_t)(L.key_pos + i) * (kHeadDim / 2) + 4 * unit);
+            st_stream(kpages + poff, rotate8(*(const uint4 *)((const uint16_t *)knew + arow), cs));
+            st_stream(vpages + poff, *(const uint4 *)((const uint16_t *)vnew + arow));
         }
     }
 }
@@ -1435,15 +1463,8 @@ hipError_t launch_decode_gqa(const PoolView &pv, const BatchView &bv, int layer,
 static int prefill_rounds(int t) { return (t + kPfRound - 1) / kPfRound; }
 static_assert(kPfRound == kWpRound, "prefill_rounds counts both kernels' rounds");
 
-// The window's rows written by the attention itself.  A row that stays takes the slot of the position W
-// before it, which may be held and read by the same launch.  Without held rows nothing reads the pages
-// (and the rounds may be groups of their own).  With them, a (stream, head) must be one group (no query
-// head shares its kv head), which loads that position's key W keys before the row: with 192 and more,
-// at least two chunks earlier, so every wave's load of it has landed, the barrier of the chunk before
-// the row's being past.  Otherwise k_window_append runs after.
-bool window_append_fused(const PoolView &pv, const BatchView &bv) {
-    return bv.wheld == 0 || (pv.H == pv.KVH && bv.wmin >= 192);
-}
+// k_prefill_window leaves held windows' rows to k_window_append where query heads share a kv head.
+bool window_append_apart(const PoolView &pv) { return pv.H != pv.KVH; }
 
 hipError_t launch_prefill_mfma(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
                                const void *v, void *out, float scale, bool fused, bool window, hipStream_t stream,
@@ -1451,8 +1472,8 @@ hipError_t launch_prefill_mfma(const PoolView &pv, const BatchView &bv, int laye
     if ((fused || window) && (!k || !v)) return hipErrorInvalidValue; // the step's own rows are read from k, v
     const float qmul = scale * 1.4426950408889634f;
     if (window)
-        XNP_LAUNCH(k_prefill_window, dim3(bv.n * pv.H * (bv.wheld == 0 ? prefill_rounds(bv.t) : 1)), dim3(64 * kWpWaves), stream, tm,
-                   pv, bv, layer, q, k, v, out, qmul, window_append_fused(pv, bv) ? 1 : 0);
+        XNP_LAUNCH(k_prefill_window, dim3(bv.n * pv.H * prefill_rounds(bv.t)), dim3(64 * kWpWaves), stream, tm, pv, bv, layer,
+                   q, k, v, out, qmul);
     else if (bv.kmax <= kPfFastKeys && fused)
         XNP_LAUNCH(k_prefill_fast<true>, dim3(bv.n * pv.H), dim3(64 * kPfWaves), stream, tm, pv, bv, layer, q, k, v,
                    out, qmul);

@@ -236,8 +236,8 @@ hipError_t launch_append(const PoolView &pv, const BatchView &bv, int layer, con
 }
 
 // ---------------------------------------------------------------------------------------------
-// A window step's rows into the window after its attention (Mimi's chunk, bf16 and f32 pools):
-// slot s takes the step's last row i with (p + i) % window == s; a row that a later row of the
+// A window step's rows into the held windows after its attention (Mimi's chunk where query heads share a kv
+// head, bf16 and f32 pools): slot s takes the step's last row i with (p + i) % window == s; a row that a later row of the
 // step overwrites is never written.  One work group per (stream, page of the window), one wave per
 // kv head for the page's 16 slots.
 //   bf16: lane l takes 16-byte unit l % 8 of the K and V rows of slots l / 8 and l / 8 + 8, and
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(1024) void k_window_append(PoolView pv, BatchView b
     const int b = blockIdx.x / pv.mbps, blk = blockIdx.x % pv.mbps;
     const StreamPlan P = bv.plans[b];
     const int W = P.window, t = bv.t, j = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (W <= 0 || kBlock * blk >= W) return;
+    if (W <= 0 || kBlock * blk >= W || P.pos_pre == 0) return; // (a fresh window's: written by k_prefill_window)
     const int page = pv.tables[(size_t)P.sid * pv.mbps + blk];
     if (page < 0 || page >= pv.NB) return; // begin took this page; never index the pool without one
     const int rb = ((kBlock * blk - P.pos) % W + W) % W; // the first row of the step in the page's slot 0

@@ -94,8 +94,8 @@ struct Stream {
     int32_t window = 0;
 };
 
-// Window steps of more rows than this on a bf16 pool run as one windowed prefill on MFMA plus an
-// append; shorter ones (Mimi's decoder takes 2 a frame), and every window step on f32 and int8 pools,
+// Window steps of more rows than this on a bf16 pool run as one windowed prefill on MFMA, which writes the
+// rows too (an append after it where query heads share a kv head); shorter ones (Mimi's decoder takes 2 a frame), and every window step on f32 and int8 pools,
 // run a few rows a launch (window_rows_max) through the decode's core.
 constexpr int32_t kWindowRowByRow = 4;
 
@@ -1335,14 +1335,6 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
     B.bv.masks = (const uint32_t *)(pool->dbatch + o_masks);
     B.bv.wrow = -1;
     B.bv.wrows = 0;
-    B.bv.wheld = B.bv.wmin = 0;
-    if (wsteps) {
-        B.bv.wmin = pool->streams[ids[0]].window;
-        for (int32_t i = 0; i < n; i++) {
-            B.bv.wmin = std::min(B.bv.wmin, pool->streams[ids[i]].window);
-            B.bv.wheld = std::max(B.bv.wheld, pool->streams[ids[i]].current_end);
-        }
-    }
     B.bv.n = n;
     B.bv.t = t;
     B.wsteps = wsteps;
@@ -1413,14 +1405,15 @@ extern "C" xnp_status xnp_attend(xnp_pool *pool, int32_t layer, const void *q, c
         pool->timing = LaunchTiming();
         if (pool->d.cache_dtype == XNP_BF16 && B.t > kWindowRowByRow) {
             // every row's windowed attention in one MFMA launch (the held rows from the pages, the
-            // step's own from k and v), then the rows that stay into their slots
+            // step's own from k and v) and the rows that stay into their slots, by the launch itself or
+            // after it
             HIP_TRY(launch_window_prefill(pool->view(), B.bv, layer, q, k, v, out, scale, B.stream, tm), "window attend");
-            if (!window_append_fused(pool->view(), B.bv))
+            if (window_append_apart(pool->view()))
                 HIP_TRY(launch_window_append(pool->view(), B.bv, layer, k, v, B.stream), "window append");
             return XNP_OK;
         }
         BatchView bv = B.bv;
-        const int32_t most = std::min(window_rows_max(pool->view()), bv.wmin); // the rows' slots distinct
+        const int32_t most = window_rows_max(pool->view());
         for (int32_t r = 0; r < B.t; r += bv.wrows) {
             bv.wrow = r; // the kernel derives the rows' record from the step's
             bv.wrows = std::min(most, B.t - r);

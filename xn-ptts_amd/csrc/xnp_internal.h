@@ -69,7 +69,6 @@ struct BatchView {
     int32_t prefix; // 1 if some stream of the batch is an absolute ring keeping a prefix
     int32_t wrow;   // a window step run a few rows a launch: the first row this launch attends (-1 otherwise)
     int32_t wrows;  // ... and how many it attends
-    int32_t wheld, wmin; // a window step of several rows: the most rows a window holds, the smallest window
     int32_t kmax;   // a prompt step (t > 1): the most key slots a stream of it attends, write_slot + t
 };
 
@@ -156,11 +155,11 @@ hipError_t launch_prefill(const PoolView &pv, const BatchView &bv, int layer, co
 hipError_t launch_window_prefill(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
                                  const void *v, void *out, float scale, hipStream_t stream, const LaunchTiming &timing);
 // Rows bv.wrow .. bv.wrow + bv.wrows - 1 of a window step, attended and appended in one launch; at most
-// window_rows_max of them (1 on int8 pools and grouped heads: row by row).
+// window_rows_max of them (1 on int8 pools and grouped heads: row by row), more than a window holds or not.
 int window_rows_max(const PoolView &pv);
 hipError_t launch_window_rows(const PoolView &pv, const BatchView &bv, int layer, const void *q, const void *k,
                               const void *v, void *out, float scale, hipStream_t stream, const LaunchTiming &timing);
-bool window_append_fused(const PoolView &pv, const BatchView &bv); // launch_window_prefill writes the rows itself
+bool window_append_apart(const PoolView &pv); // launch_window_append follows launch_window_prefill
 hipError_t launch_window_append(const PoolView &pv, const BatchView &bv, int layer, const void *k, const void *v,
                                 hipStream_t stream);
 hipError_t launch_evict_rotate(const PoolView &pv, const EvictRow *rows, int n,
