@@ -175,6 +175,26 @@ def test_abort_gives_back_the_pages_and_keeps_the_state():
     assert e.value.name == "XNP_E_STATE"
 
 
+def test_id_and_step_lists_reach_the_library_whole():
+    # lists converted in one go arrive as ctypes would pass them one by one: fewer steps than streams leave
+    # the others at step 0 (and the library reads no further), more are refused, bytes are numbers of their
+    # own, as are arrays and generators
+    p = pool()
+    ids = [p.init_state(48) for _ in range(3)]
+    for s in ids:
+        p.start_ring(s, "absolute")
+    before = p.slide_batch(ids, 0, 48, 32, 1, [5, 7])
+    assert before is None and [p.info(s)["ring_write"] for s in ids] == [5, 7, 0]
+    with pytest.raises((IndexError, ValueError)):
+        p.slide_batch(ids, 0, 48, 32, 1, [5, 7, 9, 11])
+    for steps in (bytes([1, 2, 3]), np.array([1, 2, 3]), (x for x in (1.0, 2, 3))):
+        p.slide_batch(ids, 0, 48, 32, 1, steps)
+        assert [p.info(s)["ring_write"] for s in ids] == [1, 2, 3]
+    conv = xnp.kv._int_array
+    assert list(conv(bytes([1, 2, 3, 4]), 4, "i", ctypes.c_int32)) == [1, 2, 3, 4]
+    assert list(conv([1 << 32, -1], 2, "i", ctypes.c_int32)) == [0, -1] and list(conv([], 0, "i", ctypes.c_int32)) == [0]
+
+
 def test_kernel_calls_on_a_host_only_pool_are_refused():
     p = pool()
     a = p.init_state(16)

@@ -179,7 +179,7 @@ class FlowLM:
         latent_out [n][ldim], eos_out [n], conditions [n][d_model] (each stream's
         FlowLMState::conditions; None: the model's, if set) -- f32 device tensors.  graph: replay a
         recording of the frame's launches (xnp_flow_lm_step_graph; needs a non-null stream)."""
-        _, arr = _int_array(ids, "i", ctypes.c_int32)
+        arr = _int_array(ids, len(ids), "i", ctypes.c_int32)
         fn = self._lib.xnp_flow_lm_step_graph if graph else self._lib.xnp_flow_lm_step
         _check(fn(self._h, arr, len(ids), _ptr(latent_in), _ptr(conditions), _ptr(noise), _ptr(latent_out),
                   _ptr(eos_out), _stream(stream)))

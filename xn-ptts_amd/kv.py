@@ -217,19 +217,18 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
-def _int_array(values, code: str, ctype):
-    """values (whole numbers, a sequence or an array) as a C array for one call: the array object to
-    keep alive, and what ctypes passes.  array.array converts a list several times as fast as ctypes
-    does; what it refuses (a number out of range, an empty list's address) goes the ctypes way."""
+def _int_array(values, n: int, code: str, ctype):
+    """n whole numbers as a C array for one call.  array.array converts a list several times as fast as
+    ctypes does; what it refuses (a number out of range, an empty list's address) and values of another
+    count go the ctypes way: too few leave zeros, too many are refused."""
+    values = list(values)  # bytes too as numbers, one each
     try:
         a = array.array(code, values)
-        if len(a):
-            return a, (ctype * len(a)).from_buffer(a)
+        if n and len(a) == n:
+            return (ctype * n).from_buffer(a)  # keeps a alive
     except (OverflowError, TypeError):
-        values = [int(x) for x in values] if code == "q" else values
-        a = values
-    c = (ctype * max(len(a), 1))(*a)
-    return c, c
+        pass
+    return (ctype * max(n, 1))(*([int(x) for x in values] if code == "q" else values))
 
 
 def _stream(stream) -> Optional[int]:
@@ -402,9 +401,8 @@ class KvPool:
         """slide() over many streams, stream i at steps[i], in one call."""
         ids = list(ids)
         n = len(ids)
-        _, arr = _int_array(ids, "i", _i32)
-        steps = steps.tolist() if hasattr(steps, "tolist") else list(steps)
-        _, st = _int_array(steps, "q", ctypes.c_int64)
+        arr = _int_array(ids, n, "i", _i32)
+        st = _int_array(steps.tolist() if hasattr(steps, "tolist") else steps, n, "q", ctypes.c_int64)
         failed = _i32(-1)
         _check(self._lib.xnp_ring_slide_batch(self._h, arr, n, prefix, span, window, drop, st,
                                               ctypes.byref(failed), _stream(stream)))
@@ -412,7 +410,7 @@ class KvPool:
     # -- a batched step -----------------------------------------------------------------------
     def begin(self, ids: Iterable[int], t: int = 1, stream=None):
         ids = list(ids)
-        _, arr = _int_array(ids, "i", _i32)
+        arr = _int_array(ids, len(ids), "i", _i32)
         self._stream_h = _stream(stream)
         _check(self._lib.xnp_batch_begin(self._h, arr, len(ids), t, self._stream_h))
 
