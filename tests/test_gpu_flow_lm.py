@@ -136,6 +136,31 @@ def test_bad_tokens_are_refused_and_change_nothing():
     assert pool.current_end(sid) == 0
 
 
+def test_a_prompt_under_capture_is_refused_and_changes_nothing():
+    # a prompt's tokens are staged in host memory, which a recorded upload would read again at each replay: the
+    # call is refused on a capturing stream, the capture goes on, and the prompt runs eagerly after it
+    cfg = fl.FlowLMConfig(num_layers=1, flow_depth=1, flow_dim=256, dim_feedforward=512, n_bins=10)
+    blob = fl.random_weights(cfg, 92)
+    pool = xnp.KvPool(num_layers=1, num_heads=8, num_blocks=8, max_streams=1, max_blocks_per_stream=4,
+                      cache_dtype="f32", act_dtype="f32")
+    sid = pool.init_state(64)
+    lm = xnp.FlowLM(pool, cfg, blob, max_rows=8)
+    tokens = np.array([[1, 2, 9]], np.int32)
+    s, g, x = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.zeros(4, device=DEV)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        with pytest.raises(xnp.XnpError):
+            lm.prompt_text([sid], tokens, stream=s.cuda_stream)
+        x += 1
+    assert pool.current_end(sid) == 0
+    g.replay()
+    for n in (3, 6):
+        lm.prompt_text([sid], tokens, stream=s.cuda_stream)
+        assert pool.current_end(sid) == n
+    torch.cuda.synchronize()
+    assert (x == 1).all()
+
+
 def test_graph_recorded_frames_equal_eager_frames():
     # StepGraph's analog (step_graph.rs:111-307): the frame's launches recorded once and replayed
     # after each eager plan upload, against a twin model stepping eagerly -- bit for bit, every

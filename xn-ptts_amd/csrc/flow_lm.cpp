@@ -434,6 +434,11 @@ extern "C" xnp_status xnp_flow_lm_prompt_text(xnp_flow_lm *lm, const int32_t *id
                              lm->d.n_bins + 1);
     hipStream_t hs = (hipStream_t)hip_stream;
     FL_TRY(hipSetDevice(pool_desc(lm->pool)->device), "hipSetDevice");
+    // the tokens go through one host buffer: a recorded upload would replay whatever it holds by then, and
+    // the event of the wait below cannot be waited for once a capture took it
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    FL_TRY(hipStreamIsCapturing(hs, &cap), "staging");
+    if (cap != hipStreamCaptureStatusNone) return pool_fail(XNP_E_HIP, "a text prompt cannot be captured: its tokens are staged by the host");
     // wait for the previous call's upload from the staging buffer alone, not for the stream's work
     if (lm->ids_pending) FL_TRY(hipEventSynchronize(lm->ids_read), "staging");
     lm->ids_pending = false;
