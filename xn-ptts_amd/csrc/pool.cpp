@@ -1229,12 +1229,21 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
     // decode order: longest streams first, so the short ones fill the tail of the launch
     std::vector<int32_t> order(n);
     for (int32_t i = 0; i < n; i++) order[i] = i;
-    if (t == 1) { // by counting the spans, equal ones in the batch's order
-        std::vector<int32_t> at(pool->d.max_blocks_per_stream * kBlock + 2, 0);
-        for (int32_t i = 0; i < n; i++) at[plans[i].span]++;
-        int32_t before = 0;
-        for (size_t sp = at.size(); sp-- > 0;) before += std::exchange(at[sp], before);
-        for (int32_t i = 0; i < n; i++) order[at[plans[i].span]++] = i;
+    if (t == 1 && n > 1) { // equal ones in the batch's order
+        int32_t lo = plans[0].span, hi = lo;
+        for (const StreamPlan &P : plans) lo = std::min(lo, P.span), hi = std::max(hi, P.span);
+        // by counting the spans, unless they spread far beside the batch: a count takes 0.5 ns a slot, a
+        // sort 43 and 68 ns a stream of 512 and 2048 (less of few).  Counted over every slot of a 7680-slot
+        // pool, a single stream's begin took 8.4 us instead of 4.4
+        if (hi - lo <= 16 * n) {
+            std::vector<int32_t> at(hi - lo + 1, 0);
+            for (int32_t i = 0; i < n; i++) at[plans[i].span - lo]++;
+            int32_t before = 0;
+            for (size_t sp = at.size(); sp-- > 0;) before += std::exchange(at[sp], before);
+            for (int32_t i = 0; i < n; i++) order[at[plans[i].span - lo]++] = i;
+        } else {
+            std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return plans[a].span > plans[b].span; });
+        }
     }
     // waves per decode work group, unless the caller fixed them: the pool's default (the fewest
     // whose lanes index a stream's pages), at least two on MFMA; and a batch of few groups fills

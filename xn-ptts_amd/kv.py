@@ -221,7 +221,7 @@ def _int_array(values, n: int, code: str, ctype):
     """n whole numbers as a C array for one call.  array.array converts a list several times as fast as
     ctypes does; what it refuses (a number out of range, an empty list's address) and values of another
     count go the ctypes way: too few leave zeros, too many are refused."""
-    values = list(values)  # bytes too as numbers, one each
+    values = values if isinstance(values, list) else list(values)  # bytes too as numbers, one each
     try:
         a = array.array(code, values)
         if n and len(a) == n:
