@@ -111,6 +111,51 @@ def test_f32_prompts_on_row_tiles_match_the_oracle(n, t, ff, dm):
                 assert rel_err(rows.cpu().numpy(), vals) <= 1e-5, (i, layer, kv)
 
 
+# Frames of 16 f32 streams and more take the row tiles too, in every form a frame has: the modulated norm,
+# gated, SiLU, axpy and plain epilogues, with and without z_proj and conditions, over K of 256 to 2048 (norms
+# above 512 with their operands loaded as used, two row tiles with the modulated norm from 256 streams).
+# Streams at the tiles' edges against the oracle, each frame from the oracle's latent: fed back, the oracle's
+# own sums stand 1.3e-5 from 64 bits after five drifting frames of the first of these models (the GPU's 3e-6).
+@pytest.mark.parametrize("n,flow_type,z_dim,steps,dm,fd,ff,gelu,cond", [
+    (16, "lsd", 0, 1, 512, 256, 1024, "erf", False), (17, "lsd", 256, 2, 256, 512, 512, "tanh", True),
+    (33, "drifting", 0, 1, 512, 256, 1500, "erf", False), (33, "pointwise", 128, 1, 256, 256, 1024, "tanh", False),
+    (16, "lsd", 0, 1, 1024, 1024, 2048, "erf", False), (17, "drifting", 0, 1, 2048, 2048, 512, "erf", False),
+    (257, "lsd", 0, 1, 1024, 1024, 512, "erf", False)])
+def test_f32_frames_of_many_streams_match_the_oracle(n, flow_type, z_dim, steps, dm, fd, ff, gelu, cond):
+    attn = min(dm, 1024)
+    cfg = fl.FlowLMConfig(d_model=dm, num_heads=attn // 64, attn_dim=attn, num_layers=1 if dm > 512 else 2, flow_depth=1,
+                          flow_dim=fd, dim_feedforward=ff, n_bins=100, flow_type=flow_type, z_dim=z_dim,
+                          lsd_decode_steps=steps, gelu=gelu)
+    blob = fl.random_weights(cfg, 96 + n, std=0.05 if dm <= 512 else 0.03, unit_norms=False)
+    rng = np.random.default_rng(97 + n)
+    frames, t = 3, 3
+    tokens = rng.integers(0, cfg.n_bins + 1, (n, t)).astype(np.int32)
+    noise = (0.5 * rng.standard_normal((frames, n, cfg.ldim))).astype(np.float32)
+    conds = (0.1 * rng.standard_normal((n, dm))).astype(np.float32) if cond else None
+    pool = xnp.KvPool(num_layers=cfg.num_layers, num_heads=cfg.num_heads, num_blocks=n + 8, max_streams=n,
+                      max_blocks_per_stream=1, cache_dtype="f32", act_dtype="f32", max_pos=32, page_seed=3)
+    ids = [pool.init_state(16) for _ in range(n)]
+    lm = xnp.FlowLM(pool, cfg, blob, max_rows=n * t)
+    orc = oracle.FlowLM(cfg, blob)
+    some = sorted({0, 1, 15, n - 2, n - 1} | ({16, 31, 32} & set(range(n))))
+    sts = {i: orc.stream(16) for i in some}
+    lm.prompt_text(ids, tokens)
+    for i in some:
+        orc.prompt_text(sts[i], tokens[i])
+    lat = torch.empty((n, cfg.ldim), dtype=torch.float32, device=DEV)
+    eos = torch.empty(n, dtype=torch.float32, device=DEV)
+    cdev = None if conds is None else torch.from_numpy(conds).to(DEV)
+    want = {i: None for i in some}
+    for f in range(frames):
+        lm.step(ids, None if f == 0 else lat, torch.from_numpy(noise[f]).to(DEV), lat, eos, conditions=cdev)
+        torch.cuda.synchronize()
+        got, ge = lat.cpu().numpy(), eos.cpu().numpy()
+        for i in some:
+            want[i], we = orc.step(sts[i], want[i], noise[f, i], cond=None if conds is None else conds[i])
+            assert rel_err(got[i], want[i]) <= 1e-5 and abs(ge[i] - we) <= 1e-5 * max(1.0, abs(we)), (f, i)
+            lat[i] = torch.from_numpy(want[i])
+
+
 def test_phonon_31m_shape_64_tokens_then_200_frames_at_temperature_0():
     # the single-stream configuration: 6 layers x 512, 8 heads, FF 2048, ldim 32, 4001-row LUT,
     # flow net 512 x 6, 1 LSD step; N(0, 0.02) linears, unit norms; 64 tokens, 200 greedy frames
