@@ -1097,6 +1097,18 @@ hipError_t launch_gemm_q8(const void *A, int M, int K, const int8_t *W, const fl
 // that the norm's operands load together with x instead of behind a branch after the reductions.
 constexpr int kNormLn = 1, kNormAffine = 2, kNormMod = 4;
 
+// The (epilogue, norm) pairs of the flow LM's linears, the only ones built: no norm in front of input_linear,
+// out_proj, linear2, the flow net's linears of its own rows and, behind z_proj, the EOS logit and cond_embed;
+// the affine norm in front of in_proj, linear1, z_proj, the EOS logit and cond_embed; with the modulation in
+// front of mlp.0; the modulation alone in front of the final linear.
+constexpr bool linear_built(int epi, int norm) {
+    return norm == 0 ? epi != kLinGeluErf && epi != kLinGeluTanh
+           : norm == (kNormLn | kNormAffine)
+               ? epi == kLinStore || epi == kLinGeluErf || epi == kLinGeluTanh || epi == kLinSilu || epi == kLinSiluAddVec
+           : norm == (kNormLn | kNormAffine | kNormMod) ? epi == kLinSilu
+                                                        : norm == (kNormLn | kNormMod) && (epi == kLinStore || epi == kLinAxpy);
+}
+
 // y (bias added) to the output value: eo the auxiliary operand, er the output's old value
 template <int EPI> __device__ __forceinline__ float linear_epilogue(float y, float eo, float er, float alpha) {
     if constexpr (EPI == kLinStore) {
@@ -1356,7 +1368,11 @@ template <int NST, int MT, int NORM>
 static hipError_t linear_f32_rows_mt(const float *x, int ldx, int M, int K, const float *W, const float *b, int N, int epi,
                                      const LinOut &lo, const LinNorm &ln, hipStream_t stream) {
     const dim3 grid((N + 15) / 16 * ((M + 16 * MT - 1) / (16 * MT))), block(512);
-#define XNP_LIN(E) hipLaunchKernelGGL((k_linear_f32_rows<NST, MT, E, NORM>), grid, block, 0, stream, x, ldx, M, K, W, b, N, lo, ln)
+#define XNP_LIN(E)                                                                                                 \
+    if constexpr (linear_built(E, NORM))                                                                           \
+        hipLaunchKernelGGL((k_linear_f32_rows<NST, MT, E, NORM>), grid, block, 0, stream, x, ldx, M, K, W, b, N, lo, ln); \
+    else                                                                                                           \
+        return hipErrorInvalidValue
     switch (epi) {
     case kLinStore: XNP_LIN(kLinStore); break;
     case kLinGeluErf: XNP_LIN(kLinGeluErf); break;
@@ -1385,7 +1401,11 @@ template <int KC, int NORM>
 static hipError_t linear_f32_kc(const float *x, int ldx, int M, int K, const float *W, const float *b, int N, int epi,
                                 const LinOut &lo, const LinNorm &ln, hipStream_t stream) {
     const dim3 grid((N + 3) / 4), block(256);
-#define XNP_LIN(E) hipLaunchKernelGGL((k_linear_f32<KC, E, NORM>), grid, block, 0, stream, x, ldx, M, K, W, b, N, lo, ln)
+#define XNP_LIN(E)                                                                                                 \
+    if constexpr (linear_built(E, NORM))                                                                           \
+        hipLaunchKernelGGL((k_linear_f32<KC, E, NORM>), grid, block, 0, stream, x, ldx, M, K, W, b, N, lo, ln);     \
+    else                                                                                                           \
+        return hipErrorInvalidValue
     switch (epi) {
     case kLinStore: XNP_LIN(kLinStore); break;
     case kLinGeluErf: XNP_LIN(kLinGeluErf); break;
@@ -1428,7 +1448,7 @@ hipError_t launch_linear_f32(const float *x, int ldx, int M, int K, const float 
     if (ln->w && ln->shift) return linear_f32_norm<kNormLn | kNormAffine | kNormMod>(x, ldx, M, K, W, b, N, epi, lo, *ln, stream);
     if (ln->w) return linear_f32_norm<kNormLn | kNormAffine>(x, ldx, M, K, W, b, N, epi, lo, *ln, stream);
     if (ln->shift) return linear_f32_norm<kNormLn | kNormMod>(x, ldx, M, K, W, b, N, epi, lo, *ln, stream);
-    return linear_f32_norm<kNormLn>(x, ldx, M, K, W, b, N, epi, lo, *ln, stream);
+    return hipErrorInvalidValue; // no linear of the flow LM takes the norm alone
 }
 
 // LUTConditioner::embed_tokens (conditioners.rs:239-262): out[r] = table[ids[r]], rows of dim f32.
