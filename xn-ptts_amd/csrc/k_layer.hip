@@ -1220,7 +1220,10 @@ __global__ __launch_bounds__(256) void k_linear_f32(const float *x, int ldx, int
 // whose four values go to four products of 4 k each (x and W in the same (g, value) slot, so every k
 // meets its own).  Four sums a tile, one per value, then the waves' shares through LDS in a fixed
 // order: chains of NST additions, as short as k_linear_f32's.  The LayerNorm's moments are taken the same way
-// (the lane's values, its row's 4 lanes, the 8 waves), in two passes over the registers.
+// (the lane's values, its row's 4 lanes, the 8 waves), in two passes over the registers.  Its operands are
+// loaded with x and W, or (LATE: K above 512 with many of them) as they are used, since a wave holds 256
+// registers at most: loaded ahead, the affine and modulated norm spilled 97 of K = 1024's and 456 of K = 2048's
+// (two row tiles); a 2048-wide model of 2 layers, 16 prompts of 20 tokens: 1296 and 949 us, its frame 376 and 292.
 //
 // At prompt sizes this is bound by the launch and one round trip to memory; k_linear_f32 took the rows
 // one after another, a round trip and three wave sums each (64 rows of 512: 15-27 us a launch, here
@@ -1233,28 +1236,36 @@ __global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx
     __shared__ float mom[2][8][MT * 16];
     const int ntn = (N + 15) / 16, m0 = (int)blockIdx.x / ntn * (16 * MT), n0 = (int)blockIdx.x % ntn * 16;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
+    constexpr bool AFF = (NORM & kNormAffine) != 0, MOD = (NORM & kNormMod) != 0;
+    constexpr bool LATE = (MT + 1 + 2 * AFF + 2 * MT * MOD) * NST > 40; // 16 bytes a lane each
+    constexpr int NL = LATE ? 1 : NST; // norm operands held
     // every load is unconditional, its row and k clamped; values past K are zeroed on the x side
-    f32x4_a4 xv[MT][NST], wv[NST], sh[MT][NST], sc[MT][NST], nw[NST], nb[NST];
+    f32x4_a4 xv[MT][NST], wv[NST], sh[MT][NL], sc[MT][NL], nw[NL], nb[NL];
     int k[NST];
+    auto norm_load = [&](int i, int s) { // k[i]'s norm operands, into place s
+        const int kk = min(k[i], K - 4);
+        if constexpr (AFF) {
+            nw[s] = *(const f32x4_a4 *)(ln.w + kk);
+            nb[s] = *(const f32x4_a4 *)(ln.b + kk);
+        }
+        if constexpr (MOD) {
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                const size_t o = (size_t)min(m0 + 16 * j + l16, M - 1) * ln.ld_mod + kk;
+                sh[j][s] = *(const f32x4_a4 *)(ln.shift + o);
+                sc[j][s] = *(const f32x4_a4 *)(ln.scale + o);
+            }
+        }
+    };
     const float *wr = W + (size_t)min(n0 + l16, N - 1) * K;
 #pragma unroll
     for (int i = 0; i < NST; ++i) {
         k[i] = 16 * (w * NST + i) + 4 * g;
         const int kk = min(k[i], K - 4);
         wv[i] = *(const f32x4_a4 *)(wr + kk);
-        if constexpr ((NORM & kNormAffine) != 0) {
-            nw[i] = *(const f32x4_a4 *)(ln.w + kk);
-            nb[i] = *(const f32x4_a4 *)(ln.b + kk);
-        }
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            const size_t m = min(m0 + 16 * j + l16, M - 1);
-            xv[j][i] = *(const f32x4_a4 *)(x + m * ldx + kk);
-            if constexpr ((NORM & kNormMod) != 0) {
-                sh[j][i] = *(const f32x4_a4 *)(ln.shift + m * ln.ld_mod + kk);
-                sc[j][i] = *(const f32x4_a4 *)(ln.scale + m * ln.ld_mod + kk);
-            }
-        }
+        for (int j = 0; j < MT; ++j) xv[j][i] = *(const f32x4_a4 *)(x + (size_t)min(m0 + 16 * j + l16, M - 1) * ldx + kk);
+        if constexpr (!LATE) norm_load(i, i);
     }
     // the output this thread finishes (tile row er of row tile ej, column n0 + en) and its operands
     const int ej = threadIdx.x >> 8, er_ = (threadIdx.x >> 4) & 15, en = threadIdx.x & 15;
@@ -1317,13 +1328,19 @@ __global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx
         }
         moment(v, 1, sq);
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            const float rstd = 1.0f / __builtin_sqrtf(sq[j] / (float)K + ln.eps);
+        for (int j = 0; j < MT; ++j) sq[j] = 1.0f / __builtin_sqrtf(sq[j] / (float)K + ln.eps);
 #pragma unroll
-            for (int i = 0; i < NST; ++i) {
-                xv[j][i] *= rstd;
-                if constexpr ((NORM & kNormAffine) != 0) xv[j][i] = xv[j][i] * nw[i] + nb[i];
-                if constexpr ((NORM & kNormMod) != 0) xv[j][i] = xv[j][i] * (sc[j][i] + 1.0f) + sh[j][i];
+        for (int i = 0; i < NST; ++i) {
+            const int s = LATE ? 0 : i;
+            if constexpr (LATE) {
+                if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0); // four places' loads at a time
+                norm_load(i, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                xv[j][i] *= sq[j];
+                if constexpr (AFF) xv[j][i] = xv[j][i] * nw[s] + nb[s];
+                if constexpr (MOD) xv[j][i] = xv[j][i] * (sc[j][s] + 1.0f) + sh[j][s];
             }
         }
     }
@@ -1391,9 +1408,12 @@ static hipError_t linear_f32_rows_mt(const float *x, int ldx, int M, int K, cons
 template <int NST, int NORM>
 static hipError_t linear_f32_rows(const float *x, int ldx, int M, int K, const float *W, const float *b, int N, int epi,
                                   const LinOut &lo, const LinNorm &ln, hipStream_t stream) {
-    // two row tiles a group (W read once for both) once one-tile groups fill the chip twice over
-    if ((int64_t)((N + 15) / 16) * ((M + 15) / 16) >= 1024)
-        return linear_f32_rows_mt<NST, 2, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
+    // two row tiles a group (W read once for both) once one-tile groups fill the chip twice over, where the
+    // registers hold them
+    if constexpr (NST <= 8 || NORM == 0) {
+        if ((int64_t)((N + 15) / 16) * ((M + 15) / 16) >= 1024)
+            return linear_f32_rows_mt<NST, 2, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
+    }
     return linear_f32_rows_mt<NST, 1, NORM>(x, ldx, M, K, W, b, N, epi, lo, ln, stream);
 }
 
