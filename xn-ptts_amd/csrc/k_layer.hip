@@ -1219,17 +1219,21 @@ __global__ __launch_bounds__(256) void k_linear_f32(const float *x, int ldx, int
 // and W is loaded at once, 16 bytes a lane: lane (l16, g) holds row (column) l16 at k = 16 i + 4 g .. + 3,
 // whose four values go to four products of 4 k each (x and W in the same (g, value) slot, so every k
 // meets its own).  Four sums a tile, one per value, then the waves' shares through LDS in a fixed
-// order: chains of NST additions, as short as k_linear_f32's.  The LayerNorm's moments are taken the same way
-// (the lane's values, its row's 4 lanes, the 8 waves), in two passes over the registers.  Its operands are
-// loaded with x and W, or (LATE: K above 512 with many of them) as they are used, since a wave holds 256
-// registers at most: loaded ahead, the affine and modulated norm spilled 97 of K = 1024's and 456 of K = 2048's
-// (two row tiles); a 2048-wide model of 2 layers, 16 prompts of 20 tokens: 1296 and 949 us, its frame 376 and 292.
+// order.  A product adds its 4 k one after another, so the even and the odd products are summed apart where the
+// registers hold both: chains as short as k_linear_f32's.  (Summed in one, a 1024-wide model's first frame
+// stood 6.6e-7 from 64 bits where k_linear_f32's stands 5.4e-7, and 5.7e-7 so; rms of 16 streams.)  The
+// LayerNorm's moments are taken the same way (the lane's values, its row's 4 lanes, the 8 waves), in two passes
+// over the registers.  Its operands are loaded with x and W, or (LATE: K above 512 with many of them) as they
+// are used, since a wave holds 256 registers at most: loaded ahead, the affine and modulated norm spilled 97 of
+// K = 1024's and 456 of K = 2048's (two row tiles); a 2048-wide model of 2 layers, 16 prompts of 20 tokens:
+// 1296 and 949 us, its frame 376 and 292.
 //
 // At prompt sizes this is bound by the launch and one round trip to memory; k_linear_f32 took the rows
 // one after another, a round trip and three wave sums each (64 rows of 512: 15-27 us a launch, here
 // 4-10).
 template <int NST, int MT, int EPI, int NORM>
-__global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx, int M, int K, const float *W,
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NST > 4 || (MT > 1 && (NORM & kNormMod)) ? 2 : 4)))
+void k_linear_f32_rows(const float *x, int ldx, int M, int K, const float *W,
                                                          const float *bias, int N, LinOut lo, LinNorm ln) {
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4))); // rows need word alignment only
     __shared__ float red[8][MT][16][17];
@@ -1238,7 +1242,7 @@ __global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
     constexpr bool AFF = (NORM & kNormAffine) != 0, MOD = (NORM & kNormMod) != 0;
     constexpr bool LATE = (MT + 1 + 2 * AFF + 2 * MT * MOD) * NST > 40; // 16 bytes a lane each
-    constexpr int NL = LATE ? 1 : NST; // norm operands held
+    constexpr int NL = LATE ? 1 : NST, NA = MT * NST > 16 ? 1 : 2; // norm operands held; sums a value
     // every load is unconditional, its row and k clamped; values past K are zeroed on the x side
     f32x4_a4 xv[MT][NST], wv[NST], sh[MT][NL], sc[MT][NL], nw[NL], nb[NL];
     int k[NST];
@@ -1344,11 +1348,11 @@ __global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx
             }
         }
     }
-    f32x4_t acc[MT][4];
+    f32x4_t acc[MT][4][NA];
 #pragma unroll
     for (int j = 0; j < MT; ++j)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[j][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < 4 * NA; ++c) acc[j][c / NA][c % NA] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < NST; ++i) {
 #pragma unroll
@@ -1356,15 +1360,22 @@ __global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx
             const bool in = k[i] < K;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                acc[j][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? xv[j][i][c] : 0.f, wv[i][c], acc[j][c], 0, 0, 0);
+                acc[j][c][i % NA] =
+                    __builtin_amdgcn_mfma_f32_16x16x4f32(in ? xv[j][i][c] : 0.f, wv[i][c], acc[j][c][i % NA], 0, 0, 0);
         }
+    }
+    if constexpr (NA > 1) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[j][c][0] += acc[j][c][NA - 1];
     }
     // lane: column l16, rows 4 g + r of each row tile
 #pragma unroll
     for (int j = 0; j < MT; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            red[w][j][4 * g + r][l16] = (acc[j][0][r] + acc[j][1][r]) + (acc[j][2][r] + acc[j][3][r]);
+            red[w][j][4 * g + r][l16] = (acc[j][0][0][r] + acc[j][1][0][r]) + (acc[j][2][0][r] + acc[j][3][0][r]);
     __syncthreads();
     if (!mine) return;
     float p[8];
@@ -1377,8 +1388,9 @@ __global__ __launch_bounds__(512) void k_linear_f32_rows(const float *x, int ldx
 // Rows from which k_linear_f32_rows is taken: a whole row tile.  A prompt of the 6-layer model with its
 // first frame (row by row, then on row tiles): 4 tokens 391 and 365 us, 8 tokens 431 and 373, 16 tokens
 // 560 and 387, 64 tokens 1231 and 424.  Below 16 the gain is small, and the other order of the sums there
-// takes a model that feeds its latents back (5 frames from two 5-token prompts) past the 1e-5 its f32
-// results are held to (1.1e-5).
+// moves a model that feeds its latents back (5 frames from two 5-token prompts) past the 1e-5 of the oracle that
+// f32 results are held to (1.1e-5, most of it the oracle's own: its sums stand 1.3e-5 from 64 bits after five
+// such frames, either kernel's 3e-6 to 6e-6).
 constexpr int kLinRows = 16;
 
 template <int NST, int MT, int NORM>
