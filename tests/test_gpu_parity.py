@@ -1404,6 +1404,34 @@ def test_prefill_after_a_separate_append(cache, act):
     p.step()
 
 
+def test_an_append_of_more_rows_than_one_launch_holds_threads_for():
+    # 4 195 328 rows of 16 kv heads (a wave each) are more threads than the 2^32 a launch may have: 1024 streams'
+    # appends of 4097 rows, each stream's the same rows, against one stream's append alone
+    n, t, h = 1024, 4097, 16
+    k, v = (torch.randn((1, t, h, 64), device=DEV, generator=torch.Generator(device=DEV).manual_seed(s)).to(torch.bfloat16)
+            for s in (5, 6))
+    rows = []
+    for streams in (1, n):
+        pool = xnp.KvPool(num_layers=1, num_heads=h, num_blocks=streams * 257, max_streams=streams, max_blocks_per_stream=257,
+                          cache_dtype="bf16", act_dtype="bf16", max_pos=4112)
+        ids = [pool.init_state(4112) for _ in range(streams)]
+        kk, vv = k.expand(streams, -1, -1, -1).contiguous(), v.expand(streams, -1, -1, -1).contiguous()
+        pool.begin(ids, t=t)
+        pool.append(0, kk, vv)
+        pool.end()
+        torch.cuda.synchronize()
+        for i in (0, streams // 4, streams // 2, streams - 1):
+            got = [torch.empty((t, h, 64), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+            for kv in (0, 1):
+                pool.read_rows(ids[i], 0, kv, 0, got[kv])
+            torch.cuda.synchronize()
+            rows.append(got)
+        del kk, vv, pool
+        torch.cuda.empty_cache()
+    for got in rows[1:]:
+        assert torch.equal(got[0], rows[0][0]) and torch.equal(got[1], rows[0][1])
+
+
 @pytest.mark.parametrize("cache", ["bf16", "i8"])
 def test_long_prompts_take_several_rounds(cache):
     # 300- and 530-row prompts: more than one round of 256 query rows per work group, on top of
