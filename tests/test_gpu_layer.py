@@ -72,11 +72,11 @@ def test_linear_q8_with_w_in_registers_matches_the_oracle(rows, n, epi):
     assert (host(y)[:, n:] == 7.0).all()  # nothing past the columns
 
 
-@pytest.mark.parametrize("n,epi", [(512, "residual"), (4096, "gelu_erf")])
-def test_linear_q8_on_128_column_tiles_matches_the_oracle(n, epi):
-    # 128 x 128 tiles where they fill whole rounds of 512 groups: K = 2048 (two halves a group) and 1024,
-    # the last row tile one row
-    check_linear_q8(13057 if n == 512 else 1665, 2048 if n == 512 else 1024, n, epi)
+@pytest.mark.parametrize("rows,k,n,epi", [(6017, 2048, 512, "residual"), (13057, 2048, 512, "residual"), (1665, 1024, 4096, "gelu_erf")])
+def test_linear_q8_on_128_column_tiles_matches_the_oracle(rows, k, n, epi):
+    # 128 x 128 tiles where they nearly fill whole rounds: of 256 groups with K = 2048 (two halves a group;
+    # three quarters of one round, four fifths of two), of 512 with K = 1024; the last row tile one row
+    check_linear_q8(rows, k, n, epi)
 
 
 # Few rows (up to 256) run in one pass per 16 or 32 rows x 32 columns, K of 512, 1024 and 2048: one row, a

@@ -1071,10 +1071,16 @@ hipError_t launch_gemm_q8(const void *A, int M, int K, const int8_t *W, const fl
     const bool mi1 = groups64 < 512;
     if (gemm_wres_runs(M, K, N, epi, go) > 0) return gemm_q8_wres(A, M, W, s, N, epi, go, stream);
     // 128 x 128 tiles (twice the products per barrier and per byte staged of 128 x 64) where they fill the
-    // chip's 512 places (two groups a CU) in nearly whole rounds: 16384 rows, linear2 65 -> 49 us, out_proj
-    // 20.4 -> 17.6; at 5000 rows linear1 (640 groups, the second round of 128) took 33.9 against 30.4.
-    const int64_t wide = (N + 127) / 128 * (int64_t)((M + 127) / 128), rounds = (wide + 511) / 512;
-    if (5 * wide >= 4 * 512 * rounds && !go.a_f32 && gemm_staged(N, epi, go)) {
+    // chip's places in nearly whole rounds.  K of 512 and 1024: two groups a CU (74 KB of LDS each), 512 places,
+    // four fifths and more of them in every round.  512 columns, smaller tiles then these: K = 512 at 12288
+    // rows (three quarters) 17.7 and 18.2 us, 13057 rows 20.7 and 18.1, 16384 rows 21.5 and 19.2, 20480 rows
+    // (two rounds, five eighths) 26.3 and 26.7.  K = 2048, two halves a group (147 KB): one a CU, 256 places,
+    // from three quarters on: 4096 rows (half) 23.0 and 26.7 us, 6144 rows (three quarters) 31.3 and 27.5, 8192
+    // rows 38.0 and 28.0, 10240 rows (two rounds, five eighths) 43.5 and 48.0, 12288 rows (three quarters)
+    // 51.0 and 48.3, 16384 rows 66.4 and 50.5.  (Each alone, warm.)
+    const int64_t wide = (N + 127) / 128 * (int64_t)((M + 127) / 128), places = K == 32 * kGmK ? 256 : 512;
+    const int64_t room = places * ((wide + places - 1) / places); // of every round it takes
+    if ((places == 256 ? 4 * wide >= 3 * room : 5 * wide >= 4 * room) && !go.a_f32 && gemm_staged(N, epi, go)) {
         if (K == 8 * kGmK) return gemm_q8_stg<4, 4, 1, true, 8>(A, M, K, W, s, N, epi, go, stream);
         if (K == 16 * kGmK) return gemm_q8_stg<4, 4, 1, true, 16>(A, M, K, W, s, N, epi, go, stream);
         if (K == 32 * kGmK) return gemm_q8_stg<4, 4, 2, true, 16>(A, M, K, W, s, N, epi, go, stream);
