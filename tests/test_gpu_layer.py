@@ -81,7 +81,8 @@ def test_linear_q8_on_128_column_tiles_matches_the_oracle(rows, k, n, epi):
 
 # Few rows (up to 256) run in one pass per 16 or 32 rows x 32 columns, K of 512, 1024 and 2048: one row, a
 # tile, one more, the most rows and one past them (which takes k_gemm_q8), ragged columns (the flow
-# entry: 40 and 264), every epilogue the flow LM uses there with and without a LayerNorm in front.
+# entry: 40 and 264), every epilogue the flow LM uses there.  (With a LayerNorm in front: the layer step bit for
+# bit below, and the q8 frames of 17 and 256 streams in test_gpu_flow_lm.py.)
 @pytest.mark.parametrize("rows", [1, 16, 17, 130, 256, 257])
 @pytest.mark.parametrize("k,n,epi", [(512, 40, "store"), (512, 264, "silu"), (1024, 520, "gated"), (2048, 512, "axpy_f32"),
                                      (512, 32, "store_f32"), (2048, 64, "silu_add")])
@@ -136,7 +137,7 @@ def test_quantize_rows_matches_the_oracle_bit_for_bit():
     assert np.array_equal(q, oq) and np.array_equal(s.view(np.uint32), os_.view(np.uint32))
 
 
-def make_weights(rng, H=8, KVH=8, D=64, dm=512, ff=2048, ls=False):
+def make_weights(rng, H=8, KVH=8, D=64, dm=512, ff=2048, ls=False, gelu="erf"):
     qr = lambda n, k: xnp.quantize_rows(rng.standard_normal((n, k)).astype(np.float32) * 0.02)
     parts = dict(zip(["wqkv", "sqkv"], qr((H + 2 * KVH) * D, dm)))
     parts.update(zip(["wout", "sout"], qr(dm, H * D)))
@@ -150,7 +151,7 @@ def make_weights(rng, H=8, KVH=8, D=64, dm=512, ff=2048, ls=False):
     orc = oracle.LayerWeights(**parts)
     d = {k_: (dev(v, torch.int8 if v.dtype == np.int8 else torch.float32) if v is not None else None)
          for k_, v in parts.items()}
-    return orc, xnp.LayerWeights(**d)
+    return orc, xnp.LayerWeights(**d, gelu=gelu)
 
 
 # ff 2048 (Phonon-40m's): linear2's K = 2048 runs the GEMM's two-half groups
@@ -274,17 +275,19 @@ def test_the_layer_step_configuration_at_full_size_spot_checked():
     assert pool.check_tables() == 0
 
 
-@pytest.mark.parametrize("ls", [False, True])
-def test_the_layer_step_equals_its_pieces_bit_for_bit(ls):
+@pytest.mark.parametrize("ls,gelu", [(False, "erf"), (True, "erf"), (False, "tanh")])
+def test_the_layer_step_equals_its_pieces_bit_for_bit(ls, gelu):
     # xnp_layer_step against the same layer composed of the public pieces on a second, identical
     # pool: layer_norm, linear_q8 (store, residual, gelu) and attend.  The step is those launches in
     # that order on its own workspace, so every bit must agree: the residual stream and the cache
     # rows compared as integers.  Row counts that no 16-row band divides (37 single rows, a 7-row
-    # prompt on 5 streams), 300 rows, with and without layer scales.
+    # prompt on 5 streams), those from which the projections with the norm in front take two row tiles a
+    # group (65: linear1, 81: in_proj), 130, the most rows they take (256), 300, with and without layer
+    # scales, both GELUs.
     rng = np.random.default_rng(71 + ls)
     L, H, KVH, D, dm, ff = 1, 8, 8, 64, 512, 2048
     qd, kd = H * D, KVH * D
-    orc, lw = make_weights(rng, H=H, KVH=KVH, ff=ff, ls=ls)
+    orc, lw = make_weights(rng, H=H, KVH=KVH, ff=ff, ls=ls, gelu=gelu)
     dw = {k: dev(getattr(orc, k), torch.int8 if getattr(orc, k).dtype == np.int8 else torch.float32)
           for k in ("wqkv", "sqkv", "wout", "sout", "w1", "s1", "w2", "s2", "ln1_w", "ln1_b", "ln2_w", "ln2_b")}
     dw["ls1"] = dev(orc.ls1, torch.float32) if ls else None
@@ -295,7 +298,8 @@ def test_the_layer_step_equals_its_pieces_bit_for_bit(ls):
                         page_seed=13) for _ in range(2)]
     ids = [[p.init_state(cap) for _ in range(S)] for p in pools]
     ws = torch.empty(pools[0].layer_workspace(S * 7, dm, ff), dtype=torch.uint8, device=DEV)
-    for which, t in ((list(range(37)), 1), (list(range(5)), 7), (list(range(S)), 1)):
+    for which, t in ((list(range(37)), 1), (list(range(5)), 7), (list(range(S)), 1), (list(range(65)), 1), (list(range(81)), 1),
+                     (list(range(26)), 5), (list(range(256)), 1)):
         n, M = len(which), len(which) * t
         x0 = normal(rng, (n, t, dm), "bf16")
         xa, xb = dev(x0), dev(x0)
@@ -314,7 +318,7 @@ def test_the_layer_step_equals_its_pieces_bit_for_bit(ls):
         pools[1].attend(0, q, k, v, att, 1.0 / np.sqrt(D))
         xnp.linear_q8(att, dw["wout"], dw["sout"], xv, "residual", ls=dw["ls1"])
         xnp.layer_norm(xv, dw["ln2_w"], dw["ln2_b"], h)
-        xnp.linear_q8(h, dw["w1"], dw["s1"], f, "gelu_erf")
+        xnp.linear_q8(h, dw["w1"], dw["s1"], f, "gelu_" + gelu)
         xnp.linear_q8(f, dw["w2"], dw["s2"], xv, "residual", ls=dw["ls2"])
         pools[1].end()
         torch.cuda.synchronize()
