@@ -109,6 +109,31 @@ def test_flow_linear_q8_of_few_rows_matches_the_oracle(rows, k, n, epi):
     assert rel_err(host(y), want) <= TOL
 
 
+# Every finite bf16 value through the erf GELU's epilogue on each of the three kernels that have it (few rows,
+# tiles, W in registers): W picks the value out of its row, so y is the value itself.  A result whose exponential
+# is subnormal (-13.25 to -13.5: 3e-39 and less) is zero, as the hardware's exponential is there.
+@pytest.mark.parametrize("rows,n", [(256, 64), (1020, 64), (5100, 1024)])
+def test_gelu_of_every_finite_bf16_value_is_the_nearest_normal_one(rows, n):
+    from scipy.special import erfc
+    y = (np.arange(65536, dtype=np.uint32) << 16).view(np.float32)
+    y = np.resize(y[np.isfinite(y)], (max(rows, 1020), 64))
+    with np.errstate(under="ignore"):
+        exact = y.astype(np.float64) * 0.5 * erfc(-y.astype(np.float64) / np.sqrt(2.0))
+    w = np.zeros((n, 512), np.int8)
+    w[np.arange(n), np.arange(n) % 64] = 1
+    for r in range(0, y.shape[0], rows):
+        x = np.zeros((min(rows, y.shape[0] - r), 512), np.float32)
+        x[:, :64] = y[r:r + rows]
+        out = torch.empty((x.shape[0], n), dtype=torch.bfloat16, device=DEV)
+        xnp.linear_q8(dev(x), dev(w, torch.int8), torch.ones(n, device=DEV), out, "gelu_erf")
+        torch.cuda.synchronize()
+        got, want = host(out).reshape(-1, n // 64, 64).astype(np.float64), exact[r:r + rows][:, None]
+        # half a bf16 step of the exact value (of a subnormal one: of the smallest normal's step)
+        step = np.exp2(np.floor(np.log2(np.maximum(np.abs(want), 2.0 ** -126))) - 7)
+        bad = ~((np.abs(got - want) <= 0.5 * step) | ((np.abs(want) < 2.0 ** -126) & (got == 0)))
+        assert not bad.any(), (y[r:r + rows][bad.any(1)][:8], got[bad][:8], int(bad.sum()))
+
+
 def check_linear_q8(rows, k, n, epi):
     rng = np.random.default_rng(rows * 7 + n)
     x = normal(rng, (rows, k), "bf16")

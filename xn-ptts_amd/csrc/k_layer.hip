@@ -140,23 +140,13 @@ hipError_t launch_layer_norm(const void *x, int rows, int dim, const float *w, c
     return launch_layer_norm_mod(x, rows, dim, w, b, eps, nullptr, nullptr, 0, out, stream);
 }
 
-// y = epilogue(s[n] * sum_k A[m][k] W[n][k]): A [M][K] bf16, W [N][K] int8 with one f32 scale per
-// output channel (row of W), the sum on v_mfma_f32_16x16x32_bf16 with W widened to bf16 exactly
-// (|q| <= 127).  One work group of 4 waves per 64 x 64 tile of y, each wave 32 x 32 (2 x 2 MFMA
-// tiles); K in chunks of 64 staged through LDS, double-buffered, with the loads of the next three
-// chunks in flight while one is multiplied.  The product, plus the bias when given, is rounded to bf16 (the
-// projection's output tensor), then: kStore writes it (column ranges may go to separate outputs:
-// q, k and v), kGelu* write gelu(y) rounded, kResidual adds y (times the layer scale, rounded,
-// when given) into X and rounds: X + layer_scale(linear(..)) as transformer.rs:612-633 does; the
-// flow net's epilogues are listed with their enum.  N may be any width (columns past N are
-// neither loaded nor stored) and K any multiple of 16 (the last chunk's loads past K read zeros).
 // gelu(y) = y Phi(y) for the bf16 epilogues (the erf form), from the tail Q(a) = 1 - Phi(a) = exp(-a^2 / 2)
 // p(t), t = 1 / (1 + 0.3 a), p a polynomial of degree 8 fitted to exp(a^2 / 2) Q(a) (the scaled
 // complementary error function) over a in [0, 13.5], 5.7e-8 relative at most; 17 VALU instructions in
 // one path, where 0.5 y (1 + erff(y / sqrt 2)) took 38 (linear1 at 16384 rows: 20 of its 75 us).  For
-// every finite bf16 y the result rounds to the bf16 nearest the exact value; the erff form, whose
-// 1 + erff cancels on the negative side, missed it for 197 of them.  Infinities and NaN as in the
-// erff form.
+// every finite bf16 y the result rounds to the bf16 nearest the exact value, but for -13.25 to -13.5, whose
+// results are subnormal and whose exponential the hardware rounds to zero; the erff form, whose 1 + erff
+// cancels on the negative side, missed it for 197.  Infinities and NaN as in the erff form.
 __device__ __forceinline__ float gelu_erf(float y) {
     const float a = fminf(fabsf(y), 40.f);
     const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(a, 0.3f, 1.f));
@@ -173,6 +163,16 @@ __device__ __forceinline__ float gelu_erf(float y) {
     return y * (y < 0.f ? q : 1.f - q);
 }
 
+// y = epilogue(s[n] * sum_k A[m][k] W[n][k]): A [M][K] bf16, W [N][K] int8 with one f32 scale per
+// output channel (row of W), the sum on v_mfma_f32_16x16x32_bf16 with W widened to bf16 exactly
+// (|q| <= 127).  One work group of 4 waves per 64 x 64 tile of y, each wave 32 x 32 (2 x 2 MFMA
+// tiles); K in chunks of 64 staged through LDS, double-buffered, with the loads of the next three
+// chunks in flight while one is multiplied.  The product, plus the bias when given, is rounded to bf16 (the
+// projection's output tensor), then: kStore writes it (column ranges may go to separate outputs:
+// q, k and v), kGelu* write gelu(y) rounded, kResidual adds y (times the layer scale, rounded,
+// when given) into X and rounds: X + layer_scale(linear(..)) as transformer.rs:612-633 does; the
+// flow net's epilogues are listed with their enum.  N may be any width (columns past N are
+// neither loaded nor stored) and K any multiple of 16 (the last chunk's loads past K read zeros).
 constexpr int kGmT = 64;  // tile rows and columns
 constexpr int kGmK = 64;  // K chunk
 constexpr int kGmLd = 72; // LDS row length in bf16
