@@ -811,7 +811,6 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
     const int h = (int)blockIdx.x % per % pv.H, b = (int)blockIdx.x % per / pv.H;
     const StreamPlan P = bv.plans[b];
     const bool held = P.pos_pre > 0, alone = pv.H == pv.KVH;
-    if (held && back > 0) return; // the last round's group runs them all
     const int32_t *tab = pv.tables + (size_t)P.sid * pv.mbps;
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, hi = lane >> 5, col = lane & 31;
     const int W = P.window;
@@ -828,6 +827,7 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
     // rounds, so that no register holds their addresses through them; the first round's barrier
     // precedes every read of them)
     for (int i = tid; i < min(pv.mbps, kPfMaxPages); i += 64 * kWpWaves) spages[i] = tab[i];
+    if (held && back > 0) return; // the last round's group runs them all
 
     // A chunk's keys j0 + key go straight into LDS slot `slot` by 1 KB loads: lane l of load i of
     // wave w takes key 16 w + 8 i + l / 8 and holds its unit (l % 8) ^ swz(key), and the rope piece
@@ -894,8 +894,8 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
         }
     };
     const int nqt = (t + 15) / 16, rounds = (int)gridDim.x / per;
-    const int tq_first = held ? 0 : (rounds - 1 - back) * (kWpRound / 16);
-    const int tq_end = held ? nqt : min(nqt, tq_first + kWpRound / 16);
+    const int tq_last = (rounds - 1 - back) * (kWpRound / 16), tq_first = held ? 0 : tq_last;
+    const int tq_end = min(nqt, tq_last + kWpRound / 16);
     for (int tq0 = tq_first; tq0 < tq_end; tq0 += kWpRound / 16) {
         const int nq = min(kWpRound / 16, nqt - tq0);
         // the round's keys: from the window of its first row to its last row
