@@ -80,12 +80,12 @@ def test_linear_q8_on_128_column_tiles_matches_the_oracle(rows, k, n, epi):
 
 
 # Few rows (up to 256) run in one pass per 16 or 32 rows x 32 columns, K of 512, 1024 and 2048: one row, a
-# tile, one more, the most rows and one past them (which takes k_gemm_q8), ragged columns (the flow
-# entry: 40 and 264), every epilogue the flow LM uses there.  (With a LayerNorm in front: the layer step bit for
+# tile, one more, the most rows and one past them (which takes k_gemm_q8, as do more than 256 groups: 2056 columns
+# from 130 rows on), ragged columns (the flow entry: 40, 264 and 2056), every epilogue the flow LM uses there.  (With a LayerNorm in front: the layer step bit for
 # bit below, and the q8 frames of 17 and 256 streams in test_gpu_flow_lm.py.)
 @pytest.mark.parametrize("rows", [1, 16, 17, 130, 256, 257])
 @pytest.mark.parametrize("k,n,epi", [(512, 40, "store"), (512, 264, "silu"), (1024, 520, "gated"), (2048, 512, "axpy_f32"),
-                                     (512, 32, "store_f32"), (2048, 64, "silu_add")])
+                                     (512, 32, "store_f32"), (2048, 64, "silu_add"), (1024, 2056, "store")])
 def test_flow_linear_q8_of_few_rows_matches_the_oracle(rows, k, n, epi):
     rng = np.random.default_rng(rows * 11 + k + n)
     x = normal(rng, (rows, k), "bf16")
@@ -307,8 +307,8 @@ def test_the_layer_step_equals_its_pieces_bit_for_bit(ls, gelu):
     # that order on its own workspace, so every bit must agree: the residual stream and the cache
     # rows compared as integers.  Row counts that no 16-row band divides (37 single rows, a 7-row
     # prompt on 5 streams), those from which the projections with the norm in front take two row tiles a
-    # group (65: linear1, 81: in_proj), 130, the most rows they take (256), 300, with and without layer
-    # scales, both GELUs.
+    # group (65: linear1, 81: in_proj), past the groups they run in (130: linear1 apart from its norm, 256:
+    # in_proj too), 300, with and without layer scales, both GELUs.
     rng = np.random.default_rng(71 + ls)
     L, H, KVH, D, dm, ff = 1, 8, 8, 64, 512, 2048
     qd, kd = H * D, KVH * D

@@ -990,27 +990,38 @@ static hipError_t gemm_q8_mi(const void *A, int M, int K, const int8_t *W, const
     return gemm_q8_stg<MI, 2, KS, true, 0>(A, M, K, W, s, N, epi, go, stream);
 }
 
+// k_gemm_q8_small's row tiles a group: two (its columns of W read and widened for both) once one-tile groups are
+// more than the CUs: linear1 at 128 rows 4.3 -> 4.0 us, linear2 at 331 rows 9.2 -> 7.9.  And its groups.
+static bool small_two(int M, int N) { return (int64_t)((N + 31) / 32) * ((M + 15) / 16) > 256; }
+static int64_t small_groups(int M, int N) { return (int64_t)((N + 31) / 32) * (small_two(M, N) ? (M + 31) / 32 : (M + 15) / 16); }
+
 // Rows up to which k_gemm_q8_small is taken: each of its groups reads its rows and columns over all of K
 // (no tile larger than 32 x 32), which the larger tiles of k_gemm_q8 overtake.  A step of 9 layers (512
 // wide, FF 2048, caches of up to 800 rows; k_gemm_q8 with the LayerNorms apart, then here): 32 rows 360 and
 // 272 us, 128 rows 472 and 408, 256 rows 625 and 597, 300 rows 685 and 696.  The four projections alone,
 // warm: 40 rows 20.7 and 15.1 us, 256 rows 21.4 and 19.4, 600 rows 26.1 and 36.8.
+//
+// And no more groups than CUs, since a second round costs what the first did (K x N, larger tiles and here: 1024 x
+// 3072 at 64 rows, 192 groups, 6.4 and 5.1 us, at 100 rows, 384 groups, 6.5 and 7.8; 2048 x 4096 at 64 rows, 256
+// groups, 9.0 and 8.3, at 100 rows 10.2 and 13.6; 512 x 6144 at 33 rows, 384 groups, 4.6 and 5.0).  With the norm
+// inside too, though it saves a launch there (a layer of FF 2048 at 200 rows, linear1 in 448 groups, 32.6 us and
+// apart 31.7; FF 4096 at 128 rows, 512 groups, 43.3 and 41.7; at 200 rows 51.0 and 47.5): one rule for both keeps
+// the layer step equal to its pieces to the bit.
 constexpr int kSmallRows = 256;
 static bool gemm_small(int M, int K, int N, int epi, const GemmOut &go) {
-    return M <= kSmallRows && (K == 512 || K == 1024 || K == 2048) && !go.a_f32 && gemm_staged(N, epi, go);
+    return M <= kSmallRows && (K == 512 || K == 1024 || K == 2048) && !go.a_f32 && small_groups(M, N) <= 256 &&
+           gemm_staged(N, epi, go);
 }
 
 template <int EPI, int NS, int LNM>
 static hipError_t gemm_q8_small(const void *A, int M, const int8_t *W, const float *s, int N, const GemmOut &go,
                                 const LnIn &ln, hipStream_t stream) {
-    // two row tiles a group (its columns of W read and widened for both) once one-tile groups are more than
-    // the CUs: linear1 at 128 rows 4.3 -> 4.0 us, linear2 at 331 rows 9.2 -> 7.9
-    const int ntn = (N + 31) / 32, mts = (M + 15) / 16;
+    const dim3 grid(small_groups(M, N));
     const uint16_t *a = (const uint16_t *)A;
-    if (ntn * mts > 256)
-        hipLaunchKernelGGL((k_gemm_q8_small<EPI, NS, 2, LNM>), dim3(ntn * ((M + 31) / 32)), dim3(512), 0, stream, a, M, W, s, N, go, ln);
+    if (small_two(M, N))
+        hipLaunchKernelGGL((k_gemm_q8_small<EPI, NS, 2, LNM>), grid, dim3(512), 0, stream, a, M, W, s, N, go, ln);
     else
-        hipLaunchKernelGGL((k_gemm_q8_small<EPI, NS, 1, LNM>), dim3(ntn * mts), dim3(512), 0, stream, a, M, W, s, N, go, ln);
+        hipLaunchKernelGGL((k_gemm_q8_small<EPI, NS, 1, LNM>), grid, dim3(512), 0, stream, a, M, W, s, N, go, ln);
     return hipGetLastError();
 }
 
