@@ -46,24 +46,22 @@ hipError_t launch_pull_plan(const PoolView &pv, const void *src, void *dst, size
 // ---------------------------------------------------------------------------------------------
 // standalone append of t rows per stream, f32 and bf16 pools: a work group per (stream, row), one wave
 // per kv head.  (A page's rows in turn by one wave took 8.3 us for one stream's 64 rows, a round trip
-// each; a wave per row and head 3.4 us.)  A launch holds fewer than 2^32 threads, so of more rows than
-// kAppendGroups a group takes several.
+// each; a wave per row and head 3.4 us.)  A launch holds fewer than 2^32 threads: more rows than
+// kAppendGroups take several launches, from row r0 on.
 constexpr int kAppendGroups = 1 << 20;
 
 template <int CDT, bool ABF>
-__global__ __launch_bounds__(1024) void k_append(PoolView pv, BatchView bv, int layer, const void *k, const void *v) {
-    const int t = bv.t, j = threadIdx.x >> 6; // kv head
-    for (int r = blockIdx.x; r < bv.n * t; r += gridDim.x) {
-        const int b = r / t, i = r % t;
-        const StreamPlan P = bv.plans[b];
-        const int slot = P.write_slot + i;
-        const int page = pv.tables[(size_t)P.sid * pv.mbps + (slot >> 4)];
-        if (page < 0 || page >= pv.NB) continue; // begin took this page; never index the pool without one
-        constexpr int AE = ABF ? 2 : 4;
-        const size_t arow = ((size_t)P.out_row * t + i) * pv.KVH + j;
-        append_row_wave<CDT, ABF>(pv, layer, page, slot & 15, j, P.key_pos + i, (const char *)k + arow * kHeadDim * AE,
-                                  (const char *)v + arow * kHeadDim * AE, false);
-    }
+__global__ __launch_bounds__(1024) void k_append(PoolView pv, BatchView bv, int layer, const void *k, const void *v, int r0) {
+    const int t = bv.t, r = r0 + (int)blockIdx.x, b = r / t, i = r % t;
+    const StreamPlan P = bv.plans[b];
+    const int j = threadIdx.x >> 6; // kv head
+    const int slot = P.write_slot + i;
+    const int page = pv.tables[(size_t)P.sid * pv.mbps + (slot >> 4)];
+    if (page < 0 || page >= pv.NB) return; // begin took this page; never index the pool without one
+    constexpr int AE = ABF ? 2 : 4;
+    const size_t arow = ((size_t)P.out_row * t + i) * pv.KVH + j;
+    append_row_wave<CDT, ABF>(pv, layer, page, slot & 15, j, P.key_pos + i, (const char *)k + arow * kHeadDim * AE,
+                              (const char *)v + arow * kHeadDim * AE, false);
 }
 
 // The int8 append of a step's rows, one wave per (stream, page the rows touch, kv head, keys or
@@ -223,8 +221,9 @@ static hipError_t append_impl(const PoolView &pv, const BatchView &bv, int layer
         const int nseg = (bv.t + kBlock - 1) / kBlock + 1; // the most pages a stream's rows touch
         hipLaunchKernelGGL(k_append_i8<ABF>, dim3(bv.n * nseg * pv.KVH), dim3(128), 0, stream, pv, bv, layer, k, v, nseg);
     } else {
-        hipLaunchKernelGGL((k_append<CDT, ABF>), dim3(std::min(bv.n * bv.t, kAppendGroups)), dim3(64 * pv.KVH), 0, stream, pv, bv,
-                           layer, k, v);
+        for (int r0 = 0; r0 < bv.n * bv.t; r0 += kAppendGroups)
+            hipLaunchKernelGGL((k_append<CDT, ABF>), dim3(std::min(bv.n * bv.t - r0, kAppendGroups)), dim3(64 * pv.KVH), 0, stream,
+                               pv, bv, layer, k, v, r0);
     }
     return hipGetLastError();
 }
