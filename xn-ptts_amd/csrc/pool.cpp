@@ -1260,8 +1260,9 @@ extern "C" xnp_status xnp_batch_begin(xnp_pool *pool, const int32_t *ids, int32_
         B.bv.split = std::max(B.bv.split, decode_min_split(pool->view(), B.bv.prefix != 0));
     {
         const int gq = t == 1 ? decode_heads_per_group(pool->view(), B.bv.prefix != 0) : 1;
-        // (a window step's launch attends its rows together, one group per (stream, head))
-        const int64_t groups = (int64_t)n * (wsteps ? 1 : t) * pool->d.num_heads / gq;
+        // (a window step's launch attends its rows together, one group per (stream, head); int8's, a row at a
+        // time, measured slower with the more waves: 20 windows of 40 rows, 7 a step, 43.4 and 50.5 us)
+        const int64_t groups = (int64_t)n * (wsteps && pool->d.cache_dtype != XNP_I8 ? 1 : t) * pool->d.num_heads / gq;
         while (!pool->d.decode_split && B.bv.split < 8 && groups * B.bv.split < 1024)
             B.bv.split *= 2;
     }
