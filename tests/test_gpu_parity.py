@@ -575,6 +575,50 @@ def test_int8_prompt_rows_quantize_bit_for_bit(act, kvh, grow):
         p.assert_cache_equal(i)
 
 
+# Steps of few rows append a row after another (one and two rows, and three from 256 streams of 8 kv heads), more
+# and smaller ones a page's tile at once: codes and scales of 2 to 4 rows of 255 and 256 streams, over pages that
+# hold 0 to 15 rows, byte for byte those of the same rows appended one a step.
+@pytest.mark.parametrize("act", ["bf16", "f32"])
+@pytest.mark.parametrize("n", [255, 256])
+def test_int8_steps_of_few_rows_append_as_one_row_a_step(act, n):
+    g = torch.Generator(device=DEV).manual_seed(n)
+    pools, idss = [], []
+    for _ in range(2):
+        pool = xnp.KvPool(num_layers=1, num_heads=8, num_blocks=n * 2, max_streams=n, max_blocks_per_stream=2, cache_dtype="i8",
+                          act_dtype=act, max_pos=64)
+        pools.append(pool)
+        idss.append([pool.init_state(32) for _ in range(n)])
+    for i in range(n):  # 0 to 15 rows held
+        if i % 16:
+            k, v = (torch.randn((1, i % 16, 8, 64), device=DEV, generator=g).to(TORCH_DT[act]) for _ in range(2))
+            for pool, ids in zip(pools, idss):
+                pool.begin([ids[i]], t=i % 16)
+                pool.append(0, k, v) if i % 16 > 1 else pool.attend(0, k, k, v, torch.empty_like(k), 0.125)
+                pool.end()
+    for t in (2, 3, 4):
+        k, v = (torch.randn((n, t, 8, 64), device=DEV, generator=g).to(TORCH_DT[act]) * (1 + t) for _ in range(2))
+        pools[0].begin(idss[0], t=t)
+        pools[0].append(0, k, v)
+        pools[0].end()
+        for r in range(t):
+            kr, vr = k[:, r:r + 1].contiguous(), v[:, r:r + 1].contiguous()
+            pools[1].begin(idss[1])
+            pools[1].append(0, kr, vr)
+            pools[1].end()
+    torch.cuda.synchronize()
+    for i in range(0, n, 7):
+        rows = i % 16 + 9
+        for kv in (0, 1):
+            got = []
+            for pool, ids in zip(pools, idss):
+                x = torch.empty((rows, 8, 64), dtype=torch.int8, device=DEV)
+                sc = torch.zeros(((rows + 15) // 16, 8), device=DEV)
+                pool.read_rows(ids[i], 0, kv, 0, x, sc)
+                got.append((x, sc))
+            torch.cuda.synchronize()
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (i, kv)
+
+
 def test_int8_window_cache_matches_the_ring_it_stands_for():
     # An int8 window has no counterpart in the reference; it is an absolute ring of `context`
     # slots whose every row evicts the oldest, so the oracle's ring driven that way is its bar:

@@ -214,12 +214,43 @@ __global__ __launch_bounds__(128) void k_append_i8(PoolView pv, BatchView bv, in
     if (lane == 0) pv.scales[tile] = s;
 }
 
+// The same a row after another, one wave per kv head and a work group per (stream, page), for steps of one or
+// two rows, and of three in large batches: k_append_i8 takes the page's tile whole whatever the rows.  1000
+// streams, 8 kv heads, new pages / 37 held rows: one row 20.2 (k_append_i8) and 7.1 us / 20.6 and 7.1, two rows
+// 25.2 and 22.0 / 22.2 and 9.9, three 28.9 and 33.4 / 23.3 and 12.9, four 31.8 and 42.2 / 24.8 and 16.3; 8 streams:
+// two rows 5.3 and 6.0 / 4.7 and 4.4, three 6.4 and 8.4 / 4.7 and 4.9.
+template <bool ABF>
+__global__ __launch_bounds__(1024) void k_append_i8_few(PoolView pv, BatchView bv, int layer, const void *k, const void *v,
+                                                        int nseg) {
+    const int b = blockIdx.x / nseg, seg = blockIdx.x % nseg;
+    const StreamPlan P = bv.plans[b];
+    const int j = threadIdx.x >> 6, t = bv.t, ws = P.write_slot, blk = (ws >> 4) + seg; // j: kv head
+    const int i0 = max(0, blk * kBlock - ws), i1 = min(t, (blk + 1) * kBlock - ws);
+    if (i0 >= i1) return;
+    const int page = pv.tables[(size_t)P.sid * pv.mbps + blk];
+    if (page < 0 || page >= pv.NB) return; // begin took this page; never index the pool without one
+    constexpr int AE = ABF ? 2 : 4;
+    for (int i = i0; i < i1; ++i) {
+        const size_t arow = ((size_t)P.out_row * t + i) * pv.KVH + j;
+        const bool fresh = P.ring ? (P.fresh != 0) : (((ws + i) & 15) == 0);
+        append_row_wave<DT_I8, ABF>(pv, layer, page, (ws + i) & 15, j, P.key_pos + i, (const char *)k + arow * kHeadDim * AE,
+                                    (const char *)v + arow * kHeadDim * AE, fresh);
+        __syncthreads(); // the row's codes and scale before the next row reads them
+    }
+}
+static bool append_i8_few(const PoolView &pv, const BatchView &bv) {
+    return bv.t <= 2 || (bv.t == 3 && (int64_t)bv.n * pv.KVH >= 2048);
+}
+
 template <int CDT, bool ABF>
 static hipError_t append_impl(const PoolView &pv, const BatchView &bv, int layer, const void *k,
                               const void *v, hipStream_t stream) {
     if constexpr (CDT == DT_I8) {
         const int nseg = (bv.t + kBlock - 1) / kBlock + 1; // the most pages a stream's rows touch
-        hipLaunchKernelGGL(k_append_i8<ABF>, dim3(bv.n * nseg * pv.KVH), dim3(128), 0, stream, pv, bv, layer, k, v, nseg);
+        if (append_i8_few(pv, bv))
+            hipLaunchKernelGGL(k_append_i8_few<ABF>, dim3(bv.n * nseg), dim3(64 * pv.KVH), 0, stream, pv, bv, layer, k, v, nseg);
+        else
+            hipLaunchKernelGGL(k_append_i8<ABF>, dim3(bv.n * nseg * pv.KVH), dim3(128), 0, stream, pv, bv, layer, k, v, nseg);
     } else {
         for (int r0 = 0; r0 < bv.n * bv.t; r0 += kAppendGroups)
             hipLaunchKernelGGL((k_append<CDT, ABF>), dim3(std::min(bv.n * bv.t - r0, kAppendGroups)), dim3(64 * pv.KVH), 0, stream,
