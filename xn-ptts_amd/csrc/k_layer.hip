@@ -283,8 +283,13 @@ __device__ __forceinline__ float epi_y(const uint4 &yv, int i) { // value i of t
 template <int EPI>
 __device__ __forceinline__ void epi_store(const GemmOut &go, int m, const uint4 &yv, const EpiPiece &p, const EpiCols &c) {
     float r[8];
+    if (EPI == kResidual && !go.ls) { // apart, so that the scaled form is not computed beside it
 #pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = epi_value<EPI>(epi_y(yv, i), i, p, c, go);
+        for (int i = 0; i < 8; ++i) r[i] = epi_y(p.x, i) + epi_y(yv, i);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = epi_value<EPI>(epi_y(yv, i), i, p, c, go);
+    }
     epi_write<EPI>(r, m, c);
 }
 
