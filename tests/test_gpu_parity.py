@@ -1490,6 +1490,42 @@ def test_long_prompts_take_several_rounds(cache):
     p.step()
 
 
+# Prompts whose rounds make more groups than CUs (17 streams x 8 heads x 2 and 3 rounds) and whose last full round
+# were of at most 4 tiles take even rounds: of 9 and 8 tiles (the last of one row), 10 and 10, three of 11 and
+# twice 12 after 11, against full ones, which a stream by itself takes (as do 330 rows): outputs and rows bit
+# for bit, after held rows that end mid-page.
+@pytest.mark.parametrize("cache", ["bf16", "i8"])
+@pytest.mark.parametrize("t", [257, 320, 330, 513, 560])
+def test_even_rounds_of_a_prompt_equal_full_ones(cache, t):
+    n, H, held = 17, 8, 21
+    g = torch.Generator(device=DEV).manual_seed(t)
+    pools = [xnp.KvPool(num_layers=1, num_heads=H, num_blocks=n * 38, max_streams=n, max_blocks_per_stream=38, cache_dtype=cache,
+                        act_dtype="bf16", max_pos=1024) for _ in range(2)]
+    idss = [[pool.init_state(608) for _ in range(n)] for pool in pools]
+    for rows in (held, t):
+        q, k, v = (torch.randn((n, rows, H, 64), device=DEV, generator=g).to(torch.bfloat16) for _ in range(3))
+        outs = [torch.empty_like(q) for _ in range(2)]
+        pools[0].begin(idss[0], t=rows)
+        pools[0].attend(0, q, k, v, outs[0], 0.125)
+        pools[0].end()
+        for i in range(n):
+            pools[1].begin([idss[1][i]], t=rows)
+            pools[1].attend(0, q[i:i + 1], k[i:i + 1], v[i:i + 1], outs[1][i:i + 1], 0.125)
+            pools[1].end()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1])
+    for i in (0, 9, n - 1):
+        for kv in (0, 1):
+            got = []
+            for pool, ids in zip(pools, idss):
+                x = torch.empty((held + t, H, 64), dtype=CACHE_TORCH[cache], device=DEV)
+                sc = torch.zeros(((held + t + 15) // 16, H), device=DEV)
+                pool.read_rows(ids[i], 0, kv, 0, x, sc if cache == "i8" else None)
+                got.append((x, sc))
+            torch.cuda.synchronize()
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 # The longest stream a pool takes: 480 pages of 16 rows (60 page ids per wave's lanes, 8 waves per
 # (stream, head)).  Streams one row short of full and one page short of full decode their last row
 # into the last slot and into a fresh last page; a short stream rides along in the same batch.

@@ -10,7 +10,7 @@ namespace xnp {
 // prompt prefill on MFMA (bf16 cache and activations), transformer.rs:231-248 batched, with the
 // append of the prompt's K/V rows (complete_kv, transformer.rs:84-91) fused in.
 //
-// One work group of 8 waves per (stream, head, round), a round being 256 query rows: 16 tiles of 16
+// One work group of 8 waves per (stream, head, round), a round being up to 256 query rows: 16 tiles of 16
 // rows, wave w owning tiles w and 15 - w of the round, so that every wave sees about the same number
 // of causal keys.  Rounds are groups of their own, since a few long prompts leave the chip short of
 // groups (24 streams x 600 rows after 125: 192 groups of three rounds in turn, 64 us a layer;
@@ -95,7 +95,14 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
     // addresses do not wait for the plan.  The grid is round-major, the last round (the most keys)
     // first: the groups of one (stream, head) stay n H apart, on one XCD where 8 divides n H.
     const int nqt = (t + 15) / 16, per = bv.n * pv.H;
-    const int tq0 = ((int)gridDim.x / per - 1 - (int)blockIdx.x / per) * (kPfRound / 16); // the round's first tile
+    const int rounds = (int)gridDim.x / per, round = rounds - 1 - (int)blockIdx.x / per;
+    // the round's tiles, at most 16: full rounds, unless the last were of a few tiles, which stages every key all the
+    // same: even ones then (64 streams x 513 rows 80.4 -> 72.6 us, 256 x 260 126.4 -> 111.4; with the rounds in turn
+    // 76.7 and 123.6).  With 6 tiles left, 24 x 600 after 125, full rounds are ahead (44.3 and 45.5), and while every
+    // group has a CU, where the last round, with the most keys, is the launch (16 x 400 after 125: 20.9 and 23.9).
+    const bool even = rounds > 1 && gridDim.x > 256 && nqt - (rounds - 1) * (kPfRound / 16) <= 4;
+    const int tq0 = even ? round * nqt / rounds : round * (kPfRound / 16);
+    const int nq = even ? (round + 1) * nqt / rounds - tq0 : min(kPfRound / 16, nqt - tq0);
     const int h = (int)blockIdx.x % per % pv.H, b = (int)blockIdx.x % per / pv.H;
     const StreamPlan P = bv.plans[b];
     const int32_t *tab = pv.tables + (size_t)P.sid * pv.mbps;
@@ -112,13 +119,12 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
     // before the round's queries and first chunk go out.  Loads complete in the order
     // issued, so the waits for those (every wave's query loads come after these) cover them, and
     // the barrier follows those waits; no earlier read of spages exists.
-    const int npg = min((c0 + min(t, 16 * tq0 + kPfRound) + kBlock - 1) / kBlock, kPfMaxPages);
+    const int npg = min((c0 + min(t, 16 * (tq0 + nq)) + kBlock - 1) / kBlock, kPfMaxPages);
     static_assert(kPfMaxPages <= 64 * kPfWaves, "one page id per thread");
     if (64 * w < npg) dma4_at(tab + min(tid, npg - 1), lds_addr(&spages[0]) + 256 * w);
     // this thread's share of a chunk: 16 bytes (8 dims) of one key's K and V
     const int skey = tid >> 3, spart = tid & 7;
 
-    const int nq = min(kPfRound / 16, nqt - tq0);
     const bool last = tq0 + nq == nqt;
     // this wave's tiles: (w, nq-1-w) for w < nq/2; the middle one alone when nq is odd
     int tile[2] = {-1, -1};
