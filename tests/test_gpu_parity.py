@@ -397,8 +397,8 @@ def test_window_caches_match_mimis_kv_cache(cache, act):
 
 
 # A bf16 window step of more than 4 rows writes its rows from the attention's own launch: over fresh windows
-# (every 256-row round a work group) and over held rows (as the rows pass where the window has 64 and more, else
-# after each chunk's barrier); where heads share a kv head an append runs after.  Windows of 40 to 250 rows: a fresh chunk
+# (every 256-row round a work group) and over held rows (as the rows pass, behind a barrier
+# of their own where the window has fewer than 64); where heads share a kv head an append runs after.  Windows of 40 to 250 rows: a fresh chunk
 # shorter than the window or of several rounds, chunks over held rows shorter and longer than the window
 # and than a round, single and few rows between, every held row bit for bit after each.
 @pytest.mark.parametrize("context", [40, 63, 64, 65, 191, 192, 250])

@@ -735,8 +735,9 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(4
 //   - held rows, one query head per kv head: one group runs every round in turn (the other rounds' groups
 //     end at once) and writes the rows as they pass in the last.  The slot's old key lies W keys before the
 //     row: with W >= kWpChunk in an earlier chunk, so every wave's load of it has landed, that chunk's barrier
-//     being past; smaller windows write a chunk's rows after its own barrier.  (After it for all: the clips
-//     219.5 -> 222.4 us, two more LDS reads a chunk.)  Chunks in flight behind a row hold no held keys;
+//     being past; smaller windows take a barrier of their own before a chunk's rows are written.  (Written after
+//     the chunk's barrier for all: the clips 219.5 -> 222.4 us, two more LDS reads a chunk.)  Chunks in flight
+//     behind a row hold no held keys;
 //   - held rows, query heads that share a kv head: k_window_append writes them after this launch.
 // Each group takes this from its stream's plan, not from the launch, which depends on the batch's streams, its
 // rows and the heads alone: a launch recorded in a graph serves any windows it is replayed over.
@@ -874,17 +875,7 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
     // the rows that stay (KvCache::trim): the step's last min(t, W), the first of them in slot s0; written as
     // they pass in whole rows of 128 bytes, from the lanes that hold them (one query head per kv head writes)
     const int keep = min(t, W), s0 = (P.pos + t - keep) % W;
-    const bool passing = held ? alone && W >= kWpChunk : h % (pv.H / pv.KVH) == 0, after = held && alone && W < kWpChunk;
-    auto keep_piece = [&](int r, int key, const uint4 &kk, const uint4 &vv) { // row r of those that stay, this lane's unit
-        int s = s0 + r;
-        if (s >= W) s -= W;
-        const int pg = spages[s >> 4];
-        if (pg >= 0 && pg < pv.NB) {
-            const size_t poff = (size_t)pg * page_elems + (s & 15) * kHeadDim + 8 * ((lane_here(lane) & 7) ^ swz(key));
-            st_stream(kpages + poff, kk);
-            st_stream(vpages + poff, vv);
-        }
-    };
+    const bool writes = held ? alone : h % (pv.H / pv.KVH) == 0, small = held && W < kWpChunk;
     // ...then, once they have landed, the step's own keys rotated in place by the lane that loaded
     // them
     auto settle = [&](int j0, int khi, int slot, bool last) {
@@ -896,17 +887,17 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
             uint4 *kp = (uint4 *)&ks[slot][key][8 * (ln & 7)]; // this lane's own pieces
             const uint4 kk = rotate8(*kp, rs[slot][w][i][ln]);
             *kp = kk;
-            const int r = j - ncache - (t - keep);
-            if (last && passing && r >= 0) keep_piece(r, key, kk, *(const uint4 *)&vs[slot][key][8 * (ln & 7)]);
-        }
-    };
-    auto keep_after = [&](int j0, int khi, int slot) { // the chunk's rows, its barrier being past
-        const int ln = lane_here(lane);
-#pragma unroll
-        for (int i = 0; i < kWpLoadsC; ++i) {
-            const int key = kWpKeysW * w + 8 * i + (ln >> 3), j = j0 + key, r = j - ncache - (t - keep);
-            if (j < khi && r >= 0)
-                keep_piece(r, key, *(const uint4 *)&ks[slot][key][8 * (ln & 7)], *(const uint4 *)&vs[slot][key][8 * (ln & 7)]);
+            const int r = j - ncache - (t - keep); // the row's place among those that stay
+            if (last && writes && r >= 0) {
+                int s = s0 + r;
+                if (s >= W) s -= W;
+                const int pg = spages[s >> 4];
+                if (pg >= 0 && pg < pv.NB) {
+                    const size_t poff = (size_t)pg * page_elems + (s & 15) * kHeadDim + 8 * ((ln & 7) ^ swz(key));
+                    st_stream(kpages + poff, kk);
+                    st_stream(vpages + poff, *(const uint4 *)&vs[slot][key][8 * (ln & 7)]);
+                }
+            }
         }
     };
     const int nqt = (t + 15) / 16, rounds = (int)gridDim.x / per;
@@ -993,9 +984,9 @@ __global__ __launch_bounds__(64 * kWpWaves) __attribute__((amdgpu_waves_per_eu(4
                 // this lane's loads of chunk c have landed: after them it issued chunk c + 1 (chunks
                 // 0 .. 2 went out first, then one a step)
                 wait_chunks(min(c == 0 ? kWpSlots - 1 : kWpSlots - 2, nch - 1 - c));
+                if (small) lds_barrier(); // ...and every wave's: the chunk's rows may take its held keys' slots
                 settle(j0, khi, u, tq0 + nq == nqt);
                 lds_barrier(); // chunk c is in LDS; every wave is done with chunk c - 1's slot
-                if (after && tq0 + nq == nqt) keep_after(j0, khi, u);
                 if (c > 0 && c + kWpSlots - 1 < nch)
                     issue(j0 + kWpChunk * (kWpSlots - 1), khi, (u + kWpSlots - 1) % kWpSlots);
 #pragma unroll 1
